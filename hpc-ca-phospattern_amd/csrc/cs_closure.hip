@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstdio>
+#include <cstring>
 #include <vector>
 
 #include "csparks.h"
@@ -25,6 +26,8 @@
 namespace {
 
 constexpr int LROW = 40;                   /* LDS row of 32 samples, padded */
+constexpr uint64_t IDX_CHUNK = 1u << 22;   /* indices staged in pinned memory at a time */
+constexpr int UPD_GROUPS = 16;             /* wavefronts of a k_mlp_update block */
 
 /* FP32 master parameters -> the device image: pre-permuted bfloat16
  * operands of both layers, biases, bfloat16-rounded output weights.  One
@@ -261,35 +264,86 @@ k_mlp_grad(const MlpDev* __restrict__ P, const uint16_t* __restrict__ xb, const 
   }
 }
 
-/* grad[k] = sum over the wavefront partials, in wavefront order. */
-__global__ void k_mlp_reduce(const float* __restrict__ part, uint32_t nwaves, float* __restrict__ grad,
-                             const double* __restrict__ sse, double* __restrict__ sse_out)
+/* Parameter k's places in the operand image (the inverse of k_mlp_pack's
+ * gather): one element for layer 1, a forward and a backward one for layer
+ * 2, the tables for the rest. */
+__device__ inline void pack_one(MlpDev* __restrict__ P, int k, float w)
 {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < MLP_NPARAM) {
-    double acc = 0.0;
-    for (uint32_t w = 0; w < nwaves; w++) acc += part[(uint64_t)w * MLP_NPARAM + k];
-    grad[k] = (float)acc;
-  }
-  if (k == 0) {
-    double e = 0.0;
-    for (uint32_t w = 0; w < nwaves; w++) e += sse[w];
-    *sse_out = e;
+  const uint16_t b = __builtin_bit_cast(uint16_t, to_bf16(w));
+  /* lane group and register of feature f of a 32-block: mlp_feat(g, r) = f */
+  auto group = [](int f) { return (f / 4) % 2; };
+  auto reg = [](int f) { return 4 * (f / 8) + f % 4; };
+  if (k < MLP_OFF_B1) {
+    const int i = k / MLP_H, f = k % MLP_H;
+    P->opnd[SEG_L1 + 2 * (f / 32) + i / 16][32 * ((i / 8) % 2) + f % 32][i % 8] = b;
+  } else if (k < MLP_OFF_W2) {
+    P->b1[k - MLP_OFF_B1] = w;
+  } else if (k < MLP_OFF_B2) {
+    const int i = (k - MLP_OFF_W2) / MLP_H, o = (k - MLP_OFF_W2) % MLP_H;
+    const int ri = reg(i % 32), ro = reg(o % 32);
+    P->opnd[SEG_L2F + 4 * (o / 32) + 2 * (i / 32) + ri / 8][32 * group(i % 32) + o % 32][ri % 8] = b;
+    P->opnd[SEG_L2B + 4 * (i / 32) + 2 * (o / 32) + ro / 8][32 * group(o % 32) + i % 32][ro % 8] = b;
+  } else if (k < MLP_OFF_W3) {
+    P->b2[k - MLP_OFF_B2] = w;
+  } else if (k < MLP_OFF_B3) {
+    P->w3[k - MLP_OFF_W3] = (float)to_bf16(w);
+  } else {
+    P->b3 = w;
   }
 }
 
-/* One Adam step (Kingma & Ba 2015) on the FP32 master parameters. */
-__global__ void k_mlp_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                           const float* __restrict__ g, float lr, float b1, float b2, float eps, float c1, float c2)
+/* One Adam step (Kingma & Ba 2015): its rates and bias corrections; off
+ * for a gradient alone. */
+struct AdamStep {
+  float lr, b1, b2, eps, c1, c2;
+  uint32_t on;
+};
+
+/* grad[k] = sum over the wavefront partials, then (adam.on) the Adam
+ * step on the FP32 master parameters and the parameter's places in the
+ * device image, so a training step is two launches.  A block owns 64
+ * parameters and splits their partials over its 16 wavefronts (one row of
+ * 256 bytes per load), each summing its rows in order in FP64, the 16 sums
+ * in wavefront order: a fixed order, so training is reproducible.  Bound by
+ * the latency of a wavefront's loads (nwaves / 16 rows): one thread per
+ * parameter walking all 768 partials took 222 us, and a batch of 2048 made
+ * only 64 of them. */
+__global__ void __launch_bounds__(64 * UPD_GROUPS)
+k_mlp_update(const float* __restrict__ part, uint32_t nwaves, float* __restrict__ grad, const double* __restrict__ sse,
+             double* __restrict__ sse_out, float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
+             AdamStep adam, MlpDev* __restrict__ P)
 {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= MLP_NPARAM) return;
-  const float gk = g[k];
-  const float mk = b1 * m[k] + (1.0f - b1) * gk;
-  const float vk = b2 * v[k] + (1.0f - b2) * gk * gk;
-  m[k] = mk;
-  v[k] = vk;
-  p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
+  __shared__ double sh[UPD_GROUPS][64];
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int k = blockIdx.x * 64 + lane;
+  double acc = 0.0;
+  if (k < MLP_NPARAM) {
+#pragma unroll 4
+    for (uint32_t w = g; w < nwaves; w += UPD_GROUPS) acc += part[(uint64_t)w * MLP_NPARAM + k];
+  }
+  sh[g][lane] = acc;
+  __syncthreads();
+  if (g == 0 && k < MLP_NPARAM) {
+    acc = sh[0][lane];
+    for (int q = 1; q < UPD_GROUPS; q++) acc += sh[q][lane];
+    const float gk = (float)acc;
+    grad[k] = gk;
+    if (adam.on) {
+      const float mk = adam.b1 * m[k] + (1.0f - adam.b1) * gk;
+      const float vk = adam.b2 * v[k] + (1.0f - adam.b2) * gk * gk;
+      m[k] = mk;
+      v[k] = vk;
+      const float w = p[k] - adam.lr * (mk / adam.c1) / (sqrtf(vk / adam.c2) + adam.eps);
+      p[k] = w;
+      pack_one(P, k, w);
+    }
+  }
+  if (blockIdx.x == 0 && g == 1) {
+    double e = 0.0;
+    for (uint32_t w = lane; w < nwaves; w += 64) e += sse[w];
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+    if (lane == 0) *sse_out = e;
+  }
 }
 
 }  // namespace
@@ -313,6 +367,8 @@ struct cs_mlp {
   uint32_t* d_idx = nullptr;
   uint64_t ndata = 0, cursor = 0;
   std::vector<uint32_t> order;
+  uint32_t* h_idx = nullptr;  /* pinned staging of the order's upload (IDX_CHUNK at most) */
+  hipEvent_t idx_done = nullptr;
   uint64_t shuffle_state = 0;
   /* scratch of cs_mlp_forward / cs_mlp_grad */
   float* d_xs = nullptr;
@@ -333,6 +389,8 @@ void free_mlp(cs_mlp* m)
                   m->d_idx, m->d_xs, m->d_xbs, m->d_ts, m->d_ys};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  if (m->h_idx) (void)hipHostFree(m->h_idx);
+  if (m->idx_done) (void)hipEventDestroy(m->idx_done);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
 }
@@ -366,14 +424,18 @@ int to_bf16_rows(cs_mlp* m, const float* d_x, uint64_t n, uint16_t* d_xb)
   return CS_OK;
 }
 
-/* Gradient of sum (y - t)^2 / norm over n samples into d_grad and the sum
- * of squared errors into d_sse_out. */
-int run_grad(cs_mlp* m, const uint16_t* d_xb, const float* d_t, const uint32_t* d_idx, uint64_t n, float norm)
+/* Gradient of sum (y - t)^2 / norm over n samples into d_grad, the sum of
+ * squared errors into d_sse_out and, with adam.on, the Adam step.  No more
+ * wavefronts than there are rounds of 32 samples: an idle one still writes
+ * a partial of zeros that the update then reads (25 KB each). */
+int run_grad(cs_mlp* m, const uint16_t* d_xb, const float* d_t, const uint32_t* d_idx, uint64_t n, float norm,
+             const AdamStep& adam)
 {
-  hipLaunchKernelGGL(k_mlp_grad, dim3(m->grad_waves), dim3(64), 0, m->stream, m->d_dev,
-                     d_xb, d_t, d_idx, n, norm, m->d_part, m->d_sse);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->d_part,
-                     m->grad_waves, m->d_grad, m->d_sse, m->d_sse_out);
+  const uint32_t waves = (uint32_t)std::min<uint64_t>(m->grad_waves, (n + 31) / 32);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(waves), dim3(64), 0, m->stream, m->d_dev, d_xb, d_t, d_idx, n, norm, m->d_part,
+                     m->d_sse);
+  hipLaunchKernelGGL(k_mlp_update, dim3((MLP_NPARAM + 63) / 64), dim3(64 * UPD_GROUPS), 0, m->stream, m->d_part, waves,
+                     m->d_grad, m->d_sse, m->d_sse_out, m->d_p, m->d_m, m->d_v, adam, m->d_dev);
   HIP_TRY(hipGetLastError());
   return CS_OK;
 }
@@ -507,7 +569,7 @@ int cs_mlp_grad(cs_mlp* m, const float* x, const float* t, uint64_t n, float* gr
   HIP_TRY(hipMemcpyAsync(m->d_xs, x, sizeof(float) * n * MLP_IN, hipMemcpyHostToDevice, m->stream));
   HIP_TRY(hipMemcpyAsync(m->d_ts, t, sizeof(float) * n, hipMemcpyHostToDevice, m->stream));
   if ((rc = to_bf16_rows(m, m->d_xs, n, m->d_xbs)) != CS_OK) return rc;
-  if ((rc = run_grad(m, m->d_xbs, m->d_ts, nullptr, n, (float)n)) != CS_OK) return rc;
+  if ((rc = run_grad(m, m->d_xbs, m->d_ts, nullptr, n, (float)n, AdamStep{})) != CS_OK) return rc;
   double sse = 0.0;
   HIP_TRY(hipMemcpyAsync(grad, m->d_grad, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, m->stream));
   HIP_TRY(hipMemcpyAsync(&sse, m->d_sse_out, sizeof(double), hipMemcpyDeviceToHost, m->stream));
@@ -524,6 +586,11 @@ int cs_mlp_set_data(cs_mlp* m, const float* x, const float* t, uint64_t n, uint6
   void** ptrs[] = {(void**)&m->d_x, (void**)&m->d_t, (void**)&m->d_idx};
   for (void** p : ptrs)
     if (*p) { HIP_TRY(hipFree(*p)); *p = nullptr; }
+  m->ndata = 0;
+  HIP_TRY(hipStreamSynchronize(m->stream));   /* an order's upload may still read the staging buffer */
+  if (m->h_idx) { HIP_TRY(hipHostFree(m->h_idx)); m->h_idx = nullptr; }
+  if (!m->idx_done) HIP_TRY(hipEventCreateWithFlags(&m->idx_done, hipEventDisableTiming));
+  HIP_TRY(hipHostMalloc((void**)&m->h_idx, sizeof(uint32_t) * std::min(n, IDX_CHUNK), hipHostMallocDefault));
   float* d_xf = nullptr;
   HIP_TRY(hipMalloc(&d_xf, sizeof(float) * n * MLP_IN));
   HIP_TRY(hipMalloc(&m->d_x, sizeof(uint16_t) * n * MLP_PAD));
@@ -552,24 +619,29 @@ int cs_mlp_train(cs_mlp* m, uint32_t steps, uint32_t batch, float lr, double* la
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (uint32_t st = 0; st < steps; st++) {
     if (m->cursor + batch > m->ndata) {
-      /* a new epoch: Fisher-Yates with a 64-bit LCG, uploaded once */
+      /* a new epoch: Fisher-Yates with a 64-bit LCG (31-bit numbers, so the
+       * remainder is a 32-bit one), uploaded through pinned memory in stream
+       * order: the steps already queued keep the GPU busy meanwhile */
       for (uint64_t k = m->ndata - 1; k > 0; k--) {
         m->shuffle_state = m->shuffle_state * 6364136223846793005ull + 1442695040888963407ull;
-        const uint64_t j = (m->shuffle_state >> 33) % (k + 1);
+        const uint32_t j = (uint32_t)(m->shuffle_state >> 33) % (uint32_t)(k + 1);
         std::swap(m->order[k], m->order[j]);
       }
-      HIP_TRY(hipMemcpyAsync(m->d_idx, m->order.data(), sizeof(uint32_t) * m->ndata, hipMemcpyHostToDevice, m->stream));
-      HIP_TRY(hipStreamSynchronize(m->stream));
+      for (uint64_t o = 0; o < m->ndata; o += IDX_CHUNK) {
+        const uint64_t c = std::min<uint64_t>(IDX_CHUNK, m->ndata - o);
+        HIP_TRY(hipEventSynchronize(m->idx_done));   /* the staging buffer is free again */
+        memcpy(m->h_idx, m->order.data() + o, sizeof(uint32_t) * c);
+        HIP_TRY(hipMemcpyAsync(m->d_idx + o, m->h_idx, sizeof(uint32_t) * c, hipMemcpyHostToDevice, m->stream));
+        HIP_TRY(hipEventRecord(m->idx_done, m->stream));
+      }
       m->cursor = 0;
     }
-    int rc = run_grad(m, m->d_x, m->d_t, m->d_idx + m->cursor, batch, (float)batch);
+    m->adam_step++;
+    const AdamStep adam{lr, b1, b2, eps, 1.0f - powf(b1, (float)m->adam_step), 1.0f - powf(b2, (float)m->adam_step),
+                        1u};
+    const int rc = run_grad(m, m->d_x, m->d_t, m->d_idx + m->cursor, batch, (float)batch, adam);
     if (rc != CS_OK) return rc;
     m->cursor += batch;
-    m->adam_step++;
-    const float c1 = 1.0f - powf(b1, (float)m->adam_step), c2 = 1.0f - powf(b2, (float)m->adam_step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->d_p, m->d_m, m->d_v,
-                       m->d_grad, lr, b1, b2, eps, c1, c2);
-    if ((rc = pack(m)) != CS_OK) return rc;
   }
   double sse = 0.0;
   HIP_TRY(hipMemcpyAsync(&sse, m->d_sse_out, sizeof(double), hipMemcpyDeviceToHost, m->stream));
