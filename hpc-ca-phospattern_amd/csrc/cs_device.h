@@ -547,6 +547,10 @@ __device__ inline double flux_j(const FluxParams& F, double vf, double vt, doubl
   return cs_serca_flux_d(dt, h, vf + r0, vt + r1, F.density);
 }
 
+/* Domain id bytes: bits 0-2 the domain, bit 6 a voxel of a boundary pair,
+ * bit 7 an in-grid neighbourhood of one domain. */
+constexpr uint8_t ID_PAIR = 0x40;
+
 /* marks a missing row, slot or channel state in the flat records */
 constexpr uint32_t NO_ROW = 0xFFFFFFFFu;
 
@@ -563,8 +567,9 @@ struct BChan {          /* a channel of a discrete flux, in gating order */
 struct BRow {           /* a k_flux row                                   */
   uint64_t elem;        /* the value the row adds to                      */
   uint32_t start, end;  /* its entries                                    */
-  uint32_t skip, pad;   /* 1: species fixed in the domain, or species 0 on
+  uint32_t skip;        /* 1: species fixed in the domain, or species 0 on
                            a Dirichlet face (the row takes nothing)       */
+  uint32_t slot;        /* level-1 slot of the row's voxel                */
 };
 struct BEnt {           /* a pair of a row, in k_flux's order             */
   uint64_t elem_from, elem_to;

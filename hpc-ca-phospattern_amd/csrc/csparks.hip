@@ -29,6 +29,8 @@
  * A fused pass computes two steps per trip through HBM:
  *   k_step2   both steps' stencils and reactions on tiles with a one-voxel
  *             halo, the intermediate state kept on chip;
+ *   k_pass2   the same for the reference's five-slot layout, compiled for
+ *             each pair of step masks (k_pass2.h);
  *   k_bridge  one block gates the channels and applies the boundary
  *             fluxes around the passes, with k_gate's and k_flux's code.
  */
@@ -40,6 +42,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -49,6 +52,7 @@
 #include "cs_physics.h"
 
 #include "cs_device.h"
+#include "cs_pass2.h"
 
 thread_local std::string g_err;
 
@@ -82,7 +86,7 @@ struct LaunchCfg {
   int fuse;      /* 1: pairs of eligible steps run as one k_step2 pass     */
   int fz;        /* planes per block of k_step2                             */
   int fx;        /* xcd_tile map of k_step2's blocks                        */
-  int ff;        /* 1: k_step2 compiled for the pass's step masks, if any   */
+  int ff;        /* 1: k_pass2 (compiled masks) where the model fits it */
 };
 
 template <typename T, int NS, int PF, bool NT>
@@ -614,13 +618,11 @@ k_flux(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__ 
 
 /* Voxels of the boundary pairs for the fused pass, ordered by plane
  * column (y*nx + x) and then z, so that a lane marching one column meets
- * them in order.  Pair voxel k keeps its level-1 value of species 0 in
- * slot k; row[k] is its k_flux row (every flux acts on species 0), or
- * NO_ROW. */
+ * them in order.  Pair voxel k keeps its level-1 value of species 0 and the
+ * flux sum that step 1 adds there (0 where none does) in slot k. */
 struct F2Voxels {
   const uint32_t* col_start;   /* [plane + 1] first pair voxel of each column */
   const uint32_t* z;           /* plane of pair voxel k                        */
-  const uint32_t* row;         /* k_flux row of pair voxel k, or NO_ROW         */
 };
 
 /* What one of the two steps of a fused pass does. */
@@ -641,24 +643,16 @@ struct F2Step {
  * through a double-buffered LDS plane (one barrier per plane); z
  * neighbours sit in register rings.  Each
  * level is k_stencil's per-voxel update.  The boundary fluxes of step 1,
- * summed per k_flux row before the pass (k_bridge), are added at level 1
+ * summed per pair voxel before the pass (k_bridge), are added at level 1
  * as k_flux adds them, and the level-1 value of species 0 at every pair
  * voxel is kept in its slot: step 2's gating and fluxes need only those
  * values, and its fluxes add to the result after the pass (k_bridge),
  * since no other voxel's step-2 update reads them. */
-/* Step masks of a fused pass fixed at compile time: FM1/FM2 are the
- * diffusing species of its two steps and FR the reaction mode of both, or
- * F2_DYN for values taken from s1/s2 at run time.  With fixed masks the
- * species loops keep only the species that diffuse, where run-time bits
- * leave every species' code in the loop behind a test. */
-constexpr uint32_t F2_DYN = 0xFFFFFFFFu;
-
-template <typename T, int NS, int WY, bool NT, uint32_t FM1 = F2_DYN, uint32_t FM2 = F2_DYN, uint32_t FR = F2_DYN>
+template <typename T, int NS, int WY, bool NT>
 __global__ void __launch_bounds__(BX * WY)
 k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__ ids,
         const DevParams<T>* __restrict__ P, Geo g, F2Voxels fv, const double* __restrict__ fsum,
-        const uint8_t* __restrict__ fany, T* __restrict__ l1, F2Step s1, F2Step s2, int zchunk, int tx, int ty,
-        int nblocks, int xcd)
+        T* __restrict__ l1, F2Step s1, F2Step s2, int zchunk, int tx, int ty, int nblocks, int xcd)
 {
   __shared__ BlockTables<T, NS> S;
   __shared__ T ex[2][NS][WY][BX];
@@ -708,8 +702,7 @@ k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__
   auto iofs = [&](int zz) { return (uint32_t)(min(max(zz, zb), ze - 1) - zb) * (uint32_t)plane; };
 
   const uint32_t react_nb = (uint32_t)P->nb;
-  uint32_t dm1 = FM1 != F2_DYN ? FM1 : s1.dmask, dm2 = FM2 != F2_DYN ? FM2 : s2.dmask;
-  uint32_t re1 = FR != F2_DYN ? FR : s1.react, re2 = FR != F2_DYN ? FR : s2.react, rbound = P->rbound;
+  uint32_t dm1 = s1.dmask, dm2 = s2.dmask, re1 = s1.react, re2 = s2.react, rbound = P->rbound;
   __shared__ uint32_t msk[5];
   if (lane == 0 && wy == 0) {
     msk[0] = dm1;
@@ -814,8 +807,7 @@ k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__
     }
     /* level 1 at a pair voxel: step 1's flux sum, then the slot */
     if (first && pz == zz) {
-      const uint32_t r = fv.row[pk];
-      if (r != NO_ROW && fany[r]) nw[0] = (T)((double)nw[0] + fsum[r]);
+      nw[0] = (T)((double)nw[0] + fsum[pk]);
       if (inner && zz >= z0 && zz < z1) l1[pk] = nw[0];
       pk++;
       pz = pk < pend ? (int)fv.z[pk] : 0x7FFFFFFF;
@@ -875,12 +867,10 @@ k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__
      * orders the first read after the write): each species test is then a
      * bit test of one scalar register, not a flag hoisted out of the loop,
      * of which there are too many to keep in scalar registers */
-    if constexpr (FM1 == F2_DYN) dm1 = __builtin_amdgcn_readfirstlane(msk[0]);
-    if constexpr (FM2 == F2_DYN) dm2 = __builtin_amdgcn_readfirstlane(msk[1]);
-    if constexpr (FR == F2_DYN) {
-      re1 = __builtin_amdgcn_readfirstlane(msk[2]);
-      re2 = __builtin_amdgcn_readfirstlane(msk[3]);
-    }
+    dm1 = __builtin_amdgcn_readfirstlane(msk[0]);
+    dm2 = __builtin_amdgcn_readfirstlane(msk[1]);
+    re1 = __builtin_amdgcn_readfirstlane(msk[2]);
+    re2 = __builtin_amdgcn_readfirstlane(msk[3]);
     rbound = __builtin_amdgcn_readfirstlane(msk[4]);
     const bool below = z < nz;
     if (below) {
@@ -958,7 +948,7 @@ k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__
  *     pass's level-1 slots, the fluxes added to u (the state after t+1);
  *   head, before a pass over steps t', t'+1: k_gate of step t' on u, then
  *     the flux sum of every k_flux row from u, which the pass adds at
- *     level 1.
+ *     level 1 (in the row's voxel's slot).
  * Either part may be off.  The gating (gate_one) and flux (flux_j) code,
  * the entry order and the skip rules are k_gate's and k_flux's, so the
  * results are the same.  phases selects the phases this launch runs
@@ -972,8 +962,7 @@ template <typename T>
 __global__ void __launch_bounds__(BRIDGE_THREADS)
 k_bridge(T* __restrict__ u, const DevParams<T>* __restrict__ P, const BChan* __restrict__ chans, uint32_t nchan,
          const BRow* __restrict__ rows, uint32_t nrows, const BEnt* __restrict__ ents, const T* __restrict__ l1,
-         uint8_t* __restrict__ states, uint8_t* __restrict__ recruited, double* __restrict__ fsum,
-         uint8_t* __restrict__ fany, F2Step tail, uint32_t do_tail, F2Step head, uint32_t do_head, uint32_t D,
+         uint8_t* __restrict__ states, uint8_t* __restrict__ recruited, double* __restrict__ fsum, F2Step tail, uint32_t do_tail, F2Step head, uint32_t do_head, uint32_t D,
          uint32_t seed, uint32_t instance, const double* __restrict__ uniforms, uint32_t phases)
 {
   const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
@@ -1041,8 +1030,7 @@ k_bridge(T* __restrict__ u, const DevParams<T>* __restrict__ P, const BChan* __r
         const bool any = row_flux(r, head.fluxmask,
                                   [&](const BEnt& x, bool to) { return (double)u[to ? x.elem_to : x.elem_from]; },
                                   sum);
-        fsum[r] = sum;
-        fany[r] = any ? 1 : 0;
+        fsum[rows[r].slot] = any ? sum : 0.0;
       }
   }
 }
@@ -1393,16 +1381,14 @@ struct cs_context {
   uint32_t flux_substep[MAXF] = {0};
   LaunchCfg launch{4, 32, 1, 1, 0, 0, 0, 0, 0, 32, 1};
   uint32_t rfast = 0;   /* buffer reactions admit the species-major form */
+  uint32_t rbound = 0;  /* species that a buffer binds                   */
   std::vector<uint8_t> h_ids;   /* domain ids in device order (host copy)  */
   uint64_t dcount[MAXD] = {0};  /* voxels per domain                        */
   /* fused two-step pass (k_step2) */
   uint32_t* d_f2_col = nullptr;      /* pair voxels by column, see F2Voxels   */
   uint32_t* d_f2_z = nullptr;
-  uint32_t* d_f2_row = nullptr;
-  uint32_t* d_f2_pslot = nullptr;    /* slots of each pair's from and to voxel */
   void* d_f2_l1 = nullptr;           /* level-1 species 0 at the pair voxels  */
-  double* d_f2_fsum = nullptr;       /* step-1 flux sum per k_flux row        */
-  uint8_t* d_f2_fany = nullptr;      /* the row takes its sum                 */
+  double* d_f2_fsum = nullptr;       /* step-1 flux sum per pair voxel        */
   void* d_bchan = nullptr;           /* k_bridge records: BChan, BRow, BEnt   */
   void* d_brow = nullptr;
   void* d_bent = nullptr;
@@ -1410,6 +1396,14 @@ struct cs_context {
   bool f2_ok = false;                /* the problem admits fused passes       */
   std::string f2_why;                /* why not, when it does not             */
   uint32_t fsm = 0;                  /* species the fluxes act on (bit 0)     */
+  /* k_pass2: whether the model admits it, the domain's record, its split
+   * into column tiles, and a tile list per number of planes per block */
+  bool p2_ok = false, p2_whole = false;
+  bool auto_form = true;             /* no launch shape was set or tuned yet  */
+  P2Split p2_split{0, 0};
+  P2Geo* d_p2_geo = nullptr;
+  struct TileList { P2Tile* d = nullptr; uint32_t n = 0; };
+  std::map<int, TileList> p2_lists;
 };
 
 namespace {
@@ -1431,12 +1425,13 @@ int max_zchunk(const Geo& g, size_t esize)
   return (int)std::min<uint64_t>((uint64_t)g.nz, ((1ull << 32) - 1) / group - 3);
 }
 
-/* Largest z chunk of k_step2, whose blocks span (chunk + 4) z-groups
- * under 32-bit descriptor offsets (0 when not even one plane fits). */
+/* Largest z chunk of a two-step pass, whose blocks span (chunk + 4)
+ * z-groups (and k_pass2's a last chunk's padding) under 32-bit descriptor
+ * offsets (0 when not even one plane fits). */
 int max_fused_zchunk(const Geo& g, size_t esize)
 {
   const uint64_t group = g.plane * esize * g.ns;
-  const uint64_t fit = ((1ull << 32) - 1) / group;
+  const uint64_t fit = ((1ull << 32) - 1 - P2_PAD) / group;
   return fit > 4 ? (int)std::min<uint64_t>((uint64_t)g.nz, fit - 4) : 0;
 }
 
@@ -1475,8 +1470,9 @@ void free_ctx(cs_context* c)
                   c->d_row_voxel, c->d_row_species, c->d_row_start, c->d_ent_pair,
                   c->d_ent_flux, c->d_ent_sign, c->d_uniforms, c->d_partial, c->d_stats,
                   c->d_lweights, c->d_lpart, c->d_f2_col, c->d_f2_z,
-                  c->d_f2_row, c->d_f2_pslot, c->d_f2_l1, c->d_f2_fsum, c->d_f2_fany, c->d_bchan,
-                  c->d_brow, c->d_bent};
+                  c->d_f2_l1, c->d_f2_fsum, c->d_bchan, c->d_brow, c->d_bent, c->d_p2_geo};
+  for (auto& kv : c->p2_lists)
+    if (kv.second.d) hipFree(kv.second.d);
   for (void* p : ptrs)
     if (p) hipFree(p);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -1548,6 +1544,7 @@ int upload_params(cs_context* c)
   DevParams<T> dp;
   fill_params<T>(dp, &c->prob, c->ndiscrete);
   c->rfast = dp.rfast;
+  c->rbound = dp.rbound;
   if (!c->d_params) HIP_TRY(hipMalloc(&c->d_params, sizeof(DevParams<T>)));
   HIP_TRY(hipMemcpyAsync(c->d_params, &dp, sizeof dp, hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));   /* dp lives on this stack frame */
@@ -1724,13 +1721,66 @@ F2Step step_info(const cs_context* c, uint64_t ti, uint64_t uni_base)
  * both steps, so its neighbours are at hand at both levels. */
 bool can_fuse(const cs_context* c, const LaunchCfg& L, uint64_t ti)
 {
-  if (!L.fuse || !c->f2_ok) return false;
+  if (!c->f2_ok || !(L.fuse || (c->auto_form && c->p2_ok))) return false;
   return (c->fsm & ~diffusing(c, ti)) == 0 && (c->fsm & ~diffusing(c, ti + 1)) == 0;
 }
 
-template <typename T, int NS, uint32_t FM1 = F2_DYN, uint32_t FM2 = F2_DYN, uint32_t FR = F2_DYN>
-void launch_step2_k(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
-                    const F2Step& b)
+/* The tile list of blocks of at most fz planes (built once per fz; the
+ * launch shapes that cs_autotune tries are few). */
+int pass2_tiles(cs_context* c, int fz, cs_context::TileList& out)
+{
+  auto it = c->p2_lists.find(fz);
+  if (it == c->p2_lists.end()) {
+    std::vector<P2Tile> tiles;
+    p2_tiles(0, (uint32_t)c->geo.nx, (uint32_t)c->geo.ny, (uint32_t)c->geo.nz, c->p2_split,
+             (uint32_t)((c->geo.nz + fz - 1) / fz), tiles);
+    for (const P2Tile& q : tiles)
+      if (!p2_fits(q, (uint32_t)c->geo.nx, (uint32_t)c->geo.ny, c->esize, c->p2_whole))
+        return set_err(CS_EDEVICE, "a tile of %u x %u columns does not fit its block", q.w, q.h);
+    cs_context::TileList t;
+    t.n = (uint32_t)tiles.size();
+    HIP_TRY(hipMalloc((void**)&t.d, sizeof(P2Tile) * tiles.size()));
+    const hipError_t e = hipMemcpy(t.d, tiles.data(), sizeof(P2Tile) * tiles.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      hipFree(t.d);
+      return set_err(CS_EDEVICE, "upload of tiles failed: %s", hipGetErrorString(e));
+    }
+    it = c->p2_lists.emplace(fz, t).first;
+  }
+  out = it->second;
+  return CS_OK;
+}
+
+int launch_pass2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a, const F2Step& b)
+{
+  cs_context::TileList tl;
+  const int rc = pass2_tiles(c, std::max(1, std::min(L.fz, c->geo.nz)), tl);
+  if (rc != CS_OK) return rc;
+  P2Args p{};
+  p.u = uin;
+  p.un = uout;
+  p.ids = c->d_ids;
+  p.params = c->d_params;
+  p.geos = c->d_p2_geo;
+  p.tiles = tl.d;
+  p.col_start = c->d_f2_col;
+  p.vz = c->d_f2_z;
+  p.fsum = c->d_f2_fsum;
+  p.l1 = c->d_f2_l1;
+  p.ntiles = tl.n;
+  p.xcd = L.fx;
+  p.react1 = a.react ? 1u : 0u;
+  p.react2 = b.react ? 1u : 0u;
+  for (uint32_t d = 0; d < c->nd; d++)
+    for (uint32_t s = 0; s < c->ns; s++) p.any_fixed |= c->prob.fixed[d][s] ? 1u : 0u;
+  if (!cs_internal_pass2(c->esize, c->p2_whole, a.dmask, b.dmask, p, c->stream))
+    return set_err(CS_EDEVICE, "no two-step pass for masks %x, %x", a.dmask, b.dmask);
+  return CS_OK;
+}
+
+template <typename T, int NS>
+void launch_step2_ns(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
+                     const F2Step& b)
 {
   constexpr int WY = sizeof(T) == 4 ? 16 : 8;
   const Geo& g = c->geo;
@@ -1738,49 +1788,21 @@ void launch_step2_k(cs_context* c, const LaunchCfg& L, const void* uin, void* uo
   const int zc = std::max(1, std::min(L.fz, g.nz));
   const int tz = (g.nz + zc - 1) / zc;
   const int nblocks = tx * ty * tz;
-  const F2Voxels fv{c->d_f2_col, c->d_f2_z, c->d_f2_row};
+  const F2Voxels fv{c->d_f2_col, c->d_f2_z};
   /* plain stores: on the 400x400x200 dyad non-temporal ones cost 2% (472 against
    * 463 us per pass at z chunk 40 and groups of 32) */
-  hipLaunchKernelGGL((k_step2<T, NS, WY, false, FM1, FM2, FR>), dim3(xcd_launch(nblocks, L.fx)), dim3(BX, WY), 0,
-                     c->stream, (const T*)uin, (T*)uout, c->d_ids, (const DevParams<T>*)c->d_params, g, fv,
-                     (const double*)c->d_f2_fsum, (const uint8_t*)c->d_f2_fany, (T*)c->d_f2_l1, a, b, zc, tx, ty,
-                     nblocks, L.fx);
+  hipLaunchKernelGGL((k_step2<T, NS, WY, false>), dim3(xcd_launch(nblocks, L.fx)), dim3(BX, WY), 0, c->stream,
+                     (const T*)uin, (T*)uout, c->d_ids, (const DevParams<T>*)c->d_params, g, fv,
+                     (const double*)c->d_f2_fsum, (T*)c->d_f2_l1, a, b, zc, tx, ty, nblocks, L.fx);
 }
 
-/* Pairs of step masks compiled with fixed masks, for the species layout of
- * the reference's species files (parameters/*.h5: Ca, Fluo, CMDN-CSQN,
- * ATP, TRPN): Ca and ATP diffuse on every step (0x9), the dye and CMDN on
- * their own multiples of dt (0x2, 0x4), TRPN never.  These are every pair
- * of consecutive steps when the two slow species' substeps are at least 2;
- * the reaction runs species-major on both steps.  Other pairs, species
- * counts and FP64 run the kernel with run-time masks. */
-template <typename T, int NS>
-void launch_step2_ns(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
-                     const F2Step& b)
-{
-  if constexpr (sizeof(T) == 4 && NS == 5) {
-    if (L.ff && a.react == 2 && b.react == 2) {
-      switch ((a.dmask << 8) | b.dmask) {
-        case 0x0909: return launch_step2_k<T, NS, 0x9, 0x9, 2>(c, L, uin, uout, a, b);
-        case 0x0B09: return launch_step2_k<T, NS, 0xB, 0x9, 2>(c, L, uin, uout, a, b);
-        case 0x090B: return launch_step2_k<T, NS, 0x9, 0xB, 2>(c, L, uin, uout, a, b);
-        case 0x0D09: return launch_step2_k<T, NS, 0xD, 0x9, 2>(c, L, uin, uout, a, b);
-        case 0x090D: return launch_step2_k<T, NS, 0x9, 0xD, 2>(c, L, uin, uout, a, b);
-        case 0x0F09: return launch_step2_k<T, NS, 0xF, 0x9, 2>(c, L, uin, uout, a, b);
-        case 0x090F: return launch_step2_k<T, NS, 0x9, 0xF, 2>(c, L, uin, uout, a, b);
-        case 0x0B0D: return launch_step2_k<T, NS, 0xB, 0xD, 2>(c, L, uin, uout, a, b);
-        case 0x0D0B: return launch_step2_k<T, NS, 0xD, 0xB, 2>(c, L, uin, uout, a, b);
-        default: break;
-      }
-    }
-  }
-  launch_step2_k<T, NS>(c, L, uin, uout, a, b);
-}
-
+/* Two steps in one pass: k_pass2 where it applies, else k_step2 with the
+ * masks read at run time. */
 template <typename T>
-void launch_step2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
-                  const F2Step& b)
+int launch_step2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
+                 const F2Step& b)
 {
+  if (c->p2_ok && L.ff) return launch_pass2(c, L, uin, uout, a, b);
   switch (c->ns) {
     case 1: launch_step2_ns<T, 1>(c, L, uin, uout, a, b); break;
     case 2: launch_step2_ns<T, 2>(c, L, uin, uout, a, b); break;
@@ -1791,6 +1813,7 @@ void launch_step2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout
     case 7: launch_step2_ns<T, 7>(c, L, uin, uout, a, b); break;
     default: break;   /* more species never fuse (f2_ok is false) */
   }
+  return CS_OK;
 }
 
 /* k_bridge on the state u: the tail of a pass (step `tail`) and/or the
@@ -1803,7 +1826,7 @@ void launch_bridge(cs_context* c, void* u, const F2Step& tail, bool do_tail, con
     hipLaunchKernelGGL(k_bridge<T>, dim3(blocks), dim3(BRIDGE_THREADS), 0, c->stream, (T*)u,
                        (const DevParams<T>*)c->d_params, (const BChan*)c->d_bchan, c->nbchan,
                        (const BRow*)c->d_brow, c->nrows, (const BEnt*)c->d_bent, (const T*)c->d_f2_l1, c->d_states,
-                       c->d_recruited, c->d_f2_fsum, c->d_f2_fany, tail, do_tail ? 1u : 0u, head,
+                       c->d_recruited, c->d_f2_fsum, tail, do_tail ? 1u : 0u, head,
                        do_head ? 1u : 0u, (uint32_t)c->prob.stochastic_substep, (uint32_t)c->prob.seed,
                        (uint32_t)c->prob.instance, d_uni, phases);
   };
@@ -1896,7 +1919,8 @@ int run_steps(cs_context* c, uint64_t first, uint64_t n, const double* host_uni,
       const F2Step s2 = step_info(c, ti + 1, gate_idx * spg);
       if (gates(ti + 1)) gate_idx++;
       if (ea) HIP_TRY(hipEventRecord(ea, c->stream));
-      launch_step2<T>(c, c->launch, c->d_u[c->cur], c->d_u[c->cur ^ 1], s1, s2);
+      const int rc = launch_step2<T>(c, c->launch, c->d_u[c->cur], c->d_u[c->cur ^ 1], s1, s2);
+      if (rc != CS_OK) return rc;
       if (eb) HIP_TRY(hipEventRecord(eb, c->stream));
       const bool next = i + 3 < n && can_fuse(c, c->launch, ti + 2);
       F2Step h2 = s2;
@@ -1934,6 +1958,27 @@ int run_steps(cs_context* c, uint64_t first, uint64_t n, const double* host_uni,
     if (npasses) *npasses = passes;
     if (nfused) *nfused = fused;
   }
+  return CS_OK;
+}
+
+/* Whether k_pass2 fits the problem, and its records: the five-slot layout
+ * with its substeps (then every step has a compiled mask, and reacts, if at
+ * all, in species-major form), fused passes at all, at least two columns
+ * either way, a split whose blocks hold a tile. */
+int setup_pass2(cs_context* c)
+{
+  const Geo& g = c->geo;
+  c->p2_ok = false;
+  if (!c->f2_ok || c->ns != 5 || (c->prob.num_buffers && (!c->rfast || c->rbound != 0x1Eu)) || !p2_substeps(c->substeps) ||
+      g.nx < 2 || g.ny < 2)
+    return CS_OK;
+  c->p2_whole = p2_whole(g.nv * c->ns * c->esize);
+  c->p2_split = p2_split((uint32_t)g.nx, (uint32_t)g.ny, c->esize, c->p2_whole);
+  if (!c->p2_split.kx) return CS_OK;
+  const P2Geo rec{0, 0, 0, (uint32_t)g.plane, g.nx, g.ny, g.nz, 0};
+  HIP_TRY(hipMalloc((void**)&c->d_p2_geo, sizeof rec));
+  HIP_TRY(hipMemcpy(c->d_p2_geo, &rec, sizeof rec, hipMemcpyHostToDevice));
+  c->p2_ok = true;
   return CS_OK;
 }
 
@@ -2026,22 +2071,20 @@ int build_flux_rows(cs_context* c, const cs_problem* p)
   std::sort(keys.begin(), keys.end());
   keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
   std::unordered_map<uint32_t, uint32_t> slot;
-  std::vector<uint32_t> col_start(g.plane + 1, 0), vz(keys.size()), vrow(keys.size(), NO_ROW);
+  std::vector<uint32_t> col_start(g.plane + 1, 0), vz(keys.size());
   for (size_t k = 0; k < keys.size(); k++) {
     const uint64_t colv = keys[k] >> 32, z = keys[k] & 0xFFFFFFFFu;
     slot[(uint32_t)(z * g.plane + colv)] = (uint32_t)k;
     vz[k] = (uint32_t)z;
     col_start[colv + 1]++;
+    c->h_ids[z * g.plane + colv] |= ID_PAIR;
   }
   for (size_t k = 1; k < col_start.size(); k++) col_start[k] += col_start[k - 1];
-  for (uint32_t r = 0; r < (uint32_t)row_voxel.size(); r++)
-    if (row_species[r] == 0) vrow[slot[row_voxel[r]]] = r;
   std::vector<uint32_t> pslot(pairs_dev.size());
   for (size_t k = 0; k < pairs_dev.size(); k++) pslot[k] = slot[pairs_dev[k]];
   if ((rc = up(&c->d_f2_col, col_start)) != CS_OK) return rc;
   if ((rc = up(&c->d_f2_z, vz)) != CS_OK) return rc;
-  if ((rc = up(&c->d_f2_row, vrow)) != CS_OK) return rc;
-  if ((rc = up(&c->d_f2_pslot, pslot)) != CS_OK) return rc;
+  HIP_TRY(hipMemcpyAsync(c->d_ids, c->h_ids.data(), g.nv, hipMemcpyHostToDevice, c->stream));
 
   /* k_bridge's flat records */
   std::vector<uint32_t> pair_off(p->num_fluxes + 1, 0);
@@ -2063,7 +2106,7 @@ int build_flux_rows(cs_context* c, const cs_problem* p)
     const bool face = x == 0 || y == 0 || z == 0 || x + 1 == (uint32_t)g.nx || y + 1 == (uint32_t)g.ny ||
                       z + 1 == (uint32_t)g.nz;
     const bool skip = p->fixed[dom(v)][sp] || (sp == 0 && p->force_dirichlet && face);
-    brow[r] = BRow{elem(g, sp, v), row_start[r], row_start[r + 1], skip ? 1u : 0u, 0};
+    brow[r] = BRow{elem(g, sp, v), row_start[r], row_start[r + 1], skip ? 1u : 0u, slot[v]};
     for (uint32_t e = row_start[r]; e < row_start[r + 1]; e++) {
       const uint32_t f = ent_flux[e], gp = pair_off[f] + ent_pair[e];
       const uint32_t from = pairs_dev[2 * gp], to = pairs_dev[2 * gp + 1];
@@ -2083,8 +2126,8 @@ int build_flux_rows(cs_context* c, const cs_problem* p)
   if ((rc = upb(&c->d_brow, brow.data(), sizeof(BRow) * brow.size())) != CS_OK) return rc;
   if ((rc = upb(&c->d_bent, bent.data(), sizeof(BEnt) * bent.size())) != CS_OK) return rc;
   HIP_TRY(hipMalloc(&c->d_f2_l1, c->esize * std::max<size_t>(keys.size(), 1)));
-  HIP_TRY(hipMalloc((void**)&c->d_f2_fsum, sizeof(double) * std::max<size_t>(row_voxel.size(), 1)));
-  HIP_TRY(hipMalloc((void**)&c->d_f2_fany, std::max<size_t>(row_voxel.size(), 1)));
+  HIP_TRY(hipMalloc((void**)&c->d_f2_fsum, sizeof(double) * std::max<size_t>(keys.size(), 1)));
+  HIP_TRY(hipMemsetAsync(c->d_f2_fsum, 0, sizeof(double) * std::max<size_t>(keys.size(), 1), c->stream));
   /* the host vectors above end here */
   HIP_TRY(hipStreamSynchronize(c->stream));
   return CS_OK;
@@ -2161,11 +2204,8 @@ int cs_create(const cs_problem* p, cs_context** out)
       }
   if (hipMalloc(&c->d_ids, g.nv) != hipSuccess) return bail(set_err(CS_ENOMEM, "device allocation of ids failed"));
   for (int b = 0; b < 2; b++)
-    if (hipMalloc(&c->d_u[b], c->esize * c->ns * g.nv) != hipSuccess)
+    if (hipMalloc(&c->d_u[b], c->esize * c->ns * g.nv + P2_PAD) != hipSuccess)
       return bail(set_err(CS_ENOMEM, "device allocation of %zu bytes failed", c->esize * c->ns * g.nv));
-  if (hipMemcpyAsync(c->d_ids, ids.data(), g.nv, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-      hipStreamSynchronize(c->stream) != hipSuccess)
-    return bail(set_err(CS_EDEVICE, "upload of ids failed"));
   c->h_ids.swap(ids);
   for (uint8_t id : c->h_ids)
     if ((id & 7) < MAXD) c->dcount[id & 7]++;
@@ -2179,17 +2219,34 @@ int cs_create(const cs_problem* p, cs_context** out)
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, c->device) != hipSuccess) return bail(set_err(CS_EDEVICE, "device query failed"));
   const int cus = std::max(prop.multiProcessorCount, 1);
+  rc = setup_pass2(c);
+  if (rc != CS_OK) return bail(rc);
   c->launch = default_launch(g, c->esize, cus);
-  /* fused passes by default in FP32, where they measured faster; FP64
-   * blocks hold half the rows (register file), so there one-step passes
-   * win.  A fused pass holds one block per CU, so a grid whose fused launch
-   * has fewer blocks than half the CUs leaves most of them idle: on the
-   * 84^3 G1 geometry at 12 nm (36 blocks) a step takes 79.6 us fused
-   * against 36.5 us in one-step passes (FP32, one box), while the
-   * 200x200x100 dyad (240 blocks) takes 52.4 against 62.3 us. */
+  /* Until a shape is set or tuned (auto_form), every pair of steps that
+   * k_pass2 takes runs so: it beat one-step passes on every grid measured,
+   * per step with gating and fluxes 12 against 22 us on 64x64x25 (FP64), 19
+   * against 35 on 84^3 (FP64), 16 against 27 on 131x97x53 (FP32), 335
+   * against 560 on 400x400x200 (FP64), 174 against 260 on that in FP32.
+   * launch.fuse is the same choice for k_step2, which models outside
+   * k_pass2's layout take.  In FP64 its blocks hold half the rows (register
+   * file), so one-step passes win.  It holds one block per CU, so a grid
+   * whose fused launch has fewer blocks than half the CUs leaves most of
+   * them idle: on the 84^3 G1 geometry at 12 nm (36 blocks) a step takes
+   * 79.6 us fused against 36.5 us in one-step passes (FP32, one box), while
+   * the 200x200x100 dyad (240 blocks) takes 52.4 against 62.3 us. */
   const long fused_tiles = (long)((g.nx + BX - 3) / (BX - 2)) * ((g.ny + 16 - 3) / (16 - 2));
   const long fused_blocks = fused_tiles * ((g.nz + c->launch.fz - 1) / std::max(c->launch.fz, 1));
   c->launch.fuse = (c->f2_ok && c->esize == 4 && 2 * fused_blocks >= cus) ? 1 : 0;
+  if (c->p2_ok) {
+    /* k_pass2's own planes per block and tile order */
+    const long cols = (long)c->p2_split.kx * c->p2_split.ky;
+    const uint32_t parts = p2_zparts((uint64_t)cols, (uint32_t)g.nz, c->p2_whole ? cus : 2 * cus,
+                                     (uint32_t)max_fused_zchunk(g, c->esize));
+    c->launch.fz = (g.nz + (int)parts - 1) / (int)parts;
+    c->launch.fx = 0;
+    for (int G = 16; G >= 2; G /= 2)
+      if (cols * parts >= 8L * 3 * G) { c->launch.fx = G; break; }
+  }
   rc = c->esize == 8 ? fill_init<double>(c) : fill_init<float>(c);
   if (rc != CS_OK) return bail(rc);
   if (hipStreamSynchronize(c->stream) != hipSuccess) return bail(set_err(CS_EDEVICE, "setup failed"));
@@ -2601,6 +2658,7 @@ int cs_set_launch_config(cs_context* c, const cs_launch_config* in)
   L.fx = (int)in->fuse_xcd;
   L.ff = (int)in->fuse_fixed;
   c->launch = L;
+  c->auto_form = false;
   return CS_OK;
 }
 
@@ -2738,14 +2796,15 @@ int cs_autotune(cs_context* c, uint64_t first_time_ind, uint32_t reps, cs_launch
           /* the pass and its bridge (tail and the next head, no gating) */
           auto go = [&]() {
             if (c->esize == 8) {
-              launch_step2<double>(c, L, c->d_u[c->cur], c->d_u[c->cur ^ 1], q.a, q.b);
+              rc = launch_step2<double>(c, L, c->d_u[c->cur], c->d_u[c->cur ^ 1], q.a, q.b);
               launch_bridge<double>(c, c->d_u[c->cur ^ 1], q.b, true, q.a, true, nullptr);
             } else {
-              launch_step2<float>(c, L, c->d_u[c->cur], c->d_u[c->cur ^ 1], q.a, q.b);
+              rc = launch_step2<float>(c, L, c->d_u[c->cur], c->d_u[c->cur ^ 1], q.a, q.b);
               launch_bridge<float>(c, c->d_u[c->cur ^ 1], q.b, true, q.a, true, nullptr);
             }
           };
           go();
+          if (rc != CS_OK) goto done;
           if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = set_err(CS_EDEVICE, "event record failed"); goto done; }
           for (uint32_t r = 0; r < reps; r++) go();
           if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
@@ -2769,6 +2828,7 @@ done:
   if (rc != CS_OK) return rc;
   HIP_TRY(hipGetLastError());
   c->launch = winner;
+  c->auto_form = false;
   if (best) cs_get_launch_config(c, best);
   if (best_ms) *best_ms = wms;
   return CS_OK;

@@ -221,18 +221,22 @@ int cs_fused_available(const cs_context* ctx, char* why, size_t why_len);
  * or 4), a block is `rows` wavefronts side by side along x (1 to 8) and x
  * neighbours move between lanes by DPP.  fuse = 1 runs each pair of
  * consecutive steps whose flux species (and species 0, with channels)
- * diffuse on both steps as one two-step pass (k_step2): a block computes
+ * diffuse on both steps as one two-step pass: a block computes
  * the first step on its tile plus a one-voxel ring and the second on the
  * tile, so the intermediate state stays on chip and the fields cross HBM
  * once per two steps; fuse_zchunk is its planes per block and fuse_xcd
  * its tile order (as xcd_remap).  The other steps, and every step with
  * fuse = 0, run one at a time.  cs_create sets fuse = 1 for FP32 fields
  * when the problem admits fused passes and their launch has at least
- * half as many blocks as the device has CUs, else 0.  fuse_fixed = 1 (the default) runs the
- * pairs of step masks of the reference's five-slot species layout (Ca,
- * dye, CMDN-CSQN, ATP, TRPN) in FP32 with kernels compiled for those
- * masks; 0 runs every pass with the masks read at run time (same
- * results to FP32 rounding).  No reference counterpart: the reference's
+ * half as many blocks as the device has CUs, else 0; until
+ * cs_set_launch_config or cs_autotune chooses a shape, models of the
+ * reference's five-slot species layout (Ca, dye, CMDN-CSQN, ATP, TRPN; Ca
+ * and ATP diffusing on every step, TRPN on none) run two-step passes
+ * whatever fuse says, since there they are the faster form at every size
+ * and in both precisions.  fuse_fixed = 1 (the default) runs that layout's
+ * passes with kernels compiled for each pair of step masks (k_pass2); 0
+ * runs every pass with the masks read at run time (k_step2; same results
+ * to rounding).  No reference counterpart: the reference's
  * OpenMP/AVX-512 loop has no launch shape (kernel_generic.cpp:561-600). */
 typedef struct cs_launch_config {
   uint32_t rows, zchunk, xcd_remap, prefetch, nontemporal, lds_tile, linear, yblock;
