@@ -19,7 +19,12 @@
  *   k_batch_bridge   one wavefront per realisation: the boundary fluxes of
  *                    step t added to the new state (k_flux's rows and
  *                    order) and then the gating of step t+1 from that
- *                    state (k_gate's gate_one), so a step is two launches.
+ *                    state (k_gate's gate_one), so a step is two launches;
+ *   k_pass2          two steps of every realisation of the five-slot
+ *                    layout in one pass (k_pass2.h), with k_batch_bridge2's
+ *                    gating and fluxes around it: steps run in pairs, and
+ *                    the kernels above take a single last step, and models
+ *                    of other layouts.
  *
  * Fields of realisation i live at their own offset of one stacked buffer
  * (two of them ping-pong), each in the single-domain layout [z][species]
@@ -43,10 +48,13 @@
 #include "csparks.h"
 #include "cs_device.h"
 #include "cs_mlp.h"
+#include "cs_pass2.h"
 
 namespace {
 
 constexpr int BRIDGE_BATCH_THREADS = 64;   /* one wavefront per realisation */
+constexpr int BRIDGE2_THREADS = 256;
+constexpr bool P2_HALF = false;            /* two-step passes: blocks of half a compute unit */
 constexpr int BSTAT_THREADS = 256;
 constexpr int NQUEUE = 8;                  /* one work queue per XCD        */
 
@@ -84,6 +92,7 @@ struct BatchChan {
   uint64_t elem_to;
   double rest_to;
   uint32_t flux, ch, state, uni;
+  uint32_t slot_to, pad;   /* level-1 slot of the cleft voxel */
 };
 
 /* Where a channel sits, for the closure's features: its realisation, the
@@ -95,6 +104,10 @@ struct BatchChanGeo {
   uint64_t elem_from;
   double rest_from;
 };
+
+/* Voxels whose Ca a closure reads per channel: the 27 around its cleft
+ * voxel, and its SR voxel. */
+constexpr uint32_t CLOSURE_NEAR = 28;
 
 /* Neighbour entries of a channel: state slot of a channel of the same
  * realisation whose cleft voxel lies within Chebyshev distance 2 in the
@@ -261,16 +274,113 @@ k_batch_bridge(const T* __restrict__ u, T* __restrict__ un, const DevParams<T>* 
   if (threadIdx.x == 0 && open) last_open[i] = gti;
 }
 
+/* A step's part in k_batch_bridge2: its fluxes, and its gating (time index
+ * relative to ti_base, first draw). */
+struct Bridge2Step {
+  uint32_t on, fluxmask, gate, pad;
+  uint64_t ti, uni_base;
+};
+
+/* Channel gating and boundary fluxes around two-step passes, one block per
+ * active realisation, in k_bridge's phases: the tail after a pass over
+ * steps t, t+1 gates step t+1 on the pass's level-1 values of species 0 and
+ * adds that step's fluxes, formed from them, to u; the head before a pass
+ * gates its first step on u and sums that step's fluxes per pair voxel for
+ * the pass to add.  Gating, entry order and skip rules are k_batch_bridge's;
+ * cpred and fpred as there.  What bounds it is the chain of dependent reads
+ * (record, then state, then field), so rows and channels run over four
+ * wavefronts.  Gating and fluxes of 512 dyads of 9 to 100 channels, with
+ * the launch's gap, take 18 us per two steps, where k_batch_bridge's one
+ * wavefront took 19 us per step. */
+template <typename T>
+__global__ void __launch_bounds__(BRIDGE2_THREADS)
+k_batch_bridge2(T* __restrict__ u, const T* __restrict__ l1, double* __restrict__ fsum,
+                const DevParams<T>* __restrict__ P, const BatchInst* __restrict__ insts,
+                const uint8_t* __restrict__ active, const BatchChan* __restrict__ chans,
+                const BRow* __restrict__ rows, const BEnt* __restrict__ ents, uint8_t* __restrict__ states,
+                uint8_t* __restrict__ recruited, uint64_t* __restrict__ last_open, Bridge2Step tail,
+                Bridge2Step head, const uint64_t* __restrict__ ti_base, uint32_t D,
+                const double* __restrict__ uniforms, const double* __restrict__ cpred,
+                const double* __restrict__ fpred)
+{
+  const uint32_t i = blockIdx.x;
+  if (!active[i]) return;
+  const BatchInst in = insts[i];
+  const double dt = P->dt, h = P->h, dts = dt * D;
+  const uint64_t base = ti_base ? *ti_base : 0;
+  auto gate = [&](const Bridge2Step& st, auto ca) {
+    const uint64_t gti = base + st.ti;
+    const double t = (double)gti * dt;
+    int open = 0;
+    for (uint32_t c = threadIdx.x; c < in.nchan; c += blockDim.x) {
+      const BatchChan b = chans[in.chan_off + c];
+      const FluxParams& F = P->flux[b.flux];
+      const double c0 = !F.stochastic ? 0.0 : cpred ? cpred[in.chan_off + c] : ca(b) + b.rest_to;
+      const double* draw = (uniforms && b.uni != NO_ROW) ? uniforms + st.uni_base + in.uni_off + b.uni : nullptr;
+      const uint8_t sv = gate_one(F, states[b.state], c0, gti, t, dts, in.seed, in.instance, draw, b.ch);
+      states[b.state] = sv;
+      if (sv) {
+        recruited[b.state] = 1;
+        open = 1;
+      }
+    }
+    /* the latest gating step that left a channel of the realisation open;
+     * the states are written before the fluxes read them */
+    open = __syncthreads_or(open);
+    if (threadIdx.x == 0 && open) last_open[i] = gti;
+  };
+  auto row_flux = [&](const BRow& w, uint32_t fluxmask, auto val, double& sum) -> bool {
+    sum = 0.0;
+    bool any = false;
+    for (uint32_t e = w.start; e < w.end && !w.skip; e++) {
+      const BEnt x = ents[e];
+      const uint32_t f = x.flux_sign & 0xFFu;
+      if (!((fluxmask >> f) & 1u)) continue;
+      if (x.state != NO_ROW && !states[x.state]) continue;
+      double J = flux_j(P->flux[f], val(x, false), val(x, true), x.rest_from, x.rest_to, dt, h);
+      if (fpred && x.state != NO_ROW) J *= fpred[x.state];
+      sum += (x.flux_sign >> 8) ? J : -J;
+      any = true;
+    }
+    return any;
+  };
+  if (tail.on) {
+    if (tail.gate) gate(tail, [&](const BatchChan& b) { return (double)l1[b.slot_to]; });
+    if (tail.fluxmask)
+      for (uint32_t r = in.row_off + threadIdx.x; r < in.row_off + in.nrows; r += blockDim.x) {
+        const BRow w = rows[r];
+        double sum;
+        if (row_flux(w, tail.fluxmask,
+                     [&](const BEnt& x, bool to) { return (double)l1[to ? x.slot_to : x.slot_from]; }, sum))
+          u[w.elem] = (T)((double)u[w.elem] + sum);
+      }
+    __syncthreads();   /* the fluxes are in u before the head reads it */
+  }
+  if (head.on) {
+    if (head.gate) gate(head, [&](const BatchChan& b) { return (double)u[b.elem_to]; });
+    for (uint32_t r = in.row_off + threadIdx.x; r < in.row_off + in.nrows; r += blockDim.x) {
+      const BRow w = rows[r];
+      double sum;
+      const bool any = row_flux(w, head.fluxmask,
+                                [&](const BEnt& x, bool to) { return (double)u[to ? x.elem_to : x.elem_from]; }, sum);
+      fsum[w.slot] = any ? sum : 0.0;
+    }
+  }
+}
+
 /* The closure's raw input k of channel c: the absolute Ca of the 3x3x3
  * coarse voxels around its cleft voxel (k = 9 (dz+1) + 3 (dy+1) + dx+1,
  * clamped at the grid faces), the absolute Ca of its SR voxel (27), and
  * the open channels within Chebyshev distance 1 (28) and 2 (29) in the
- * cleft plane, itself included; 0 for the padding inputs 30, 31. */
+ * cleft plane, itself included; 0 for the padding inputs 30, 31.  With
+ * near, u holds level-1 values of species 0 by slot and near[28 c + k] is
+ * the slot of input k's voxel. */
 template <typename T>
 __device__ inline float closure_raw(int k, uint32_t c, const BatchChanGeo& cg, const BatchGeo& gg,
                                     const T* __restrict__ u, const uint8_t* __restrict__ ids,
                                     const DevParams<T>* __restrict__ P, const uint8_t* __restrict__ states,
-                                    const uint32_t* __restrict__ nb_start, const uint32_t* __restrict__ nb)
+                                    const uint32_t* __restrict__ nb_start, const uint32_t* __restrict__ nb,
+                                    const uint32_t* __restrict__ near = nullptr)
 {
   if (k < 27) {
     const int x = min(max(cg.x + k % 3 - 1, 0), gg.nx - 1);
@@ -278,9 +388,10 @@ __device__ inline float closure_raw(int k, uint32_t c, const BatchChanGeo& cg, c
     const int z = min(max(cg.z + k / 9 - 1, 0), gg.nz - 1);
     const uint64_t col = (uint64_t)y * gg.nx + x;
     const int d = ids[gg.id_off + (uint64_t)z * gg.plane + col] & 7;
-    return (float)((double)u[gg.u_off + (uint64_t)z * gg.ns * gg.plane + col] + P->init64[d][0]);
+    const uint64_t at = near ? near[CLOSURE_NEAR * c + k] : gg.u_off + (uint64_t)z * gg.ns * gg.plane + col;
+    return (float)((double)u[at] + P->init64[d][0]);
   }
-  if (k == 27) return (float)((double)u[cg.elem_from] + cg.rest_from);
+  if (k == 27) return (float)((double)u[near ? near[CLOSURE_NEAR * c + k] : cg.elem_from] + cg.rest_from);
   if (k == 28 || k == 29) {
     uint32_t n = 0;
     for (uint32_t e = nb_start[c]; e < nb_start[c + 1]; e++) {
@@ -358,8 +469,8 @@ k_closure_predict(const T* __restrict__ u, const uint8_t* __restrict__ ids, cons
                   const MlpDev* __restrict__ N, const MlpDev* __restrict__ F, const BatchGeo* __restrict__ geos,
                   const uint8_t* __restrict__ active, const BatchChanGeo* __restrict__ cgeo,
                   const uint8_t* __restrict__ states, const uint32_t* __restrict__ nb_start,
-                  const uint32_t* __restrict__ nb, uint32_t nchan, double* __restrict__ cpred,
-                  double* __restrict__ fpred, uint32_t* __restrict__ flags)
+                  const uint32_t* __restrict__ nb, const uint32_t* __restrict__ near, uint32_t nchan,
+                  double* __restrict__ cpred, double* __restrict__ fpred, uint32_t* __restrict__ flags)
 {
   const int lane = threadIdx.x & 63, g = lane >> 5;
   const uint64_t tile = (uint64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
@@ -403,7 +514,7 @@ k_closure_predict(const T* __restrict__ u, const uint8_t* __restrict__ ids, cons
       feat[ch][j] = !valid ? 0.0f
                  : k == 28 ? (float)n1
                  : k == 29 ? (float)n2
-                 : closure_raw<T>(k, cc, cg, gg, u, ids, P, states, nb_start, nb);
+                 : closure_raw<T>(k, cc, cg, gg, u, ids, P, states, nb_start, nb, near);
       feat[ch][j] = closure_feature(k, feat[ch][j]);   /* once, for both networks */
     }
   auto predict = [&](const MlpDev* __restrict__ M, bool& oor) {
@@ -642,8 +753,33 @@ struct cs_batch {
   uint32_t substeps[MAXS] = {0};
   uint32_t flux_substep[MAXF] = {0};
   uint32_t ndiscrete = 0;
-  uint32_t rfast = 0;
+  uint32_t rfast = 0, rbound = 0;
   uint32_t fsm = 0;
+  /* two-step passes: whether the model and every grid admit them (p2_ok),
+   * whether they run (autotune may find one-step passes faster), a record
+   * and a split per realisation, the tiles of the active
+   * ones, the kept voxels (pair voxels, and with near_ok those around the
+   * channels) by column, and what the passes keep there */
+  bool p2_ok = false, p2_on = false, near_ok = false;
+  std::vector<P2Split> p2_split;
+  P2Geo* d_p2_geo = nullptr;
+  P2Tile* d_p2_tiles = nullptr;
+  uint32_t n_p2_tiles = 0, cap_p2_tiles = 0;
+  int p2_xcd = 0, cus = 1;
+  uint32_t* d_p2_col = nullptr;
+  uint32_t* d_p2_z = nullptr;
+  double* d_p2_fsum = nullptr;
+  void* d_p2_l1 = nullptr;
+  uint32_t* d_near = nullptr;              /* CLOSURE_NEAR slots per channel   */
+  /* host copies of the records that name slots */
+  std::vector<std::vector<uint32_t>> h_pairs;   /* pair voxels per realisation */
+  std::vector<BatchInst> h_inst;
+  std::vector<BatchChan> h_chan;
+  std::vector<BatchChanGeo> h_cgeo;
+  std::vector<BRow> h_rows;
+  std::vector<BEnt> h_ents;
+  std::vector<uint32_t> row_voxel, ent_voxel;   /* per row; from, to per entry */
+  std::vector<uint8_t> h_active;
   /* launch shape */
   cs_batch_launch launch{4, 32, 1, 1, 0};
   int tile_xcd = 0;                        /* k_batch_tiles' XCD groups       */
@@ -651,7 +787,8 @@ struct cs_batch {
   /* captured step periods, keyed by (phase within the period, buffer) */
   bool use_graph = false;
   uint64_t* d_ti = nullptr;
-  std::map<std::pair<uint64_t, int>, hipGraphExec_t> graphs;
+  struct Graph { hipGraphExec_t exec; int cur; };   /* and the buffer it ends in */
+  std::map<std::pair<uint64_t, int>, Graph> graphs;
   std::vector<hipGraph_t> graph_defs;
 };
 
@@ -661,12 +798,13 @@ void free_batch(cs_batch* b)
 {
   if (!b) return;
   (void)hipSetDevice(b->device);
-  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
+  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second.exec);
   for (auto g : b->graph_defs) (void)hipGraphDestroy(g);
   void* ptrs[] = {b->d_u[0], b->d_u[1], b->d_ids, b->d_params, b->d_geo, b->d_tiles, b->d_queue, b->d_inst,
                   b->d_chan, b->d_rows, b->d_ents, b->d_states, b->d_recruited, b->d_active, b->d_last_open,
                   b->d_cgeo, b->d_nb_start, b->d_nb, b->d_cpred, b->d_fpred, b->d_chca, b->d_feat, b->d_flags,
-                  b->d_uniforms, b->d_stats, b->d_lw, b->d_lpart, b->d_lproj, b->d_loff, b->d_ti};
+                  b->d_uniforms, b->d_stats, b->d_lw, b->d_lpart, b->d_lproj, b->d_loff, b->d_ti,
+                  b->d_p2_geo, b->d_p2_tiles, b->d_p2_col, b->d_p2_z, b->d_p2_fsum, b->d_p2_l1, b->d_near};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -743,6 +881,167 @@ int upload_tiles(cs_batch* b)
   b->tile_xcd = 0;
   for (int G = 16; G >= 2; G /= 2)
     if ((int64_t)b->ntiles >= 8LL * 3 * G) { b->tile_xcd = G; break; }
+  return CS_OK;
+}
+
+/* Whether two-step passes (k_pass2) fit the ensemble: the five-slot layout
+ * with its substeps, fluxes on Ca only, and on every grid at least two
+ * columns either way and a split whose blocks hold a tile.  Half blocks:
+ * planes of 43 to 171 columns a side leave little to gain from wider tiles
+ * (512 dyads at 6 nm 342 us per step and 338 with whole blocks, 8 dyads at
+ * 3 nm 155 and 158, 1024 dyads at 12 nm 368 and 382). */
+int setup_pass2(cs_batch* b)
+{
+  b->p2_ok = b->p2_on = false;
+  if (b->ns != 5 || !p2_substeps(b->substeps) || (b->model.num_buffers && (!b->rfast || b->rbound != 0x1Eu)) ||
+      (b->fsm & ~1u))
+    return CS_OK;
+  std::vector<P2Geo> recs;
+  uint64_t cols = 0;
+  b->p2_split.clear();
+  for (const BatchGeo& g : b->geo) {
+    if (g.nx < 2 || g.ny < 2 || g.nv * b->ns * b->esize >= (1ull << 32) - P2_PAD) return CS_OK;
+    const P2Split sp = p2_split((uint32_t)g.nx, (uint32_t)g.ny, b->esize, P2_HALF);
+    if (!sp.kx) return CS_OK;
+    b->p2_split.push_back(sp);
+    recs.push_back(P2Geo{g.u_off, g.id_off, (uint32_t)cols, (uint32_t)g.plane, g.nx, g.ny, g.nz, 0});
+    cols += g.plane + 1;
+  }
+  if (cols >= (1ull << 32)) return CS_OK;
+  HIP_TRY(hipMalloc(&b->d_p2_geo, sizeof(P2Geo) * recs.size()));
+  HIP_TRY(hipMemcpy(b->d_p2_geo, recs.data(), sizeof(P2Geo) * recs.size(), hipMemcpyHostToDevice));
+  b->p2_ok = b->p2_on = true;
+  return CS_OK;
+}
+
+/* The tiles of the active realisations: planes per block as p2_zparts finds
+ * for a grid as deep as the deepest and all their tiles. */
+int upload_pass2_tiles(cs_batch* b)
+{
+  if (!b->p2_ok) return CS_OK;
+  uint64_t cols = 0;
+  uint32_t deep = 1;
+  for (uint32_t i = 0; i < b->count; i++)
+    if (b->h_active[i]) {
+      cols += (uint64_t)b->p2_split[i].kx * b->p2_split[i].ky;
+      deep = std::max(deep, (uint32_t)b->geo[i].nz);
+    }
+  const uint32_t parts = p2_zparts(cols, deep, 2 * b->cus, deep);
+  const uint32_t zc = (deep + parts - 1) / parts;
+  std::vector<P2Tile> tiles;
+  for (uint32_t i = 0; i < b->count; i++)
+    if (b->h_active[i])
+      p2_tiles(i, (uint32_t)b->geo[i].nx, (uint32_t)b->geo[i].ny, (uint32_t)b->geo[i].nz, b->p2_split[i],
+               ((uint32_t)b->geo[i].nz + zc - 1) / zc, tiles);
+  for (const P2Tile& t : tiles)
+    if (!p2_fits(t, (uint32_t)b->geo[t.inst].nx, (uint32_t)b->geo[t.inst].ny, b->esize, P2_HALF))
+      return set_err(CS_EDEVICE, "a tile of %u x %u columns does not fit its block", t.w, t.h);
+  if (tiles.size() > b->cap_p2_tiles) {
+    if (b->d_p2_tiles) HIP_TRY(hipFree(b->d_p2_tiles));
+    b->d_p2_tiles = nullptr;
+    b->cap_p2_tiles = 0;
+    HIP_TRY(hipMalloc(&b->d_p2_tiles, sizeof(P2Tile) * tiles.size()));
+    b->cap_p2_tiles = (uint32_t)tiles.size();
+  }
+  if (!tiles.empty()) {
+    HIP_TRY(hipMemcpyAsync(b->d_p2_tiles, tiles.data(), sizeof(P2Tile) * tiles.size(), hipMemcpyHostToDevice,
+                           b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+  }
+  b->n_p2_tiles = (uint32_t)tiles.size();
+  b->p2_xcd = 0;
+  for (int G = 16; G >= 2; G /= 2)
+    if (tiles.size() >= 8ull * 3 * G) { b->p2_xcd = G; break; }
+  return CS_OK;
+}
+
+/* The voxels whose level-1 Ca the passes keep: those of the boundary pairs
+ * and, with near, those a closure reads.  Marks them in the ids, indexes
+ * them by column and plane, and gives every record its slots. */
+int index_kept_voxels(cs_batch* b, bool near)
+{
+  std::vector<uint32_t> col_start, vz, slots;
+  std::vector<uint8_t> ids(b->total_ids, 0);
+  if (near) slots.assign((size_t)CLOSURE_NEAR * b->h_chan.size(), 0);
+  for (uint32_t i = 0; i < b->count; i++) {
+    const BatchGeo& g = b->geo[i];
+    const BatchInst& in = b->h_inst[i];
+    auto key = [&g](uint64_t v) { return (v % g.plane) << 32 | v / g.plane; };
+    auto around = [&](uint32_t c, uint32_t k) -> uint64_t {
+      const BatchChanGeo& cg = b->h_cgeo[c];
+      if (k == 27) {
+        const uint64_t e = cg.elem_from - g.u_off, z = e / (g.plane * g.ns);
+        return z * g.plane + (e - z * g.plane * g.ns);
+      }
+      const int x = std::min(std::max(cg.x + (int)(k % 3) - 1, 0), g.nx - 1);
+      const int y = std::min(std::max(cg.y + (int)(k / 3) % 3 - 1, 0), g.ny - 1);
+      const int z = std::min(std::max(cg.z + (int)(k / 9) - 1, 0), g.nz - 1);
+      return (uint64_t)z * g.plane + (uint64_t)y * g.nx + x;
+    };
+    std::vector<uint64_t> keys;
+    for (uint32_t v : b->h_pairs[i]) keys.push_back(key(v));
+    if (near)
+      for (uint32_t c = in.chan_off; c < in.chan_off + in.nchan; c++)
+        for (uint32_t k = 0; k < CLOSURE_NEAR; k++) keys.push_back(key(around(c, k)));
+    std::sort(keys.begin(), keys.end());
+    keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
+    const uint32_t base = (uint32_t)vz.size();
+    const size_t c0 = col_start.size();
+    col_start.resize(c0 + g.plane + 1, 0);
+    for (uint8_t& id : b->h_ids[i]) id &= (uint8_t)~ID_PAIR;
+    for (uint64_t k : keys) {
+      const uint64_t col = k >> 32, z = k & 0xFFFFFFFFu;
+      vz.push_back((uint32_t)z);
+      col_start[c0 + col + 1]++;
+      b->h_ids[i][z * g.plane + col] |= ID_PAIR;
+    }
+    col_start[c0] = base;
+    for (uint64_t k = 1; k <= g.plane; k++) col_start[c0 + k] += col_start[c0 + k - 1];
+    memcpy(ids.data() + g.id_off, b->h_ids[i].data(), g.nv);
+    auto slot = [&](uint64_t v) {
+      return base + (uint32_t)(std::lower_bound(keys.begin(), keys.end(), key(v)) - keys.begin());
+    };
+    for (uint32_t c = in.chan_off; c < in.chan_off + in.nchan; c++) {
+      const BatchChanGeo& cg = b->h_cgeo[c];
+      b->h_chan[c].slot_to = slot((uint64_t)cg.z * g.plane + (uint64_t)cg.y * g.nx + cg.x);
+      if (near)
+        for (uint32_t k = 0; k < CLOSURE_NEAR; k++) slots[(size_t)CLOSURE_NEAR * c + k] = slot(around(c, k));
+    }
+    for (uint32_t r = in.row_off; r < in.row_off + in.nrows; r++) {
+      b->h_rows[r].slot = slot(b->row_voxel[r]);
+      for (uint32_t e = b->h_rows[r].start; e < b->h_rows[r].end; e++) {
+        b->h_ents[e].slot_from = slot(b->ent_voxel[2 * e]);
+        b->h_ents[e].slot_to = slot(b->ent_voxel[2 * e + 1]);
+      }
+    }
+  }
+  for (void** p : {(void**)&b->d_p2_col, (void**)&b->d_p2_z, (void**)&b->d_p2_fsum, &b->d_p2_l1, (void**)&b->d_near}) {
+    if (*p) HIP_TRY(hipFree(*p));
+    *p = nullptr;
+  }
+  const size_t n = std::max<size_t>(vz.size(), 1);
+  HIP_TRY(hipMalloc(&b->d_p2_col, sizeof(uint32_t) * col_start.size()));
+  HIP_TRY(hipMalloc(&b->d_p2_z, sizeof(uint32_t) * n));
+  HIP_TRY(hipMalloc(&b->d_p2_fsum, sizeof(double) * n));
+  HIP_TRY(hipMalloc(&b->d_p2_l1, b->esize * n));
+  if (near) HIP_TRY(hipMalloc(&b->d_near, sizeof(uint32_t) * std::max<size_t>(slots.size(), 1)));
+  const std::vector<double> zero(n, 0.0);   /* voxels without a row keep a zero sum */
+  auto up = [b](void* dst, const void* src, size_t bytes) -> int {
+    if (bytes) HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream));
+    return CS_OK;
+  };
+  int rc;
+  if ((rc = up(b->d_p2_col, col_start.data(), sizeof(uint32_t) * col_start.size())) != CS_OK ||
+      (rc = up(b->d_p2_z, vz.data(), sizeof(uint32_t) * vz.size())) != CS_OK ||
+      (rc = up(b->d_p2_fsum, zero.data(), sizeof(double) * n)) != CS_OK ||
+      (rc = up(b->d_near, slots.data(), sizeof(uint32_t) * slots.size())) != CS_OK ||
+      (rc = up(b->d_ids, ids.data(), ids.size())) != CS_OK ||
+      (rc = up(b->d_chan, b->h_chan.data(), sizeof(BatchChan) * b->h_chan.size())) != CS_OK ||
+      (rc = up(b->d_rows, b->h_rows.data(), sizeof(BRow) * b->h_rows.size())) != CS_OK ||
+      (rc = up(b->d_ents, b->h_ents.data(), sizeof(BEnt) * b->h_ents.size())) != CS_OK)
+    return rc;
+  HIP_TRY(hipStreamSynchronize(b->stream));   /* the host vectors end here */
+  b->near_ok = near;
   return CS_OK;
 }
 
@@ -846,31 +1145,126 @@ void launch_bbridge(cs_batch* b, const void* u, void* un, const BridgeArgs& a, c
  * network's mouth Ca (with the range monitor) and, when set, the flux
  * network's release ratios. */
 template <typename T>
-void launch_predict(cs_batch* b, const void* u)
+void launch_predict(cs_batch* b, const void* u, const uint32_t* near = nullptr)
 {
   const unsigned blocks = (b->nchan_total + 127) / 128;
   if (!blocks) return;
   hipLaunchKernelGGL(k_closure_predict<T>, dim3(blocks), dim3(256), 0, b->stream, (const T*)u, b->d_ids,
                      (const DevParams<T>*)b->d_params, b->d_net, b->d_fnet, b->d_geo, b->d_active, b->d_cgeo,
-                     b->d_states, b->d_nb_start, b->d_nb, b->nchan_total, b->d_cpred, b->d_fpred, b->d_flags);
+                     b->d_states, b->d_nb_start, b->d_nb, near, b->nchan_total, b->d_cpred, b->d_fpred, b->d_flags);
 }
 
-/* Steps [first, first + n) on the stream: gating of the first step, then
+int launch_bpass2(cs_batch* b, const void* uin, void* uout, uint64_t ti)
+{
+  P2Args p{};
+  p.u = uin;
+  p.un = uout;
+  p.ids = b->d_ids;
+  p.params = b->d_params;
+  p.geos = b->d_p2_geo;
+  p.tiles = b->d_p2_tiles;
+  p.col_start = b->d_p2_col;
+  p.vz = b->d_p2_z;
+  p.fsum = b->d_p2_fsum;
+  p.l1 = b->d_p2_l1;
+  p.ntiles = b->n_p2_tiles;
+  p.xcd = b->p2_xcd;
+  const uint32_t m1 = b_diffusing(b, ti), m2 = b_diffusing(b, ti + 1);
+  p.react1 = b_react(b, ti, m1) ? 1u : 0u;
+  p.react2 = b_react(b, ti + 1, m2) ? 1u : 0u;
+  for (uint32_t d = 0; d < b->nd; d++)
+    for (uint32_t s = 0; s < b->ns; s++) p.any_fixed |= b->model.fixed[d][s] ? 1u : 0u;
+  if (p.ntiles && !cs_internal_pass2(b->esize, P2_HALF, m1, m2, p, b->stream))
+    return set_err(CS_EDEVICE, "no two-step pass for masks %x, %x", m1, m2);
+  return CS_OK;
+}
+
+/* Whether steps run in pairs: two-step passes are on and, when a closure
+ * gates, the passes keep what it reads. */
+bool b_pairs(const cs_batch* b) { return b->p2_on && (b->gating != CS_GATE_CLOSURE || b->near_ok); }
+
+/* Steps [first, first + n) in pairs (n even): per pair the pass and the
+ * bridge (the second step's gating and fluxes, then the next pair's first
+ * gating and flux sums).  With a closure the tail and the head are
+ * launches of their own, each after the predictions from the state it
+ * gates on (with the flux network every state is predicted from, since
+ * its fluxes read the ratios).  gate_idx counts gating steps; ev and d_ti
+ * as in b_run. */
+template <typename T>
+int b_run_pairs(cs_batch* b, uint64_t first, uint64_t n, const double* d_uni, hipEvent_t* ev, const uint64_t* d_ti,
+                uint64_t& gate_idx)
+{
+  const bool closure = b->gating == CS_GATE_CLOSURE, fclosure = closure && b->d_fnet;
+  auto part = [&](uint64_t ti) {
+    Bridge2Step s{};
+    s.on = 1;
+    s.fluxmask = b->nf ? b_fluxmask(b, ti) : 0u;
+    s.gate = (b->gating != CS_GATE_REPLAY && b_gates(b, ti)) ? 1u : 0u;
+    s.ti = d_ti ? ti - first : ti;
+    s.uni_base = d_uni ? gate_idx * b->uni_stride : 0;
+    if (s.gate) gate_idx++;
+    return s;
+  };
+  auto launch = [&](const Bridge2Step& tail, const Bridge2Step& head, void* u) {
+    hipLaunchKernelGGL(k_batch_bridge2<T>, dim3(b->count), dim3(BRIDGE2_THREADS), 0, b->stream, (T*)u,
+                       (const T*)b->d_p2_l1, b->d_p2_fsum, (const DevParams<T>*)b->d_params, b->d_inst, b->d_active,
+                       b->d_chan, b->d_rows, b->d_ents, b->d_states, b->d_recruited, b->d_last_open, tail, head, d_ti,
+                       b->model.stochastic_substep, d_uni, closure ? b->d_cpred : nullptr,
+                       fclosure ? b->d_fpred : nullptr);
+  };
+  auto bridge = [&](const Bridge2Step& tail, const Bridge2Step& head, void* u) {
+    if (!closure) return launch(tail, head, u);
+    const Bridge2Step none{};
+    if (tail.on) {
+      if (tail.gate || fclosure) launch_predict<T>(b, b->d_p2_l1, b->d_near);
+      launch(tail, none, u);
+    }
+    if (head.gate || fclosure) launch_predict<T>(b, u);
+    if (head.on) launch(none, head, u);
+  };
+  bridge(Bridge2Step{}, part(first), b->d_u[b->cur]);
+  for (uint64_t i = 0; i < n; i += 2) {
+    if (ev) HIP_TRY(hipEventRecord(ev[i], b->stream));
+    const int rc = launch_bpass2(b, b->d_u[b->cur], b->d_u[b->cur ^ 1], first + i);
+    if (rc != CS_OK) return rc;
+    if (ev) HIP_TRY(hipEventRecord(ev[i + 1], b->stream));
+    const Bridge2Step tail = part(first + i + 1);
+    const Bridge2Step head = i + 2 < n ? part(first + i + 2) : Bridge2Step{};
+    b->cur ^= 1;
+    bridge(tail, head, b->d_u[b->cur]);
+  }
+  HIP_TRY(hipGetLastError());
+  return CS_OK;
+}
+
+/* Steps [first, first + n) on the stream: in pairs where two-step passes
+ * run; what is left, step by step: gating of the first step, then
  * per step the stencil pass and the bridge (its fluxes, and the gating of
  * the next step unless it is the last).  ev, when given, holds 2n events
- * that bracket every stencil launch.  With d_ti (a captured range), the
- * bridges read the first time index from the device and carry offsets. */
+ * of which pairs bracket the passes, *npasses of them.  With d_ti (a
+ * captured range), the bridges read the first time index from the device
+ * and carry offsets. */
 template <typename T>
 int b_run(cs_batch* b, uint64_t first, uint64_t n, const double* d_uni, hipEvent_t* ev,
-          const uint64_t* d_ti = nullptr)
+          const uint64_t* d_ti = nullptr, uint64_t* npasses = nullptr)
 {
   const uint32_t D = b->model.stochastic_substep;
   uint64_t gate_idx = 0;
+  const uint64_t first0 = first;
+  const uint64_t paired = b_pairs(b) ? n / 2 * 2 : 0;
+  if (npasses) *npasses = paired / 2 + (n - paired);
+  if (paired) {
+    const int rc = b_run_pairs<T>(b, first, paired, d_uni, ev, d_ti, gate_idx);
+    if (rc != CS_OK) return rc;
+    first += paired;
+    n -= paired;
+    if (ev) ev += paired;
+  }
   auto bridge = [&](uint32_t fluxmask, uint64_t gti, bool gate_next, const void* u, void* un) {
     BridgeArgs a{};
     a.fluxmask = fluxmask;
     a.gate = (gate_next && b->gating != CS_GATE_REPLAY && b_gates(b, gti)) ? 1u : 0u;
-    a.gate_ti = d_ti ? gti - first : gti;
+    a.gate_ti = d_ti ? gti - first0 : gti;
     a.ti_base = d_ti;
     a.uni_base = d_uni ? gate_idx * b->uni_stride : 0;
     a.D = D;
@@ -968,7 +1362,8 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
   /* whole periods of the step pattern replay one captured graph each; the
    * rest runs directly.  The captured bridges read the period's first
    * time index from d_ti, set before every replay.  A period holds an even
-   * number of steps, so it leaves the ping-pong buffers as it found them. */
+   * number of steps; in two-step passes it may still end in the other
+   * ping-pong buffer, which its record keeps. */
   uint64_t P = b_period(b);
   if (P % 2) P *= 2;
   uint64_t done = 0;
@@ -981,6 +1376,7 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
       HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
       const int cur0 = b->cur;
       const int rc = b_run<T>(b, ti, P, nullptr, nullptr, b->d_ti);
+      const int cur1 = b->cur;
       b->cur = cur0;
       const hipError_t e = hipStreamEndCapture(b->stream, &g);
       if (rc != CS_OK) {
@@ -995,11 +1391,12 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
         return set_err(CS_EDEVICE, "graph instantiation failed: %s", hipGetErrorString(ei));
       }
       b->graph_defs.push_back(g);
-      it = b->graphs.emplace(key, ex).first;
+      it = b->graphs.emplace(key, cs_batch::Graph{ex, cur1}).first;
     }
     hipLaunchKernelGGL(k_batch_set_ti, dim3(1), dim3(64), 0, b->stream, b->d_ti, ti);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipGraphLaunch(it->second, b->stream));
+    HIP_TRY(hipGraphLaunch(it->second.exec, b->stream));
+    b->cur = it->second.cur;
     done += P;
   }
   if (done < n) return b_run<T>(b, first + done, n - done, nullptr, nullptr);
@@ -1008,7 +1405,7 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
 
 void drop_graphs(cs_batch* b)
 {
-  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
+  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second.exec);
   for (auto g : b->graph_defs) (void)hipGraphDestroy(g);
   b->graphs.clear();
   b->graph_defs.clear();
@@ -1185,7 +1582,7 @@ int cs_batch_create(const cs_problem* problems, uint32_t count, cs_batch** out)
       for (uint32_t k = 0; k < F.num_pairs; k++) {
         const uint32_t from = pairs_dev[2 * (pair_off[f] + k)], to = pairs_dev[2 * (pair_off[f] + k) + 1];
         const uint32_t st = (uint32_t)b->init_states.size();
-        chans.push_back(BatchChan{elem_of(0, to), p.init[dom(to)][0], f, k, st, stochastic ? ndraw++ : NO_ROW});
+        chans.push_back(BatchChan{elem_of(0, to), p.init[dom(to)][0], f, k, st, stochastic ? ndraw++ : NO_ROW, 0, 0});
         cgeo.push_back(BatchChanGeo{i, (int)(to % n0), (int)((to / n0) % n1), (int)(to / g.plane), elem_of(0, from),
                                     p.init[dom(from)][0]});
         b->init_states.push_back(F.init_states[k] ? 1 : 0);
@@ -1219,11 +1616,17 @@ int cs_batch_create(const cs_problem* problems, uint32_t count, cs_batch** out)
         ents.push_back(BEnt{elem_of(sp, from), elem_of(sp, to), p.init[dom(from)][sp], p.init[dom(to)][sp], NO_ROW,
                             NO_ROW, p.fluxes[f].discrete ? b->flux_state_off[i][f] + es[e].pair : NO_ROW,
                             f | (es[e].sign > 0 ? 1u : 0u) << 8});
+        b->ent_voxel.push_back(from);
+        b->ent_voxel.push_back(to);
       }
+      b->row_voxel.push_back(v);
       rows.push_back(BRow{elem_of(sp, v), start, (uint32_t)ents.size(), skip ? 1u : 0u, 0});
       k = e2;
     }
     in.nrows = (uint32_t)rows.size() - in.row_off;
+    std::sort(pairs_dev.begin(), pairs_dev.end());
+    pairs_dev.erase(std::unique(pairs_dev.begin(), pairs_dev.end()), pairs_dev.end());
+    b->h_pairs.push_back(std::move(pairs_dev));
   }
   b->total_elems = uoff;
   b->total_ids = idoff;
@@ -1236,10 +1639,11 @@ int cs_batch_create(const cs_problem* problems, uint32_t count, cs_batch** out)
   };
   int rc;
   if (hipMalloc(&b->d_ids, std::max<uint64_t>(idoff, 16)) != hipSuccess ||
-      hipMalloc(&b->d_u[0], std::max<uint64_t>(uoff * b->esize, 16)) != hipSuccess ||
-      hipMalloc(&b->d_u[1], std::max<uint64_t>(uoff * b->esize, 16)) != hipSuccess)
+      hipMalloc(&b->d_u[0], uoff * b->esize + P2_PAD) != hipSuccess ||
+      hipMalloc(&b->d_u[1], uoff * b->esize + P2_PAD) != hipSuccess)
     return bail(set_err(CS_ENOMEM, "device allocation of %llu field bytes failed",
                         (unsigned long long)(2 * uoff * b->esize)));
+  ids_all.resize(idoff);
   if (hipMemcpyAsync(b->d_ids, ids_all.data(), ids_all.size(), hipMemcpyHostToDevice, b->stream) != hipSuccess)
     return bail(set_err(CS_EDEVICE, "upload of ids failed"));
   if ((rc = upload((void**)&b->d_geo, b->geo.data(), sizeof(BatchGeo) * count)) != CS_OK ||
@@ -1253,8 +1657,8 @@ int cs_batch_create(const cs_problem* problems, uint32_t count, cs_batch** out)
       (rc = upload((void**)&b->d_states, b->init_states.data(), b->init_states.size())) != CS_OK ||
       (rc = upload((void**)&b->d_recruited, b->init_states.data(), b->init_states.size())) != CS_OK)
     return bail(rc);
-  std::vector<uint8_t> act(count, 1);
-  if ((rc = upload((void**)&b->d_active, act.data(), count)) != CS_OK) return bail(rc);
+  b->h_active.assign(count, 1);
+  if ((rc = upload((void**)&b->d_active, b->h_active.data(), count)) != CS_OK) return bail(rc);
   if (hipMalloc(&b->d_last_open, sizeof(uint64_t) * count) != hipSuccess ||
       hipMalloc(&b->d_flags, sizeof(uint32_t) * count) != hipSuccess ||
       hipMalloc(&b->d_cpred, sizeof(double) * std::max<size_t>(chans.size(), 1)) != hipSuccess ||
@@ -1270,17 +1674,30 @@ int cs_batch_create(const cs_problem* problems, uint32_t count, cs_batch** out)
     DevParams<double> dp;
     fill_params<double>(dp, &problems[0], b->ndiscrete);
     b->rfast = dp.rfast;
+    b->rbound = dp.rbound;
     if ((rc = upload(&b->d_params, &dp, sizeof dp)) != CS_OK) return bail(rc);
     if (hipStreamSynchronize(b->stream) != hipSuccess) return bail(set_err(CS_EDEVICE, "upload failed"));
   } else {
     DevParams<float> dp;
     fill_params<float>(dp, &problems[0], b->ndiscrete);
     b->rfast = dp.rfast;
+    b->rbound = dp.rbound;
     if ((rc = upload(&b->d_params, &dp, sizeof dp)) != CS_OK) return bail(rc);
     if (hipStreamSynchronize(b->stream) != hipSuccess) return bail(set_err(CS_EDEVICE, "upload failed"));
   }
+  hipDeviceProp_t prop;
+  if (hipGetDeviceProperties(&prop, b->device) != hipSuccess) return bail(set_err(CS_EDEVICE, "device query failed"));
+  b->cus = std::max(prop.multiProcessorCount, 1);
   rc = b->esize == 8 ? upload_tiles<double>(b) : upload_tiles<float>(b);
-  if (rc != CS_OK) return bail(rc);
+  if (rc != CS_OK || (rc = setup_pass2(b)) != CS_OK) return bail(rc);
+  if (b->p2_ok) {
+    b->h_inst.swap(insts);
+    b->h_chan.swap(chans);
+    b->h_cgeo.swap(cgeo);
+    b->h_rows.swap(rows);
+    b->h_ents.swap(ents);
+    if ((rc = index_kept_voxels(b, false)) != CS_OK || (rc = upload_pass2_tiles(b)) != CS_OK) return bail(rc);
+  }
   rc = cs_batch_reset(b);
   if (rc != CS_OK) return bail(rc);
   *out = b;
@@ -1355,6 +1772,10 @@ int cs_batch_upload_species(cs_batch* b, uint32_t inst, uint32_t s, const double
   const size_t pb = g.plane * b->esize;
   char* base = (char*)b->d_u[b->cur] + (g.u_off + (uint64_t)s * g.plane) * b->esize;
   HIP_TRY(hipMemcpy2DAsync(base, pb * b->ns, buf.data(), pb, pb, (size_t)g.nz, hipMemcpyHostToDevice, b->stream));
+  if (!b->h_active[inst]) {   /* a retired realisation's state is in both buffers */
+    char* other = (char*)b->d_u[b->cur ^ 1] + (base - (char*)b->d_u[b->cur]);
+    HIP_TRY(hipMemcpy2DAsync(other, pb * b->ns, buf.data(), pb, pb, (size_t)g.nz, hipMemcpyHostToDevice, b->stream));
+  }
   HIP_TRY(hipStreamSynchronize(b->stream));
   return CS_OK;
 }
@@ -1561,6 +1982,15 @@ int cs_batch_set_active(cs_batch* b, const uint8_t* active)
   HIP_TRY(hipSetDevice(b->device));
   std::vector<uint8_t> act(active, active + b->count);
   HIP_TRY(hipMemcpyAsync(b->d_active, act.data(), b->count, hipMemcpyHostToDevice, b->stream));
+  /* passes leave a retired realisation alone, and the buffer that holds the
+   * others' state alternates: its state goes into both */
+  for (uint32_t i = 0; i < b->count; i++)
+    if (b->h_active[i] && !act[i]) {
+      const BatchGeo& g = b->geo[i];
+      const size_t off = g.u_off * b->esize, bytes = g.nv * g.ns * b->esize;
+      HIP_TRY(hipMemcpyAsync((char*)b->d_u[b->cur ^ 1] + off, (const char*)b->d_u[b->cur] + off, bytes,
+                             hipMemcpyDeviceToDevice, b->stream));
+    }
   /* the stencil pass keeps only the active realisations' tiles */
   std::vector<BatchTile> all, keep;
   make_tiles(b, BX * b->launch.rows, b->launch.zchunk, all);
@@ -1570,7 +2000,9 @@ int cs_batch_set_active(cs_batch* b, const uint8_t* active)
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->ntiles = (uint32_t)keep.size();
   drop_graphs(b);
-  return CS_OK;
+  if (act == b->h_active) return CS_OK;
+  b->h_active.swap(act);
+  return upload_pass2_tiles(b);
 }
 
 int cs_batch_get_launch(const cs_batch* b, cs_batch_launch* out)
@@ -1595,8 +2027,7 @@ int cs_batch_set_launch(cs_batch* b, const cs_batch_launch* in)
   int rc = b->esize == 8 ? upload_tiles<double>(b) : upload_tiles<float>(b);
   if (rc != CS_OK) return rc;
   /* keep retired realisations out */
-  std::vector<uint8_t> act(b->count);
-  HIP_TRY(hipMemcpy(act.data(), b->d_active, b->count, hipMemcpyDeviceToHost));
+  const std::vector<uint8_t> act = b->h_active;
   return cs_batch_set_active(b, act.data());
 }
 
@@ -1631,13 +2062,15 @@ int cs_batch_time_steps(cs_batch* b, uint64_t first, uint64_t n, double* total_m
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
   HIP_TRY(hipEventRecord(ev[2 * n], b->stream));
   int rc;
+  uint64_t npasses = 0;
   if (b->use_graph) {
     /* the whole range as the caller runs it (graphs included); the
      * stencil's share is not separated (reported as 0): time a range with
      * graphs off for it */
     rc = b->esize == 8 ? b_step<double>(b, first, n, nullptr, 0) : b_step<float>(b, first, n, nullptr, 0);
   } else {
-    rc = b->esize == 8 ? b_run<double>(b, first, n, nullptr, ev.data()) : b_run<float>(b, first, n, nullptr, ev.data());
+    rc = b->esize == 8 ? b_run<double>(b, first, n, nullptr, ev.data(), nullptr, &npasses)
+                       : b_run<float>(b, first, n, nullptr, ev.data(), nullptr, &npasses);
   }
   if (rc != CS_OK) return rc;
   HIP_TRY(hipEventRecord(ev[2 * n + 1], b->stream));
@@ -1647,7 +2080,7 @@ int cs_batch_time_steps(cs_batch* b, uint64_t first, uint64_t n, double* total_m
   *total_ms = ms;
   double ksum = 0.0;
   if (!b->use_graph) {
-    for (uint64_t i = 0; i < n; i++) {
+    for (uint64_t i = 0; i < npasses; i++) {
       HIP_TRY(hipEventElapsedTime(&ms, ev[2 * i], ev[2 * i + 1]));
       ksum += ms;
     }
@@ -1665,6 +2098,12 @@ int cs_batch_set_gating(cs_batch* b, uint32_t mode, const cs_mlp* net)
   if (mode == CS_GATE_CLOSURE) {
     if (!net) return set_err(CS_EINVAL, "closure gating needs a network");
     if (b->model.rng == CS_RNG_MT && b->uni_stride) return set_err(CS_EINVAL, "closure gating draws Philox uniforms");
+    if (b->p2_ok && !b->near_ok) {
+      HIP_TRY(hipSetDevice(b->device));
+      HIP_TRY(hipStreamSynchronize(b->stream));
+      const int rc = index_kept_voxels(b, true);
+      if (rc != CS_OK) return rc;
+    }
     b->d_net = (const MlpDev*)cs_internal_mlp_device(net);
   }
   b->gating = mode;
@@ -1865,6 +2304,42 @@ int cs_batch_autotune(cs_batch* b, uint64_t first, uint32_t reps, cs_batch_launc
   }
   rc = cs_batch_set_launch(b, &wcfg);
   if (rc != CS_OK) return rc;
+  /* two-step passes over the pairs of two periods, each counting as two
+   * steps: they run unless the one-step shape found above beats them */
+  if (b->p2_ok && b->n_p2_tiles) {
+    HIP_TRY(hipEventCreate(&e0));
+    if (hipEventCreate(&e1) != hipSuccess) {
+      (void)hipEventDestroy(e0);
+      return set_err(CS_EDEVICE, "event creation failed");
+    }
+    std::map<std::array<uint32_t, 4>, std::pair<uint64_t, uint32_t>> pairs;
+    for (uint64_t k = 0; k < 2 * P; k += 2) {
+      const uint64_t ti = first + k;
+      const uint32_t m1 = b_diffusing(b, ti), m2 = b_diffusing(b, ti + 1);
+      auto& v = pairs[{m1, b_react(b, ti, m1), m2, b_react(b, ti + 1, m2)}];
+      v.first = ti;
+      v.second++;
+    }
+    double tot = 0.0;
+    for (const auto& kv : pairs) {
+      auto one = [&]() { return launch_bpass2(b, b->d_u[b->cur], b->d_u[b->cur ^ 1], kv.second.first); };
+      float ms = 0;
+      rc = one();
+      if (rc == CS_OK && hipEventRecord(e0, b->stream) != hipSuccess) rc = set_err(CS_EDEVICE, "event record failed");
+      for (uint32_t r = 0; rc == CS_OK && r < reps; r++) rc = one();
+      if (rc == CS_OK && (hipEventRecord(e1, b->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+                          hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+        rc = set_err(CS_EDEVICE, "timing a two-step pass failed");
+      if (rc != CS_OK) break;
+      tot += kv.second.second * (double)ms / reps;
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    if (rc != CS_OK) return rc;
+    const double per_step = tot / (2.0 * (double)P);
+    b->p2_on = per_step <= win;
+    if (b->p2_on) win = per_step;
+  }
   if (best) *best = wcfg;
   if (best_ms) *best_ms = win;
   return CS_OK;

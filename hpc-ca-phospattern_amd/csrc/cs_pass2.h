@@ -65,7 +65,8 @@ struct P2Args {
 constexpr int p2_threads(size_t esize, bool whole) { return (esize == 4 ? 512 : 256) << (whole ? 1 : 0); }
 constexpr int p2_chunk(size_t esize) { return (int)(16 / esize); }
 constexpr int p2_stage(size_t esize, bool whole) { return (esize == 4 ? 680 : 340) << (whole ? 1 : 0); }
-/* Whole blocks for field stacks beyond the last-level cache (256 MB). */
+/* Whole blocks for a domain whose field stacks are beyond the last-level
+ * cache (256 MB). */
 inline bool p2_whole(uint64_t stack_bytes) { return 2 * stack_bytes > (256ull << 20); }
 /* The field stacks end in this many bytes that a row's last chunk may read. */
 constexpr size_t P2_PAD = 64;

@@ -365,20 +365,25 @@ int cs_batch_flux_predictions(cs_batch* b, double* ratio);
  * left the training range since cs_batch_reset (the range monitor). */
 int cs_batch_monitor(cs_batch* b, uint32_t* flags);
 
-/* Launch shape of the ensemble's stencil pass: blocks of 64 x rows
+/* Launch shape of the ensemble's one-step pass: blocks of 64 x rows
  * threads, each tile 64*rows consecutive plane columns of one realisation
  * by zchunk planes; prefetch and nontemporal as in cs_launch_config.
  * persistent = 1 runs one persistent block per resident slot, taking tiles
  * from eight per-XCD work queues; 0 launches one block per tile, the tiles
  * numbered in groups per XCD, and leaves the scheduling to the hardware
- * (same results, bit for bit).  No reference counterpart. */
+ * (same results, bit for bit).  Ensembles of the five-slot species layout
+ * run their steps in pairs, as two-step passes of their own shape (see
+ * cs_launch_config); there one-step passes take only a last odd step.  No
+ * reference counterpart. */
 typedef struct cs_batch_launch {
   uint32_t rows, zchunk, prefetch, nontemporal, persistent;
 } cs_batch_launch;
 int cs_batch_get_launch(const cs_batch* b, cs_batch_launch* cfg);
 int cs_batch_set_launch(cs_batch* b, const cs_batch_launch* cfg);
 /* Time every candidate shape on one period of the step pattern from
- * first_time_ind (state unchanged) and keep the fastest. */
+ * first_time_ind (state unchanged) and keep the fastest; two-step passes
+ * stay off if the best one-step shape beats them.  best_ms is the mean
+ * kernel time per step of the form that runs. */
 int cs_batch_autotune(cs_batch* b, uint64_t first_time_ind, uint32_t reps, cs_batch_launch* best,
                       double* best_ms);
 /* on != 0: cs_batch_step replays whole periods of the step pattern (the
@@ -389,7 +394,8 @@ int cs_batch_set_graph(cs_batch* b, uint32_t on);
  * substep, doubled if odd): step counts that are multiples of it replay
  * graphs only. */
 int cs_batch_step_period(const cs_batch* b, uint64_t* period);
-/* Time nsteps steps: total ms, and the mean stencil pass (0 with graphs). */
+/* Time nsteps steps: total ms, and the stencil passes' mean per step (0
+ * with graphs). */
 int cs_batch_time_steps(cs_batch* b, uint64_t first_time_ind, uint64_t nsteps, double* total_ms,
                         double* stencil_ms);
 
