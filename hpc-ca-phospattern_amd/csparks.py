@@ -434,6 +434,12 @@ def gauss(x, sigma):
     return np.sqrt(0.5) * (2.0 / np.sqrt(np.pi)) * (1.0 / np.sqrt(sigma)) / 2 * np.exp(-np.asarray(x) * x / 2 / sigma)
 
 
+def _axis_gauss(k: int, h: float, sigma: float) -> np.ndarray:
+    """Gaussian weights of the linescan along its axis by distance in
+    voxels, from 1 - k to k - 1."""
+    return gauss(np.arange(1 - k, k) * h, sigma)
+
+
 @dataclass
 class Options:
     """Command-line options of the reference (options.c:502-542)."""
@@ -819,8 +825,7 @@ class Simulation:
         ptr = lambda a: a.ctypes.data_as(C.POINTER(C.c_double))
         _check(device_lib().cs_linescan(self.ctx, species, axis, ptr(w[0]), ptr(w[1]), ptr(w[2]), mask, ptr(proj)),
                "cs_linescan")
-        k = np.arange(n[axis]) * h
-        return np.array([float(np.dot(proj, gauss(p - k, conv[axis]))) for p in k])
+        return np.convolve(proj, _axis_gauss(n[axis], h, conv[axis]), "valid")
 
     def recruited(self, flux: int) -> np.ndarray:
         """Channels of discrete flux `flux` open at some gating step so far
@@ -928,13 +933,15 @@ class Ensemble:
         self.ns = int(self.setups[0].s.num_species)
         self.nd = int(self.setups[0].s.num_domains)
         self.mt = self.setups[0].problem.rng == RNG_MT
+        self._n = [s.n for s in self.setups]
+        self._h = float(self.setups[0].problem.h)
 
     @property
     def dt(self):
         return self.setups[0].dt
 
     def n(self, i: int):
-        return self.setups[i].n
+        return self._n[i]
 
     def step(self, nsteps: int = 1):
         lib = device_lib()
@@ -992,26 +999,32 @@ class Ensemble:
 
     def linescans(self, species: int, axis: int, offsets, conv, num_domains: int = 0):
         """Simulation.linescan of every member (one device pass for all)."""
-        w, ks = [], []
-        for i in range(self.count):
-            n = self.n(i)
-            h = self.setups[i].problem.h
-            off = [(n[ax] // 2 + int(offsets[ax])) * h for ax in range(3)]
-            w.extend(gauss(off[ax] - np.arange(n[ax]) * h, conv[ax]) for ax in range(3))
-            ks.append(n[axis])
-        weights = np.ascontiguousarray(np.concatenate(w))
+        # members share h, so weights depend on a length and an axis only
+        h, of = self._h, {}
+
+        def weight(k, ax):
+            if (k, ax) not in of:
+                of[k, ax] = gauss((k // 2 + int(offsets[ax])) * h - np.arange(k) * h, conv[ax])
+            return of[k, ax]
+
+        weights = np.concatenate([weight(n[ax], ax) for n in self._n for ax in range(3)])
+        ks = [n[axis] for n in self._n]
         proj = np.empty(sum(ks))
         mask = 0xFFFFFFFF if not num_domains else (0xFF if num_domains >= 8 else (1 << num_domains) - 1)
         ptr = lambda a: a.ctypes.data_as(C.POINTER(C.c_double))
         _check(device_lib().cs_batch_linescan(self.handle, species, axis, ptr(weights), mask, ptr(proj)),
                "cs_batch_linescan")
-        out, o = [], 0
+        # one product per axis length: row i of the matrix holds the weights
+        # of the distances i - j
+        start, group = np.cumsum([0] + ks), {}
         for i, k in enumerate(ks):
-            h = self.setups[i].problem.h
-            pos = np.arange(k) * h
-            g = gauss(pos[:, None] - pos[None, :], conv[axis])
-            out.append(g @ proj[o:o + k])
-            o += k
+            group.setdefault(k, []).append(i)
+        out = [None] * self.count
+        for k, members in group.items():
+            g = np.lib.stride_tricks.sliding_window_view(_axis_gauss(k, h, conv[axis]), k)[::-1]
+            lines = proj[start[members][:, None] + np.arange(k)] @ g.T
+            for i, line in zip(members, lines):
+                out[i] = line
         return out
 
     def _flux_size(self, i: int, flux: int) -> int:
