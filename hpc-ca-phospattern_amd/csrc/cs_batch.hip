@@ -609,7 +609,11 @@ k_batch_stats(const T* __restrict__ u, const uint8_t* __restrict__ ids, const De
 /* Linescan projections of every realisation (cs_linescan's sums): part[i]
  * holds, per plane z, the sums over y of u w_y (axis 0: one entry per x)
  * or over x of u w_x (axes 1, 2: one entry per y); one block per (plane,
- * realisation).  w[i] is the realisation's [n0 | n1 | n2] weights. */
+ * realisation).  w[i] is the realisation's [n0 | n1 | n2] weights.  Bound
+ * by the latency of its loads: for axis 0 the block's lanes cover as many
+ * rows at once as fit, several rows of a lane are in flight, and the value
+ * is loaded whatever its domain: 91 us for 512 dyads at 6 nm, where one row
+ * at a time, waiting for each id, took 252. */
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_batch_scan_planes(const T* __restrict__ u, const uint8_t* __restrict__ ids, const DevParams<T>* __restrict__ P,
@@ -627,14 +631,31 @@ k_batch_scan_planes(const T* __restrict__ u, const uint8_t* __restrict__ ids, co
   double* pz = part + poff[i] + (uint64_t)z * (axis == 0 ? gg.nx : gg.ny);
   if (axis == 0) {
     const double* wy = wi + gg.nx;
-    for (int x = threadIdx.x; x < gg.nx; x += blockDim.x) {
+    __shared__ double rest[MAXD], sums[256];
+    if (threadIdx.x < MAXD) rest[threadIdx.x] = P->init64[threadIdx.x][s];
+    __syncthreads();
+    /* lane (x, q) of `rows` rows at once sums every rows-th row */
+    const int cols = min(gg.nx, (int)blockDim.x), rows = (int)blockDim.x / cols;
+    const int xl = (int)threadIdx.x % cols, q = (int)threadIdx.x / cols;
+    for (int x0 = 0; x0 < gg.nx; x0 += cols) {
+      const int x = x0 + xl;
       double acc = 0.0;
-      for (int y = 0; y < gg.ny; y++) {
-        const uint64_t c = (uint64_t)y * gg.nx + x;
-        const int d = iz[c] & 7;
-        if ((dmask >> d) & 1u) acc += ((double)us[c] + P->init64[d][s]) * wy[y];
+      if (q < rows && x < gg.nx) {
+#pragma unroll 8
+        for (int y = q; y < gg.ny; y += rows) {
+          const uint64_t c = (uint64_t)y * gg.nx + x;
+          const int d = iz[c] & 7;
+          const double v = ((double)us[c] + rest[d]) * wy[y];
+          acc = ((dmask >> d) & 1u) ? acc + v : acc;
+        }
       }
-      pz[x] = acc;
+      sums[threadIdx.x] = acc;
+      __syncthreads();
+      if (q == 0 && x < gg.nx) {
+        for (int k = 1; k < rows; k++) acc += sums[k * cols + xl];
+        pz[x] = acc;
+      }
+      __syncthreads();
     }
   } else {
     const double* wx = wi;
