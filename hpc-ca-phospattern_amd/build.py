@@ -49,7 +49,8 @@ def _hipcc():
     return path
 
 
-DEVICE_SOURCES = ("csparks.hip", "cs_batch.hip", "cs_closure.hip", "cs_pass2_f32.hip", "cs_pass2_f64.hip")
+DEVICE_SOURCES = ("csparks.hip", "cs_batch.hip", "cs_closure.hip", "cs_pass2_f32.hip", "cs_pass2_f64.hip",
+                  "cs_bridge.hip")
 
 
 def build_device():

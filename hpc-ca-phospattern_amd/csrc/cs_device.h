@@ -526,12 +526,11 @@ __device__ inline uint8_t gate_one(const FluxParams& F, uint8_t st, double c0, u
   if (!F.stochastic) {
     if (p[8] <= t + dts) st = 0;
   } else {
-    const double kc = cs_rate_close(c0, p);
-    const double ko = cs_rate_open(c0, p);
+    const double k = cs_rate(st != 0, c0, p);
     /* the caller's uniform for this channel, or the Philox stream */
     const double r = draw ? *draw : cs_gate_uniform(seed, instance, ti, F.group, ch);
-    if (st == 0) { if (r <= dts * ko) st = 1; }
-    else if (st == 1) { if (r <= dts * kc) st = 0; }
+    if (st == 0) { if (r <= dts * k) st = 1; }
+    else if (st == 1) { if (r <= dts * k) st = 0; }
   }
   return st;
 }
@@ -562,7 +561,7 @@ struct BChan {          /* a channel of a discrete flux, in gating order */
   double rest_to;       /* resting species 0 there                        */
   uint32_t slot_to;     /* level-1 slot of that voxel                     */
   uint32_t flux, ch;    /* flux index, channel index within the flux      */
-  uint32_t pad;
+  uint32_t state;       /* its state slot                                 */
 };
 struct BRow {           /* a k_flux row                                   */
   uint64_t elem;        /* the value the row adds to                      */

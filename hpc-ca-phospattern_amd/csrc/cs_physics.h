@@ -62,14 +62,15 @@ CS_HD double cs_serca_flux_d(double dt, double h, double u0, double u1, double d
 }
 
 /* Clamped power-law rates of evaluate_RyR_stochastically
- * (boundaryfluxes.c:339-342). p uses the reference parameter order. */
-CS_HD double cs_rate_close(double c, const double* p)
+ * (boundaryfluxes.c:339-342): the closing rate of an open channel, the
+ * opening rate of a closed one.  p uses the reference parameter order.  A
+ * gating step needs one of the two, so the parameters are chosen first and
+ * the power is taken once. */
+CS_HD double cs_rate(bool open, double c, const double* p)
 {
-  return fmax(fmin(pow(c / p[0], p[5]), p[1]), p[7]);
-}
-CS_HD double cs_rate_open(double c, const double* p)
-{
-  return fmax(fmin(pow(c / p[9], p[2]), p[3]), p[4]);
+  const double K = open ? p[0] : p[9], n = open ? p[5] : p[2];
+  const double most = open ? p[1] : p[3], least = open ? p[7] : p[4];
+  return fmax(fmin(pow(c / K, n), most), least);
 }
 
 /* Philox4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers:

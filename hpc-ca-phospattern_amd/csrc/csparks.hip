@@ -51,6 +51,7 @@
 #include "csparks.h"
 #include "cs_physics.h"
 
+#include "cs_bridge.h"
 #include "cs_device.h"
 #include "cs_pass2.h"
 
@@ -623,12 +624,6 @@ k_flux(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__ 
 struct F2Voxels {
   const uint32_t* col_start;   /* [plane + 1] first pair voxel of each column */
   const uint32_t* z;           /* plane of pair voxel k                        */
-};
-
-/* What one of the two steps of a fused pass does. */
-struct F2Step {
-  uint32_t dmask, react, fluxmask, gate;
-  uint64_t ti, uni_base;
 };
 
 /* Two time steps in one pass over HBM.  A block owns a 64 x WY tile of
@@ -1454,6 +1449,13 @@ struct cs_context {
   void* d_brow = nullptr;
   void* d_bent = nullptr;
   uint32_t nbchan = 0;
+  /* k_bridge_groups' records (none when a component is too large) */
+  uint32_t nbgroups = 0;
+  BgGroup* d_bg_group = nullptr;
+  BgVox* d_bg_vox = nullptr;
+  BgChan* d_bg_chan = nullptr;
+  BgRow* d_bg_row = nullptr;
+  BgEnt* d_bg_ent = nullptr;
   bool f2_ok = false;                /* the problem admits fused passes       */
   std::string f2_why;                /* why not, when it does not             */
   uint32_t fsm = 0;                  /* species the fluxes act on (bit 0)     */
@@ -1531,7 +1533,8 @@ void free_ctx(cs_context* c)
                   c->d_row_voxel, c->d_row_species, c->d_row_start, c->d_ent_pair,
                   c->d_ent_flux, c->d_ent_sign, c->d_uniforms, c->d_partial, c->d_stats,
                   c->d_lweights, c->d_lpart, c->d_xyz, c->d_f2_col, c->d_f2_z,
-                  c->d_f2_l1, c->d_f2_fsum, c->d_bchan, c->d_brow, c->d_bent, c->d_p2_geo};
+                  c->d_f2_l1, c->d_f2_fsum, c->d_bchan, c->d_brow, c->d_bent, c->d_p2_geo,
+                  c->d_bg_group, c->d_bg_vox, c->d_bg_chan, c->d_bg_row, c->d_bg_ent};
   for (auto& kv : c->p2_lists)
     if (kv.second.d) hipFree(kv.second.d);
   for (void* p : ptrs)
@@ -1877,12 +1880,38 @@ int launch_step2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout,
   return CS_OK;
 }
 
-/* k_bridge on the state u: the tail of a pass (step `tail`) and/or the
- * head of the next (step `head`). */
+/* The bridge on the state u: the tail of a pass (step `tail`) and/or the
+ * head of the next (step `head`); k_bridge_groups where every component of
+ * pairs fits a block, else k_bridge. */
 template <typename T>
 void launch_bridge(cs_context* c, void* u, const F2Step& tail, bool do_tail, const F2Step& head, bool do_head,
                    const double* d_uni)
 {
+  if (c->nbgroups) {
+    BgArgs a{};
+    a.u = u;
+    a.l1 = c->d_f2_l1;
+    a.fsum = c->d_f2_fsum;
+    a.params = c->d_params;
+    a.groups = c->d_bg_group;
+    a.vox = c->d_bg_vox;
+    a.chan = c->d_bg_chan;
+    a.row = c->d_bg_row;
+    a.ent = c->d_bg_ent;
+    a.states = c->d_states;
+    a.recruited = c->d_recruited;
+    a.uniforms = d_uni;
+    a.tail = tail;
+    a.head = head;
+    a.ngroups = c->nbgroups;
+    a.do_tail = do_tail ? 1u : 0u;
+    a.do_head = do_head ? 1u : 0u;
+    a.D = (uint32_t)c->prob.stochastic_substep;
+    a.seed = (uint32_t)c->prob.seed;
+    a.instance = (uint32_t)c->prob.instance;
+    return cs_internal_bridge_groups(c->esize, a, c->stream);
+  }
+  if (c->nrows == 0 && c->nbchan == 0) return;
   auto go = [&](uint32_t blocks, uint32_t phases) {
     hipLaunchKernelGGL(k_bridge<T>, dim3(blocks), dim3(BRIDGE_THREADS), 0, c->stream, (T*)u,
                        (const DevParams<T>*)c->d_params, (const BChan*)c->d_bchan, c->nbchan,
@@ -2208,7 +2237,7 @@ int build_flux_rows(cs_context* c, const cs_problem* p)
     if (!p->fluxes[f].discrete) continue;
     for (uint32_t ch = 0; ch < p->fluxes[f].num_pairs; ch++) {
       const uint32_t gp = pair_off[f] + ch, to = pairs_dev[2 * gp + 1];
-      bchan.push_back(BChan{elem(g, 0, to), p->init[dom(to)][0], pslot[2 * gp + 1], f, ch, 0});
+      bchan.push_back(BChan{elem(g, 0, to), p->init[dom(to)][0], pslot[2 * gp + 1], f, ch, c->state_off[f] + ch});
     }
   }
   std::vector<BRow> brow(row_voxel.size());
@@ -2238,6 +2267,16 @@ int build_flux_rows(cs_context* c, const cs_problem* p)
   if ((rc = upb(&c->d_bchan, bchan.data(), sizeof(BChan) * bchan.size())) != CS_OK) return rc;
   if ((rc = upb(&c->d_brow, brow.data(), sizeof(BRow) * brow.size())) != CS_OK) return rc;
   if ((rc = upb(&c->d_bent, bent.data(), sizeof(BEnt) * bent.size())) != CS_OK) return rc;
+  BgTables bg;
+  if (c->f2_ok && bg_build(keys.size(), bchan, brow, bent, bg)) {
+    c->nbgroups = (uint32_t)bg.groups.size();
+    if ((rc = upb((void**)&c->d_bg_group, bg.groups.data(), sizeof(BgGroup) * bg.groups.size())) != CS_OK ||
+        (rc = upb((void**)&c->d_bg_vox, bg.vox.data(), sizeof(BgVox) * bg.vox.size())) != CS_OK ||
+        (rc = upb((void**)&c->d_bg_chan, bg.chan.data(), sizeof(BgChan) * bg.chan.size())) != CS_OK ||
+        (rc = upb((void**)&c->d_bg_row, bg.row.data(), sizeof(BgRow) * bg.row.size())) != CS_OK ||
+        (rc = upb((void**)&c->d_bg_ent, bg.ent.data(), sizeof(BgEnt) * bg.ent.size())) != CS_OK)
+      return rc;
+  }
   HIP_TRY(hipMalloc(&c->d_f2_l1, c->esize * std::max<size_t>(keys.size(), 1)));
   HIP_TRY(hipMalloc((void**)&c->d_f2_fsum, sizeof(double) * std::max<size_t>(keys.size(), 1)));
   HIP_TRY(hipMemsetAsync(c->d_f2_fsum, 0, sizeof(double) * std::max<size_t>(keys.size(), 1), c->stream));
