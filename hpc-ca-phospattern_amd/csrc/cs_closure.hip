@@ -104,135 +104,172 @@ k_mlp_forward(const MlpDev* __restrict__ P, const uint16_t* __restrict__ xb, uin
 }
 
 /* Forward and backward passes over n samples (rows idx[k] of xb when idx
- * is given, else rows k), one wavefront per block, writing each
- * wavefront's gradient of L = sum (y - t)^2 / norm into
- * part[wave][MLP_NPARAM] and its sum of squared errors into sse[wave].
- * The weight operands sit in LDS; the weight gradients are products over
- * the 32 samples of a round, formed on the matrix cores from activations
- * and back-propagated gradients transposed through LDS. */
-__global__ void __launch_bounds__(64)
+ * is given, else rows k), 32 samples to a block, writing each block's
+ * gradient of L = sum (y - t)^2 / norm into part[block][MLP_NPARAM] and its
+ * sum of squared errors into sse[block].
+ *
+ * Two wavefronts share the samples: wavefront m owns features 32 m .. 32 m
+ * + 31 of either layer, as mlp_forward's block m, and hands the other its
+ * bfloat16 layer outputs and back-propagated gradients through LDS; the
+ * output sum runs through block 0 and then block 1, so every sum keeps
+ * mlp_forward's order.  The weight gradients are products over the 32
+ * samples, formed on the matrix cores from activations and gradients
+ * transposed through LDS.
+ *
+ * A training batch of 2048 is 64 blocks of one round, so the length of one
+ * wavefront's chain of GELU arithmetic and loads is the time: half of it
+ * each, the weight operands and tables loaded once into registers at the
+ * start instead of through LDS, and each layer's pre-activations kept, so
+ * GELU and its derivative share the error function.  A batch of 2048 takes
+ * 8.2 us, where one wavefront per 32 samples took 19.0; 200001 samples 75
+ * and 99 us. */
+__global__ void __launch_bounds__(128)
 k_mlp_grad(const MlpDev* __restrict__ P, const uint16_t* __restrict__ xb, const float* __restrict__ tv,
            const uint32_t* __restrict__ idx, uint64_t n, float norm, float* __restrict__ part,
            double* __restrict__ sse)
 {
-  __shared__ alignas(16) uint16_t Lop[NSEG][64][8];
   /* x, h1, h2, g_z2, g_z1 as [feature][sample] bfloat16; g_y per sample */
   __shared__ alignas(16) uint16_t Lx[MLP_PAD][LROW];
   __shared__ alignas(16) uint16_t Lh1[MLP_H][LROW];
   __shared__ alignas(16) uint16_t Lh2[MLP_H][LROW];
   __shared__ alignas(16) uint16_t Lz2[MLP_H][LROW];
   __shared__ alignas(16) uint16_t Lz1[MLP_H][LROW];
-  __shared__ float Lgy[32];
-  const int lane = threadIdx.x & 63, g = lane >> 5, l = lane & 31;
-  {
-    const uint4* src = reinterpret_cast<const uint4*>(&P->opnd[0][0][0]);
-    uint4* dst = reinterpret_cast<uint4*>(&Lop[0][0][0]);
-    for (int k = lane; k < NSEG * 64; k += 64) dst[k] = src[k];
-  }
-  auto lop = [&](int seg) { return *reinterpret_cast<const bf16x8*>(&Lop[seg][lane][0]); };
-  const uint64_t waves = gridDim.x;
-  const uint64_t wid = blockIdx.x;
-  const uint64_t tiles = (n + 31) / 32;
+  __shared__ bf16x8 Lop[2][2][64];   /* operands in register order: [block][chunk][lane] */
+  __shared__ float Lgy[32], Ly[32], Lpart[64];
+  const int lane = threadIdx.x & 63, m = threadIdx.x >> 6, g = lane >> 5, l = lane & 31;
+  const uint64_t blocks = gridDim.x, wid = blockIdx.x, tiles = (n + 31) / 32;
 
-  f32x16 gw1[2], gw2[2][2];
+  bf16x8 w1[2], w2f[2][2], w2b[2][2];
 #pragma unroll
-  for (int a = 0; a < 2; a++) {
-    gw1[a] = f32x16{};
-    gw2[a][0] = f32x16{};
-    gw2[a][1] = f32x16{};
-  }
+  for (int c = 0; c < 2; c++) w1[c] = mlp_opnd(P, SEG_L1 + 2 * m + c, lane);
+#pragma unroll
+  for (int o = 0; o < 2; o++)
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      w2f[o][q] = mlp_opnd(P, SEG_L2F + 4 * m + 2 * o + q, lane);
+      w2b[o][q] = mlp_opnd(P, SEG_L2B + 4 * m + 2 * o + q, lane);
+    }
+  float b1[16], b2[16], w3[16];
+  feat_vec(P->b1, m, g, b1);
+  feat_vec(P->b2, m, g, b2);
+  feat_vec(P->w3, m, g, w3);
+  const float b3 = P->b3;
+
+  f32x16 gw1 = f32x16{}, gw2[2] = {f32x16{}, f32x16{}};
   float gb1 = 0.0f, gb2 = 0.0f, gw3 = 0.0f, gb3 = 0.0f;
   double err2 = 0.0;
-  __syncthreads();
 
-  for (uint64_t t = wid; t < tiles; t += waves) {
-    /* reload the weights every round instead of holding them all in
-     * registers across the loop */
-    asm volatile("" ::: "memory");
+  for (uint64_t t = wid; t < tiles; t += blocks) {
     const uint64_t k = t * 32 + l;
     const bool valid = k < n;
     const uint64_t s = valid ? (idx ? (uint64_t)idx[k] : k) : 0;
     bf16x8 x[2];
     load_x(xb, s, valid, x);
-    f32x16 z1[2], z2[2];
-    bf16x8 h1b[2][2];
-    const float y = mlp_forward(P, lop, x, z1, z2, h1b, [&](int m, int r, float h2) {
-      Lh2[32 * m + mlp_feat(g, r)][l] = __builtin_bit_cast(uint16_t, to_bf16(h2));
-    });
-    const float gy = valid ? 2.0f * (y - tv[s]) / norm : 0.0f;
-    if (g == 0) {
+    const float target = tv[s];
+    /* layer 1 */
+    f32x16 z1;
+#pragma unroll
+    for (int r = 0; r < 16; r++) z1[r] = b1[r];
+#pragma unroll
+    for (int c = 0; c < 2; c++) z1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1[c], x[c], z1, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      bf16x8 h;
+#pragma unroll
+      for (int j = 0; j < 8; j++) h[j] = to_bf16(mlp_gelu(z1[8 * q + j]));
+      Lop[m][q][lane] = h;
+#pragma unroll
+      for (int j = 0; j < 8; j++) Lh1[32 * m + mlp_feat(g, 8 * q + j)][l] = bf16_bits(h, j);
+    }
+    /* x for the weight gradients, a chunk to each wavefront */
+#pragma unroll
+    for (int j = 0; j < 8; j++) Lx[16 * m + 8 * g + j][l] = bf16_bits(m ? x[1] : x[0], j);
+    __syncthreads();
+    /* layer 2 and the output */
+    f32x16 z2;
+#pragma unroll
+    for (int r = 0; r < 16; r++) z2[r] = b2[r];
+#pragma unroll
+    for (int mb = 0; mb < 2; mb++)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        z2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w2f[mb][q], Lop[mb][q][lane], z2, 0, 0, 0);
+    float h2[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const __bf16 h = to_bf16(mlp_gelu(z2[r]));
+      Lh2[32 * m + mlp_feat(g, r)][l] = __builtin_bit_cast(uint16_t, h);
+      h2[r] = (float)h;
+    }
+    if (m == 0) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; r++) sum += w3[r] * h2[r];
+      Lpart[lane] = sum;
+    }
+    __syncthreads();
+    if (m == 1) {
+      float sum = Lpart[lane];
+#pragma unroll
+      for (int r = 0; r < 16; r++) sum += w3[r] * h2[r];
+      const float y = sum + __shfl_xor(sum, 32, 64) + b3;
+      if (g == 0) Ly[l] = y;
+    }
+    __syncthreads();
+    const float y = Ly[l];
+    const float gy = valid ? 2.0f * (y - target) / norm : 0.0f;
+    if (m == 0 && g == 0) {
       Lgy[l] = gy;
       gb3 += gy;
-      if (valid) err2 += (double)(y - tv[s]) * (double)(y - tv[s]);
+      if (valid) err2 += (double)(y - target) * (double)(y - target);
     }
     /* g_z2 = w3 g_y gelu'(z2), bfloat16 */
-    bf16x8 gz2b[2][2];
 #pragma unroll
-    for (int m = 0; m < 2; m++) {
-      float w[16];
-      feat_vec(P->w3, m, g, w);
+    for (int q = 0; q < 2; q++) {
+      bf16x8 h;
 #pragma unroll
-      for (int r = 0; r < 16; r++) gz2b[m][r / 8][r % 8] = to_bf16(w[r] * gy * mlp_gelu_grad(z2[m][r]));
+      for (int j = 0; j < 8; j++) h[j] = to_bf16(w3[8 * q + j] * gy * mlp_gelu_grad(z2[8 * q + j]));
+      Lop[m][q][lane] = h;
+#pragma unroll
+      for (int j = 0; j < 8; j++) Lz2[32 * m + mlp_feat(g, 8 * q + j)][l] = bf16_bits(h, j);
     }
-    /* transposes for the weight gradients */
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-      for (int j = 0; j < 8; j++) Lx[16 * c + 8 * g + j][l] = bf16_bits(x[c], j);
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int f = 32 * m + mlp_feat(g, r);
-        Lh1[f][l] = bf16_bits(h1b[m][r / 8], r % 8);
-        Lz2[f][l] = bf16_bits(gz2b[m][r / 8], r % 8);
-      }
+    __syncthreads();
     /* g_h1 = W2 g_z2 on the matrix cores, then g_z1 = g_h1 gelu'(z1) */
+    f32x16 gh1 = f32x16{};
 #pragma unroll
-    for (int mi = 0; mi < 2; mi++) {
-      f32x16 gh1 = f32x16{};
+    for (int mo = 0; mo < 2; mo++)
 #pragma unroll
-      for (int mo = 0; mo < 2; mo++)
+      for (int q = 0; q < 2; q++)
+        gh1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w2b[mo][q], Lop[mo][q][lane], gh1, 0, 0, 0);
 #pragma unroll
-        for (int q = 0; q < 2; q++)
-          gh1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lop(SEG_L2B + 4 * mi + 2 * mo + q), gz2b[mo][q], gh1, 0, 0, 0);
-      /* z1 of this block again (two products), rather than holding it
-       * in registers through the layer-2 backward pass */
-      f32x16 z = f32x16{};
-      {
-        float b[16];
-        feat_vec(P->b1, mi, g, b);
-#pragma unroll
-        for (int r = 0; r < 16; r++) z[r] = b[r];
-      }
-#pragma unroll
-      for (int c = 0; c < 2; c++)
-        z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lop(SEG_L1 + 2 * mi + c), x[c], z, 0, 0, 0);
-#pragma unroll
-      for (int r = 0; r < 16; r++)
-        Lz1[32 * mi + mlp_feat(g, r)][l] = __builtin_bit_cast(uint16_t, to_bf16(gh1[r] * mlp_gelu_grad(z[r])));
-    }
+    for (int r = 0; r < 16; r++)
+      Lz1[32 * m + mlp_feat(g, r)][l] = __builtin_bit_cast(uint16_t, to_bf16(gh1[r] * mlp_gelu_grad(z1[r])));
     __syncthreads();
     /* dW^T[o][i] += sum over the round's samples of g_z[o][s] a[i][s] */
     auto row = [&](const uint16_t (*L)[LROW], int r, int c) {
       return *reinterpret_cast<const bf16x8*>(&L[r][16 * c + 8 * g]);
     };
 #pragma unroll
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < 2; c++) {
+      const bf16x8 az2 = row(Lz2, 32 * m + l, c);
 #pragma unroll
-      for (int mo = 0; mo < 2; mo++) {
-        const bf16x8 az2 = row(Lz2, 32 * mo + l, c);
-#pragma unroll
-        for (int mi = 0; mi < 2; mi++)
-          gw2[mo][mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(az2, row(Lh1, 32 * mi + l, c), gw2[mo][mi], 0, 0, 0);
-        gw1[mo] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row(Lz1, 32 * mo + l, c), row(Lx, l, c), gw1[mo], 0, 0, 0);
-      }
-    /* lane f: bias gradients and the output weight's gradient of feature f */
+      for (int mi = 0; mi < 2; mi++)
+        gw2[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(az2, row(Lh1, 32 * mi + l, c), gw2[mi], 0, 0, 0);
+      gw1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row(Lz1, 32 * m + l, c), row(Lx, l, c), gw1, 0, 0, 0);
+    }
+    /* lane f: bias gradients (wavefront 0) and the output weight's gradient
+     * (wavefront 1) of feature f */
+    auto at = [](const uint16_t (*L)[LROW], int f, int j) { return (float)__builtin_bit_cast(__bf16, L[f][j]); };
     float s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-    for (int j = 0; j < 32; j++) {
-      s1 += (float)__builtin_bit_cast(__bf16, Lz1[lane][j]);
-      s2 += (float)__builtin_bit_cast(__bf16, Lz2[lane][j]);
-      s3 += (float)__builtin_bit_cast(__bf16, Lh2[lane][j]) * Lgy[j];
+    if (m == 0) {
+#pragma unroll 8
+      for (int j = 0; j < 32; j++) {
+        s1 += at(Lz1, lane, j);
+        s2 += at(Lz2, lane, j);
+      }
+    } else {
+#pragma unroll 8
+      for (int j = 0; j < 32; j++) s3 += at(Lh2, lane, j) * Lgy[j];
     }
     gb1 += s1;
     gb2 += s2;
@@ -240,20 +277,21 @@ k_mlp_grad(const MlpDev* __restrict__ P, const uint16_t* __restrict__ xb, const 
     __syncthreads();   /* reads done before the next round writes */
   }
 
-  /* this wavefront's gradient, in the packed parameter order */
+  /* this block's gradient, in the packed parameter order */
   float* o = part + wid * (uint64_t)MLP_NPARAM;
 #pragma unroll
-  for (int mo = 0; mo < 2; mo++)
+  for (int r = 0; r < 16; r++) {
+    const int of = 32 * m + mlp_feat(g, r);
+    o[MLP_OFF_W1 + l * MLP_H + of] = gw1[r];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int of = 32 * mo + mlp_feat(g, r);
-      o[MLP_OFF_W1 + l * MLP_H + of] = gw1[mo][r];
-#pragma unroll
-      for (int mi = 0; mi < 2; mi++) o[MLP_OFF_W2 + (32 * mi + l) * MLP_H + of] = gw2[mo][mi][r];
-    }
+    for (int mi = 0; mi < 2; mi++) o[MLP_OFF_W2 + (32 * mi + l) * MLP_H + of] = gw2[mi][r];
+  }
+  if (m == 1) {
+    o[MLP_OFF_W3 + lane] = gw3;
+    return;
+  }
   o[MLP_OFF_B1 + lane] = gb1;
   o[MLP_OFF_B2 + lane] = gb2;
-  o[MLP_OFF_W3 + lane] = gw3;
   for (int off = 16; off > 0; off >>= 1) {
     gb3 += __shfl_xor(gb3, off, 64);
     err2 += __shfl_xor(err2, off, 64);
@@ -299,17 +337,17 @@ struct AdamStep {
   uint32_t on;
 };
 
-/* grad[k] = sum over the wavefront partials, then (adam.on) the Adam
+/* grad[k] = sum over the blocks' partials, then (adam.on) the Adam
  * step on the FP32 master parameters and the parameter's places in the
  * device image, so a training step is two launches.  A block owns 64
  * parameters and splits their partials over its 16 wavefronts (one row of
  * 256 bytes per load), each summing its rows in order in FP64, the 16 sums
  * in wavefront order: a fixed order, so training is reproducible.  Bound by
- * the latency of a wavefront's loads (nwaves / 16 rows): one thread per
+ * the latency of a wavefront's loads (nparts / 16 rows): one thread per
  * parameter walking all 768 partials took 222 us, and a batch of 2048 made
  * only 64 of them. */
 __global__ void __launch_bounds__(64 * UPD_GROUPS)
-k_mlp_update(const float* __restrict__ part, uint32_t nwaves, float* __restrict__ grad, const double* __restrict__ sse,
+k_mlp_update(const float* __restrict__ part, uint32_t nparts, float* __restrict__ grad, const double* __restrict__ sse,
              double* __restrict__ sse_out, float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
              AdamStep adam, MlpDev* __restrict__ P)
 {
@@ -319,7 +357,7 @@ k_mlp_update(const float* __restrict__ part, uint32_t nwaves, float* __restrict_
   double acc = 0.0;
   if (k < MLP_NPARAM) {
 #pragma unroll 4
-    for (uint32_t w = g; w < nwaves; w += UPD_GROUPS) acc += part[(uint64_t)w * MLP_NPARAM + k];
+    for (uint32_t w = g; w < nparts; w += UPD_GROUPS) acc += part[(uint64_t)w * MLP_NPARAM + k];
   }
   sh[g][lane] = acc;
   __syncthreads();
@@ -340,7 +378,7 @@ k_mlp_update(const float* __restrict__ part, uint32_t nwaves, float* __restrict_
   }
   if (blockIdx.x == 0 && g == 1) {
     double e = 0.0;
-    for (uint32_t w = lane; w < nwaves; w += 64) e += sse[w];
+    for (uint32_t w = lane; w < nparts; w += 64) e += sse[w];
     for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
     if (lane == 0) *sse_out = e;
   }
@@ -359,7 +397,7 @@ struct cs_mlp {
   float* d_part = nullptr;
   double* d_sse = nullptr;
   double* d_sse_out = nullptr;
-  uint32_t grad_waves = 0;    /* wavefronts of a gradient launch */
+  uint32_t grad_blocks = 0;   /* blocks of a gradient launch */
   uint64_t adam_step = 0;
   /* training set */
   uint16_t* d_x = nullptr;
@@ -426,15 +464,15 @@ int to_bf16_rows(cs_mlp* m, const float* d_x, uint64_t n, uint16_t* d_xb)
 
 /* Gradient of sum (y - t)^2 / norm over n samples into d_grad, the sum of
  * squared errors into d_sse_out and, with adam.on, the Adam step.  No more
- * wavefronts than there are rounds of 32 samples: an idle one still writes
+ * blocks than there are rounds of 32 samples: an idle one still writes
  * a partial of zeros that the update then reads (25 KB each). */
 int run_grad(cs_mlp* m, const uint16_t* d_xb, const float* d_t, const uint32_t* d_idx, uint64_t n, float norm,
              const AdamStep& adam)
 {
-  const uint32_t waves = (uint32_t)std::min<uint64_t>(m->grad_waves, (n + 31) / 32);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(waves), dim3(64), 0, m->stream, m->d_dev, d_xb, d_t, d_idx, n, norm, m->d_part,
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>(m->grad_blocks, (n + 31) / 32);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(blocks), dim3(128), 0, m->stream, m->d_dev, d_xb, d_t, d_idx, n, norm, m->d_part,
                      m->d_sse);
-  hipLaunchKernelGGL(k_mlp_update, dim3((MLP_NPARAM + 63) / 64), dim3(64 * UPD_GROUPS), 0, m->stream, m->d_part, waves,
+  hipLaunchKernelGGL(k_mlp_update, dim3((MLP_NPARAM + 63) / 64), dim3(64 * UPD_GROUPS), 0, m->stream, m->d_part, blocks,
                      m->d_grad, m->d_sse, m->d_sse_out, m->d_p, m->d_m, m->d_v, adam, m->d_dev);
   HIP_TRY(hipGetLastError());
   return CS_OK;
@@ -455,13 +493,13 @@ int cs_mlp_create(const float* params, cs_mlp** out)
     return bail(set_err(CS_EDEVICE, "hipStreamCreate failed"));
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, m->device) != hipSuccess) return bail(set_err(CS_EDEVICE, "device query failed"));
-  m->grad_waves = (uint32_t)std::max(1, prop.multiProcessorCount) * 3;   /* three blocks per CU */
+  m->grad_blocks = (uint32_t)std::max(1, prop.multiProcessorCount) * 3;   /* three blocks per CU */
   if (hipMalloc(&m->d_dev, sizeof(MlpDev)) != hipSuccess || hipMalloc(&m->d_p, sizeof(float) * MLP_NPARAM) != hipSuccess ||
       hipMalloc(&m->d_m, sizeof(float) * MLP_NPARAM) != hipSuccess ||
       hipMalloc(&m->d_v, sizeof(float) * MLP_NPARAM) != hipSuccess ||
       hipMalloc(&m->d_grad, sizeof(float) * MLP_NPARAM) != hipSuccess ||
-      hipMalloc(&m->d_part, sizeof(float) * MLP_NPARAM * (size_t)m->grad_waves) != hipSuccess ||
-      hipMalloc(&m->d_sse, sizeof(double) * m->grad_waves) != hipSuccess ||
+      hipMalloc(&m->d_part, sizeof(float) * MLP_NPARAM * (size_t)m->grad_blocks) != hipSuccess ||
+      hipMalloc(&m->d_sse, sizeof(double) * m->grad_blocks) != hipSuccess ||
       hipMalloc(&m->d_sse_out, sizeof(double)) != hipSuccess)
     return bail(set_err(CS_ENOMEM, "device allocation of the network failed"));
   /* identity normalisation until cs_mlp_set_normalisation */
