@@ -784,6 +784,7 @@ struct cs_batch {
   bool p2_ok = false, p2_on = false, near_ok = false;
   std::vector<P2Split> p2_split;
   P2Geo* d_p2_geo = nullptr;
+  uint32_t* d_p2_words = nullptr;
   P2Tile* d_p2_tiles = nullptr;
   uint32_t n_p2_tiles = 0, cap_p2_tiles = 0;
   int p2_xcd = 0, cus = 1;
@@ -825,7 +826,7 @@ void free_batch(cs_batch* b)
                   b->d_chan, b->d_rows, b->d_ents, b->d_states, b->d_recruited, b->d_active, b->d_last_open,
                   b->d_cgeo, b->d_nb_start, b->d_nb, b->d_cpred, b->d_fpred, b->d_chca, b->d_feat, b->d_flags,
                   b->d_uniforms, b->d_stats, b->d_lw, b->d_lpart, b->d_lproj, b->d_loff, b->d_ti,
-                  b->d_p2_geo, b->d_p2_tiles, b->d_p2_col, b->d_p2_z, b->d_p2_fsum, b->d_p2_l1, b->d_near};
+                  b->d_p2_geo, b->d_p2_words, b->d_p2_tiles, b->d_p2_col, b->d_p2_z, b->d_p2_fsum, b->d_p2_l1, b->d_near};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -1040,6 +1041,7 @@ int index_kept_voxels(cs_batch* b, bool near)
     if (*p) HIP_TRY(hipFree(*p));
     *p = nullptr;
   }
+  if (!b->d_p2_words) HIP_TRY(hipMalloc(&b->d_p2_words, sizeof(uint32_t) * std::max<uint64_t>(b->total_ids, 1)));
   const size_t n = std::max<size_t>(vz.size(), 1);
   HIP_TRY(hipMalloc(&b->d_p2_col, sizeof(uint32_t) * col_start.size()));
   HIP_TRY(hipMalloc(&b->d_p2_z, sizeof(uint32_t) * n));
@@ -1061,6 +1063,10 @@ int index_kept_voxels(cs_batch* b, bool near)
       (rc = up(b->d_rows, b->h_rows.data(), sizeof(BRow) * b->h_rows.size())) != CS_OK ||
       (rc = up(b->d_ents, b->h_ents.data(), sizeof(BEnt) * b->h_ents.size())) != CS_OK)
     return rc;
+  uint64_t most = 0;
+  for (const BatchGeo& g : b->geo) most = std::max(most, g.nv);
+  cs_internal_id_words(b->d_ids, b->d_p2_geo, b->count, most, b->d_p2_words, b->stream);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(b->stream));   /* the host vectors end here */
   b->near_ok = near;
   return CS_OK;
@@ -1180,7 +1186,7 @@ int launch_bpass2(cs_batch* b, const void* uin, void* uout, uint64_t ti)
   P2Args p{};
   p.u = uin;
   p.un = uout;
-  p.ids = b->d_ids;
+  p.words = b->d_p2_words;
   p.params = b->d_params;
   p.geos = b->d_p2_geo;
   p.tiles = b->d_p2_tiles;

@@ -22,6 +22,11 @@ struct P2Geo {
   uint32_t pad;
 };
 
+/* A voxel's word: its id byte (cs_device.h), then three bits each for the
+ * domains of its neighbours at x-1, x+1, y-1, y+1, z-1, z+1 (its own domain
+ * beyond the grid's faces). */
+constexpr uint32_t P2_NB = 8;
+
 /* A block's work: lanes cover the w x h columns from (x0, y0), a ring of
  * one column around the owned columns [ix0, ix1) x [iy0, iy1) wherever
  * those do not end at the grid's face; planes [z0, z1). */
@@ -40,7 +45,7 @@ struct P2Tile {
 struct P2Args {
   const void* u;
   void* un;
-  const uint8_t* ids;
+  const uint32_t* words;   /* per voxel, at id_off + voxel */
   const void* params;
   const P2Geo* geos;
   const P2Tile* tiles;
@@ -73,6 +78,10 @@ constexpr size_t P2_PAD = 64;
 
 /* Launch the pass compiled for the step masks m1, m2; false when there is
  * none. */
+/* The words of `count` domains from their ids (blocks of 256 voxels of the
+ * largest one, for each). */
+void cs_internal_id_words(const uint8_t* ids, const P2Geo* geos, uint32_t count, uint64_t most_voxels,
+                          uint32_t* words, hipStream_t stream);
 bool cs_internal_pass2(size_t esize, bool whole, uint32_t m1, uint32_t m2, const P2Args& a, hipStream_t stream);
 bool cs_internal_pass2_f32(bool whole, uint32_t m1, uint32_t m2, const P2Args& a, hipStream_t stream);
 bool cs_internal_pass2_f64(bool whole, uint32_t m1, uint32_t m2, const P2Args& a, hipStream_t stream);

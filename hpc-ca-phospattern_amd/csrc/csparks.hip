@@ -1465,6 +1465,7 @@ struct cs_context {
   bool auto_form = true;             /* no launch shape was set or tuned yet  */
   P2Split p2_split{0, 0};
   P2Geo* d_p2_geo = nullptr;
+  uint32_t* d_p2_words = nullptr;
   struct TileList { P2Tile* d = nullptr; uint32_t n = 0; };
   std::map<int, TileList> p2_lists;
 };
@@ -1533,7 +1534,7 @@ void free_ctx(cs_context* c)
                   c->d_row_voxel, c->d_row_species, c->d_row_start, c->d_ent_pair,
                   c->d_ent_flux, c->d_ent_sign, c->d_uniforms, c->d_partial, c->d_stats,
                   c->d_lweights, c->d_lpart, c->d_xyz, c->d_f2_col, c->d_f2_z,
-                  c->d_f2_l1, c->d_f2_fsum, c->d_bchan, c->d_brow, c->d_bent, c->d_p2_geo,
+                  c->d_f2_l1, c->d_f2_fsum, c->d_bchan, c->d_brow, c->d_bent, c->d_p2_geo, c->d_p2_words,
                   c->d_bg_group, c->d_bg_vox, c->d_bg_chan, c->d_bg_row, c->d_bg_ent};
   for (auto& kv : c->p2_lists)
     if (kv.second.d) hipFree(kv.second.d);
@@ -1823,7 +1824,7 @@ int launch_pass2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout,
   P2Args p{};
   p.u = uin;
   p.un = uout;
-  p.ids = c->d_ids;
+  p.words = c->d_p2_words;
   p.params = c->d_params;
   p.geos = c->d_p2_geo;
   p.tiles = tl.d;
@@ -2120,6 +2121,10 @@ int setup_pass2(cs_context* c)
   const P2Geo rec{0, 0, 0, (uint32_t)g.plane, g.nx, g.ny, g.nz, 0};
   HIP_TRY(hipMalloc((void**)&c->d_p2_geo, sizeof rec));
   HIP_TRY(hipMemcpy(c->d_p2_geo, &rec, sizeof rec, hipMemcpyHostToDevice));
+  if (hipMalloc((void**)&c->d_p2_words, sizeof(uint32_t) * g.nv) != hipSuccess)
+    return set_err(CS_ENOMEM, "device allocation of %zu bytes failed", (size_t)(sizeof(uint32_t) * g.nv));
+  cs_internal_id_words(c->d_ids, c->d_p2_geo, 1, g.nv, c->d_p2_words, c->stream);
+  HIP_TRY(hipGetLastError());
   c->p2_ok = true;
   return CS_OK;
 }

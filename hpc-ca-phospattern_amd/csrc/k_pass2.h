@@ -24,8 +24,14 @@
  * per value and neighbour, tiles wide in x, and two blocks to a compute
  * unit where the smaller tile's traffic stays in the cache (p2_whole).  A
  * pass over two steps, before (k_step2 in FP32, two k_stencil in FP64) and
- * now: 400x400x200 FP32 455 and 334 us, FP64 1076 and 661 us; 201x187x91
- * FP32 78 and 42 us; 84^3 FP64 43 and 26 us; 64x64x25 FP64 21 and 14 us.
+ * now: 400x400x200 FP32 455 and 329 us, FP64 1076 and 669 us; 201x187x91
+ * FP32 78 and 39 us; 84^3 FP64 43 and 23 us; 64x64x25 FP64 21 and 14 us.
+ *
+ * A lane reads one word per voxel, its id and its six neighbours' domains
+ * (k_id_words), three planes ahead.  Bytes of ids, with six more loads where
+ * a wave meets an interface, held a whole block up at each such plane: 512
+ * dyads at 6 nm, 25 planes each, took 683 us a pass with them, 631 with the
+ * words and 582 with no interface at all.
  *
  * Per voxel and level the arithmetic is stencil_columns' and
  * react_species_major's.  A lane keeps the rate and coefficient tables of
@@ -186,12 +192,14 @@ k_pass2(P2Args a)
   const int zb = max(z0 - 2, 0), ze = min(nz, z1 + 2);
   const T* u = (const T*)a.u + g.u_off;
   T* un = (T*)a.un + g.u_off;
-  const uint8_t* ids = a.ids + g.id_off;
   const Rsrc rin = make_rsrc(u + (size_t)zb * NS * plane, (uint32_t)(ze - zb) * gbytes + 16);
   const Rsrc rout = make_rsrc(un + (size_t)z0 * NS * plane, (uint32_t)(z1 - z0) * gbytes);
-  const Rsrc rid = make_rsrc(ids + (size_t)zb * plane, (uint32_t)(ze - zb) * (uint32_t)plane);
+  const Rsrc rid = make_rsrc(a.words + g.id_off + (size_t)zb * plane, (uint32_t)(ze - zb) * (uint32_t)plane * 4u);
   auto gofs = [&](int zz) { return (uint32_t)(min(max(zz, zb), ze - 1) - zb) * gbytes; };
-  auto iofs = [&](int zz) { return (uint32_t)(min(max(zz, zb), ze - 1) - zb) * (uint32_t)plane; };
+  auto word = [&](int zz) {
+    return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
+        rid, (int)(col * 4u), (int)((uint32_t)(min(max(zz, zb), ze - 1) - zb) * (uint32_t)plane * 4u), 0);
+  };
 
   const bool dirichlet = P->dirichlet != 0;
   const bool gface = x == 0 || y == 0 || x + 1 == nx || y + 1 == ny;
@@ -237,16 +245,8 @@ k_pass2(P2Args a)
           nw[s] = fma(R.diag[s], (ezm + ezp) + (eym + eyp) + (exm + exp_), c);
         }
     } else {
-      const uint32_t szi = iofs(zz);
-      int dxm = d, dxp = d, dym = d, dyp = d, dzm = d, dzp = d;
-      if (!uni) {
-        dxm = bload_u8(rid, x > 0 ? col - 1 : col, szi) & 7;
-        dxp = bload_u8(rid, x + 1 < nx ? col + 1 : col, szi) & 7;
-        dym = bload_u8(rid, y > 0 ? col - (uint32_t)nx : col, szi) & 7;
-        dyp = bload_u8(rid, y + 1 < ny ? col + (uint32_t)nx : col, szi) & 7;
-        dzm = bload_u8(rid, col, iofs(zz - 1)) & 7;
-        dzp = bload_u8(rid, col, iofs(zz + 1)) & 7;
-      }
+      auto nb = [&](int k) { return (int)(id >> (P2_NB + 3 * k)) & 7; };
+      const int dxm = nb(0), dxp = nb(1), dym = nb(2), dyp = nb(3), dzm = nb(4), dzp = nb(5);
 #pragma unroll
       for (int s = 0; s < NS; s++)
         if ((M >> s) & 1u) {
@@ -308,7 +308,7 @@ k_pass2(P2Args a)
   /* Registers.  A0..A2: this column at planes z-1, z, z+1 of the species
    * step 1 diffuses; B0..B2: level 1 at z-2, z-1, z; Q: chunks of plane z+2
    * (from the middle of a plane's work on, of z+3) on their way to LDS;
-   * I0..I5: ids.  The names rotate with period six, so nothing is copied. */
+   * I0..I5: words.  The names rotate with period six, so nothing is copied. */
   T A0[NS], A1[NS], A2[NS], B0[NS], B1[NS], B2[NS];
   u32x4v Q[NQ];
   uint32_t I0, I1, I2, I3, I4 = 0, I5 = 0;
@@ -323,10 +323,10 @@ k_pass2(P2Args a)
       A0[s] = A1[s] = A2[s] = T(0);
       if ((M1 >> s) & 1u) A0[s] = bload<T>(rin, bc, gofs(zs - 1) + s * pbytes);
     }
-    I0 = bload_u8(rid, col, iofs(zs - 1));
-    I1 = bload_u8(rid, col, iofs(zs));
-    I2 = bload_u8(rid, col, iofs(zs + 1));
-    I3 = bload_u8(rid, col, iofs(zs + 2));
+    I0 = word(zs - 1);
+    I1 = word(zs);
+    I2 = word(zs + 1);
+    I3 = word(zs + 2);
     put(0, q);
     put(1, r);
     __builtin_amdgcn_s_waitcnt(0);
@@ -381,7 +381,7 @@ k_pass2(P2Args a)
     L1.put(buf, ln, wn);
     put(s2, Q);
     fetch(z + 3, Q);
-    iqn = bload_u8(rid, col, iofs(z + 3));
+    iqn = word(z + 3);
     if constexpr (l2) {
       const int zo = z - 1;
       T xm2[NS], xp2[NS], ym2[NS], yp2[NS], nw[NS];
