@@ -1063,7 +1063,11 @@ struct DomCounts {
  * The resting value is added once per domain by k_stats_final: rounding
  * is monotone, so min(u' + r) = min(u') + r exactly, and the sum is
  * sum(u') dV + n r dV.  A wavefront whose lanes share one domain updates
- * only that domain's accumulators. */
+ * only that domain's accumulators.  A block takes one species: the blocks
+ * of all species run at once, so their reductions at the end overlap the
+ * loads of others.  Per call, one species after the other in a block and
+ * now: 20x18x14 FP64 24.5 and 7.0 us, 400x400x200 FP32 410 and 315 us, FP64
+ * 608 and 482 us. */
 template <typename T>
 __global__ void __launch_bounds__(STAT_THREADS)
 k_stats(const T* __restrict__ u, const uint8_t* __restrict__ ids, Geo g, uint32_t ns, double dV,
@@ -1076,77 +1080,75 @@ k_stats(const T* __restrict__ u, const uint8_t* __restrict__ ids, Geo g, uint32_
   const int nw = STAT_THREADS / 64;
   const uint32_t blk = blockIdx.y * gridDim.x + blockIdx.x;
   const T inf = (T)INFINITY;
-  for (uint32_t s = 0; s < ns; s++) {
-    T mn[MAXD], mx[MAXD];
-    double sm[MAXD];
+  const uint32_t s = blockIdx.z;
+  T mn[MAXD], mx[MAXD];
+  double sm[MAXD];
 #pragma unroll
-    for (int d = 0; d < MAXD; d++) { mn[d] = inf; mx[d] = -inf; sm[d] = 0.0; }
-    auto upd = [&](int d, T v) {
-      mn[d] = v < mn[d] ? v : mn[d];
-      mx[d] = v > mx[d] ? v : mx[d];
-      sm[d] += (double)v;
-    };
-    /* eight strided elements per lane are loaded before any is used, so
-     * each wavefront keeps several loads in flight */
-    constexpr int U = 8;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (int z = blockIdx.y; z < g.nz; z += gridDim.y) {
-      const T* us = u + ((uint64_t)z * ns + s) * g.plane;
-      const uint8_t* iz = ids + (uint64_t)z * g.plane;
-      for (uint64_t c0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c0 < g.plane; c0 += U * stride) {
-        T v[U];
-        int dv[U];
+  for (int d = 0; d < MAXD; d++) { mn[d] = inf; mx[d] = -inf; sm[d] = 0.0; }
+  auto upd = [&](int d, T v) {
+    mn[d] = v < mn[d] ? v : mn[d];
+    mx[d] = v > mx[d] ? v : mx[d];
+    sm[d] += (double)v;
+  };
+  /* eight strided elements per lane are loaded before any is used, so
+   * each wavefront keeps several loads in flight */
+  constexpr int U = 8;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (int z = blockIdx.y; z < g.nz; z += gridDim.y) {
+    const T* us = u + ((uint64_t)z * ns + s) * g.plane;
+    const uint8_t* iz = ids + (uint64_t)z * g.plane;
+    for (uint64_t c0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c0 < g.plane; c0 += U * stride) {
+      T v[U];
+      int dv[U];
 #pragma unroll
-        for (int k = 0; k < U; k++) {
-          const uint64_t c = c0 + k * stride;
-          dv[k] = -1;   /* past the plane: no domain */
-          v[k] = T(0);
-          if (c < g.plane) {
-            dv[k] = iz[c] & 7;
-            v[k] = us[c];
-          }
+      for (int k = 0; k < U; k++) {
+        const uint64_t c = c0 + k * stride;
+        dv[k] = -1;   /* past the plane: no domain */
+        v[k] = T(0);
+        if (c < g.plane) {
+          dv[k] = iz[c] & 7;
+          v[k] = us[c];
         }
+      }
 #pragma unroll
-        for (int k = 0; k < U; k++) {
-          const int d0 = __builtin_amdgcn_readfirstlane(dv[k]);
-          if (__ballot(dv[k] != d0) == 0) {
-            switch (d0) {
-              case 0: upd(0, v[k]); break;
-              case 1: upd(1, v[k]); break;
-              case 2: upd(2, v[k]); break;
-              case 3: upd(3, v[k]); break;
-              case 4: upd(4, v[k]); break;
-              default: break;   /* every lane past the plane */
-            }
-          } else {
-#pragma unroll
-            for (int d = 0; d < MAXD; d++)
-              if (d == dv[k]) upd(d, v[k]);
+      for (int k = 0; k < U; k++) {
+        const int d0 = __builtin_amdgcn_readfirstlane(dv[k]);
+        if (__ballot(dv[k] != d0) == 0) {
+          switch (d0) {
+            case 0: upd(0, v[k]); break;
+            case 1: upd(1, v[k]); break;
+            case 2: upd(2, v[k]); break;
+            case 3: upd(3, v[k]); break;
+            case 4: upd(4, v[k]); break;
+            default: break;   /* every lane past the plane */
           }
+        } else {
+#pragma unroll
+          for (int d = 0; d < MAXD; d++)
+            if (d == dv[k]) upd(d, v[k]);
         }
       }
     }
-    double dmn[MAXD], dmx[MAXD];
+  }
+  double dmn[MAXD], dmx[MAXD];
 #pragma unroll
-    for (int d = 0; d < MAXD; d++) {
-      dmn[d] = (double)mn[d];
-      dmx[d] = (double)mx[d];
-      sm[d] *= dV;
+  for (int d = 0; d < MAXD; d++) {
+    dmn[d] = (double)mn[d];
+    dmx[d] = (double)mx[d];
+    sm[d] *= dV;
+  }
+  block_reduce3<T>(dmn, dmx, sm, sh);
+  __syncthreads();
+  if (threadIdx.x < MAXD) {
+    const int d = threadIdx.x;
+    double a = sh[(0 * MAXD + d) * nw], b = sh[(1 * MAXD + d) * nw], c = sh[(2 * MAXD + d) * nw];
+    for (int w = 1; w < nw; w++) {
+      a = fmin(a, sh[(0 * MAXD + d) * nw + w]);
+      b = fmax(b, sh[(1 * MAXD + d) * nw + w]);
+      c += sh[(2 * MAXD + d) * nw + w];
     }
-    block_reduce3<T>(dmn, dmx, sm, sh);
-    __syncthreads();
-    if (threadIdx.x < MAXD) {
-      const int d = threadIdx.x;
-      double a = sh[(0 * MAXD + d) * nw], b = sh[(1 * MAXD + d) * nw], c = sh[(2 * MAXD + d) * nw];
-      for (int w = 1; w < nw; w++) {
-        a = fmin(a, sh[(0 * MAXD + d) * nw + w]);
-        b = fmax(b, sh[(1 * MAXD + d) * nw + w]);
-        c += sh[(2 * MAXD + d) * nw + w];
-      }
-      double* o = partial + (((uint64_t)blk * ns + s) * MAXD + d) * 3;
-      o[0] = a; o[1] = b; o[2] = c;
-    }
-    __syncthreads();
+    double* o = partial + (((uint64_t)blk * ns + s) * MAXD + d) * 3;
+    o[0] = a; o[1] = b; o[2] = c;
   }
 }
 
@@ -2521,12 +2523,12 @@ int cs_reduce_stats(cs_context* c, double* mn, double* mx, double* tot)
   DomCounts cnt{};
   for (uint32_t d = 0; d < MAXD; d++) cnt.n[d] = c->dcount[d];
   if (c->esize == 8) {
-    hipLaunchKernelGGL(k_stats<double>, dim3(gx, gy), dim3(STAT_THREADS), 0, c->stream,
+    hipLaunchKernelGGL(k_stats<double>, dim3(gx, gy, c->ns), dim3(STAT_THREADS), 0, c->stream,
                        (const double*)c->d_u[c->cur], c->d_ids, c->geo, c->ns, dV, c->d_partial);
     hipLaunchKernelGGL(k_stats_final<double>, dim3(c->ns * MAXD), dim3(STAT_THREADS), 0, c->stream, c->d_partial,
                        blocks, c->ns, (const DevParams<double>*)c->d_params, cnt, dV, c->d_stats);
   } else {
-    hipLaunchKernelGGL(k_stats<float>, dim3(gx, gy), dim3(STAT_THREADS), 0, c->stream,
+    hipLaunchKernelGGL(k_stats<float>, dim3(gx, gy, c->ns), dim3(STAT_THREADS), 0, c->stream,
                        (const float*)c->d_u[c->cur], c->d_ids, c->geo, c->ns, dV, c->d_partial);
     hipLaunchKernelGGL(k_stats_final<float>, dim3(c->ns * MAXD), dim3(STAT_THREADS), 0, c->stream, c->d_partial,
                        blocks, c->ns, (const DevParams<float>*)c->d_params, cnt, dV, c->d_stats);
