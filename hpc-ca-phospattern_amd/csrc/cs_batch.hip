@@ -1045,10 +1045,10 @@ int index_kept_voxels(cs_batch* b, bool near)
   const size_t n = std::max<size_t>(vz.size(), 1);
   HIP_TRY(hipMalloc(&b->d_p2_col, sizeof(uint32_t) * col_start.size()));
   HIP_TRY(hipMalloc(&b->d_p2_z, sizeof(uint32_t) * n));
-  HIP_TRY(hipMalloc(&b->d_p2_fsum, sizeof(double) * n));
+  HIP_TRY(hipMalloc(&b->d_p2_fsum, sizeof(double) * (n + 1)));
   HIP_TRY(hipMalloc(&b->d_p2_l1, b->esize * n));
   if (near) HIP_TRY(hipMalloc(&b->d_near, sizeof(uint32_t) * std::max<size_t>(slots.size(), 1)));
-  const std::vector<double> zero(n, 0.0);   /* voxels without a row keep a zero sum */
+  const std::vector<double> zero(n + 1, 0.0);   /* voxels without a row keep a zero sum */
   auto up = [b](void* dst, const void* src, size_t bytes) -> int {
     if (bytes) HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream));
     return CS_OK;
@@ -1056,7 +1056,7 @@ int index_kept_voxels(cs_batch* b, bool near)
   int rc;
   if ((rc = up(b->d_p2_col, col_start.data(), sizeof(uint32_t) * col_start.size())) != CS_OK ||
       (rc = up(b->d_p2_z, vz.data(), sizeof(uint32_t) * vz.size())) != CS_OK ||
-      (rc = up(b->d_p2_fsum, zero.data(), sizeof(double) * n)) != CS_OK ||
+      (rc = up(b->d_p2_fsum, zero.data(), sizeof(double) * (n + 1))) != CS_OK ||
       (rc = up(b->d_near, slots.data(), sizeof(uint32_t) * slots.size())) != CS_OK ||
       (rc = up(b->d_ids, ids.data(), ids.size())) != CS_OK ||
       (rc = up(b->d_chan, b->h_chan.data(), sizeof(BatchChan) * b->h_chan.size())) != CS_OK ||

@@ -39,8 +39,8 @@ struct P2Tile {
 /* One launch.  react: the step runs the buffer reactions (species-major).
  * The pair voxels of every domain, ordered by column and then z: vz[k] the
  * plane of pair voxel k, col_start[geo.col_off + column] its column's
- * first; fsum[k] the flux sum that step 1 adds to species 0 there, l1[k]
- * receives species 0 after step 1.  any_fixed: some domain holds fixed
+ * first; fsum[k] the flux sum that step 1 adds to species 0 there (one entry
+ * more than there are pair voxels), l1[k] receives species 0 after step 1.  any_fixed: some domain holds fixed
  * species. */
 struct P2Args {
   const void* u;

@@ -2285,8 +2285,8 @@ int build_flux_rows(cs_context* c, const cs_problem* p)
       return rc;
   }
   HIP_TRY(hipMalloc(&c->d_f2_l1, c->esize * std::max<size_t>(keys.size(), 1)));
-  HIP_TRY(hipMalloc((void**)&c->d_f2_fsum, sizeof(double) * std::max<size_t>(keys.size(), 1)));
-  HIP_TRY(hipMemsetAsync(c->d_f2_fsum, 0, sizeof(double) * std::max<size_t>(keys.size(), 1), c->stream));
+  HIP_TRY(hipMalloc((void**)&c->d_f2_fsum, sizeof(double) * (keys.size() + 1)));
+  HIP_TRY(hipMemsetAsync(c->d_f2_fsum, 0, sizeof(double) * (keys.size() + 1), c->stream));
   /* the host vectors above end here */
   HIP_TRY(hipStreamSynchronize(c->stream));
   return CS_OK;
