@@ -13,7 +13,7 @@ Prints one JSON line.  `value` is the whole-step algorithmic HBM
 bandwidth: 41 B per voxel-step (1 B domain id + 5 species x (4 B read +
 4 B write)) x voxels / step time.  `roofline` prices the stencil pass
 alone (HIP events on its stream): a one-step pass (k_stencil) or a fused
-two-step pass (k_step2, the default where the problem admits it), priced
+two-step pass (k_pass2, the default for this species layout), priced
 at 41 B per voxel-step times the voxel-steps one launch processes (one
 or two per voxel).  `traffic` is the HBM bytes per launch that committed
 rocprofv3 counters measured for the same launch shape and kernel source
@@ -21,7 +21,7 @@ rocprofv3 counters measured for the same launch shape and kernel source
 FP64 C oracle on the host cores for a bounded sample of the same workload.
 
 Sub-records of the same line:
-  fp64      the same dyad with FP64 fields (one-step passes), the
+  fp64      the same dyad with FP64 fields, the
             reference's own precision, and the per-species error of the
             FP32 fields against the FP64 ones after 200 steps;
   g1        the run the reference publishes its own timing for (G1 at 12
@@ -90,12 +90,13 @@ def cpu_baseline(d, budget_s=15.0):
     return nv * steps / el, cores, steps, el
 
 
-TRAFFIC_SOURCES = ("csparks.hip", "cs_device.h", "cs_physics.h")
+TRAFFIC_SOURCES = ("csparks.hip", "cs_device.h", "cs_physics.h", "cs_pass2.h", "k_pass2.h", "cs_pass2_f32.hip",
+                   "cs_pass2_f64.hip")
 
 
 def kernel_source_hash() -> str:
     """SHA-256 of the HIP sources of the single-domain kernels (k_stencil,
-    k_step2 and what they include), which the committed traffic profile
+    k_step2, k_pass2 and what they include), which the committed traffic profile
     records: a profile of other sources is stale."""
     h = hashlib.sha256()
     csrc = os.path.join(REPO, "hpc-ca-phospattern_amd", "csrc")
@@ -105,8 +106,15 @@ def kernel_source_hash() -> str:
     return h.hexdigest()
 
 
+def pass_kernel(launch, passes, fused):
+    """The kernel of a timed range: two-step passes run as k_pass2 unless
+    the launch asks for run-time masks (fuse_fixed 0)."""
+    two = "k_pass2" if launch["fuse_fixed"] else "k_step2"
+    return two if fused == passes else "k_stencil" if fused == 0 else two + "+k_stencil"
+
+
 def fp64_record(size, steps):
-    """The headline dyad with FP64 fields (one-step passes)."""
+    """The headline dyad with FP64 fields."""
     d = dyad.cluster_dyad(seed=1, n=tuple(size))
     sim = cs.Simulation(d.geometry, d.model, cs.Options(h=3.0, seed=1, open={"ryr": [0]}, precision="f64"))
     nv = int(np.prod(sim.n))
@@ -116,12 +124,13 @@ def fp64_record(size, steps):
     total_ms, pass_ms, passes, fused = sim.time_passes(steps)
     sim.synchronize()
     wall = time.perf_counter() - t1
+    kernel = pass_kernel(sim.launch_config(), passes, fused)
     sim.close()
     ms = wall * 1e3 / steps
     kern = (steps / passes) * nv * BYTES_F64 / (pass_ms * 1e-3) / 1e9
     log(f"fp64: {ms:.4f} ms/step, pass {pass_ms * 1e3:.1f} us ({kern:.0f} GB/s)")
     return {"ms_per_step": round(ms, 4), "value": round(nv * BYTES_F64 / (ms * 1e-3) / 1e9, 1), "unit": "GB/s",
-            "bytes_per_voxel_step": BYTES_F64, "kernel": "k_stencil" if fused == 0 else "k_step2",
+            "bytes_per_voxel_step": BYTES_F64, "kernel": kernel,
             "kernel_ms": round(pass_ms, 5),
             "roofline": {"bound": "hbm", "achieved": round(kern, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                          "frac": round(kern / PEAK_HBM_GBS, 4)}}
@@ -130,7 +139,7 @@ def fp64_record(size, steps):
 def fp32_error_record(size, steps=200):
     """Per-species error of the FP32 fields against FP64 ones on the same
     dyad after `steps` steps from rest (same seed and channel trajectories;
-    FP32 in its default fused passes, FP64 in one-step passes): the largest
+    both in their default two-step passes): the largest
     |f32 - f64| over the grid divided by the largest deviation of the FP64
     field from rest.  The FP64 device path equals the FP64 oracle to 1e-10
     in the parity tests."""
@@ -247,7 +256,7 @@ def ensemble_record(count=512, steps=100):
     return {"workload": f"{count} dyads, edges 256-512 nm at 6 nm, 9-100 RyRs, 0-50% pRyR, Philox, FP32, 20 ms runs",
             "realisations": count, "voxels": nv, "ms_per_step": round(ms, 4), "steps_per_realisation": run_steps,
             "realisations_per_s": round(rate, 4), "launch": launch, "graphs": True,
-            "stencil": {"kernel": "k_batch_stencil" if launch.get("persistent") else "k_batch_tiles",
+            "stencil": {"kernel": "k_pass2",
                         "kernel_ms": round(stencil_ms, 5),
                         "achieved": round(gbs, 1), "unit": "GB/s", "frac": round(gbs / PEAK_HBM_GBS, 4)}}
 
@@ -372,7 +381,7 @@ def main():
     steps_per_launch = args.steps / passes
     kern_gbs = steps_per_launch * nv * bpv / (kernel_ms * 1e-3) / 1e9
     steps_per_real = cs.host_lib().cs_count_steps(TSTOP_MS, sim.dt)
-    kernel = "k_step2" if fused == passes else "k_stencil" if fused == 0 else "k_step2+k_stencil"
+    kernel = pass_kernel(launch, passes, fused)
     log(f"{args.steps} steps in {passes} passes ({fused} fused): wall {wall * 1e3:.1f} ms, "
         f"events {total_ms:.1f} ms, pass {kernel_ms * 1e3:.1f} us ({kern_gbs:.0f} GB/s)")
 
