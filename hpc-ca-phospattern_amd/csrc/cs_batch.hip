@@ -932,6 +932,12 @@ int setup_pass2(cs_batch* b)
   if (cols >= (1ull << 32)) return CS_OK;
   HIP_TRY(hipMalloc(&b->d_p2_geo, sizeof(P2Geo) * recs.size()));
   HIP_TRY(hipMemcpy(b->d_p2_geo, recs.data(), sizeof(P2Geo) * recs.size(), hipMemcpyHostToDevice));
+  if (hipMalloc(&b->d_p2_words, sizeof(uint32_t) * std::max<uint64_t>(b->total_ids, 1)) != hipSuccess) {
+    /* no room beside the fields: one-step passes need none */
+    (void)hipGetLastError();
+    b->d_p2_words = nullptr;
+    return CS_OK;
+  }
   b->p2_ok = b->p2_on = true;
   return CS_OK;
 }
@@ -1041,7 +1047,6 @@ int index_kept_voxels(cs_batch* b, bool near)
     if (*p) HIP_TRY(hipFree(*p));
     *p = nullptr;
   }
-  if (!b->d_p2_words) HIP_TRY(hipMalloc(&b->d_p2_words, sizeof(uint32_t) * std::max<uint64_t>(b->total_ids, 1)));
   const size_t n = std::max<size_t>(vz.size(), 1);
   HIP_TRY(hipMalloc(&b->d_p2_col, sizeof(uint32_t) * col_start.size()));
   HIP_TRY(hipMalloc(&b->d_p2_z, sizeof(uint32_t) * n));

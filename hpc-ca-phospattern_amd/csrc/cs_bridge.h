@@ -98,45 +98,62 @@ namespace {
     const uint32_t a = find(e.slot_from), b = find(e.slot_to);
     root[std::max(a, b)] = std::min(a, b);
   }
-  struct Part { std::vector<uint32_t> vox, chan, row; uint32_t nent = 0; };
-  std::vector<Part> parts(nslots);
-  for (uint32_t v = 0; v < nslots; v++) parts[find(v)].vox.push_back(v);
-  for (uint32_t c = 0; c < chans.size(); c++) parts[find(chans[c].slot_to)].chan.push_back(c);
-  for (uint32_t r = 0; r < rows.size(); r++) {
-    Part& p = parts[find(rows[r].slot)];
-    p.row.push_back(r);
-    p.nent += rows[r].end - rows[r].start;
-  }
+  /* components in the order of their first slot, and the voxels, channels
+   * and rows of each (a root is its component's first slot) */
+  uint32_t ncomp = 0;
+  std::vector<uint32_t> comp(nslots);
+  for (uint32_t v = 0; v < nslots; v++) comp[v] = find(v) == v ? ncomp++ : comp[find(v)];
+  struct Lists {
+    std::vector<uint32_t> start, item;
+    Lists(size_t n, uint32_t ncomp) : start(ncomp + 1, 0), item(n) {}
+    uint32_t size(uint32_t c) const { return start[c + 1] - start[c]; }
+    const uint32_t* begin(uint32_t c) const { return item.data() + start[c]; }
+  };
+  auto lists = [&](size_t n, auto slot) {
+    Lists l(n, ncomp);
+    for (size_t k = 0; k < n; k++) l.start[comp[slot(k)] + 1]++;
+    for (uint32_t c = 0; c < ncomp; c++) l.start[c + 1] += l.start[c];
+    std::vector<uint32_t> next(l.start.begin(), l.start.end() - 1);
+    for (size_t k = 0; k < n; k++) l.item[next[comp[slot(k)]]++] = (uint32_t)k;
+    return l;
+  };
+  const Lists pvox = lists(nslots, [](size_t k) { return (uint32_t)k; });
+  const Lists pchan = lists(chans.size(), [&](size_t k) { return chans[k].slot_to; });
+  const Lists prow = lists(rows.size(), [&](size_t k) { return rows[k].slot; });
   out = BgTables{};
   std::vector<uint16_t> local(nslots, 0);
   BgGroup g{};
-  for (const Part& p : parts) {
-    if (p.vox.empty()) continue;
-    if (p.vox.size() > BG_VOX || p.chan.size() > BG_CHAN || p.row.size() > BG_ROW || p.nent > BG_ENT) return false;
-    if (g.nvox && (g.nrow + p.row.size() > BG_FILL || g.nvox + p.vox.size() > BG_VOX ||
-                   g.nchan + p.chan.size() > BG_CHAN || g.nent + p.nent > BG_ENT)) {
+  for (uint32_t p = 0; p < ncomp; p++) {
+    const uint32_t nvox = pvox.size(p), nchan = pchan.size(p), nrow = prow.size(p);
+    uint32_t nent = 0;
+    for (uint32_t k = 0; k < nrow; k++) nent += rows[prow.begin(p)[k]].end - rows[prow.begin(p)[k]].start;
+    if (nvox > BG_VOX || nchan > BG_CHAN || nrow > BG_ROW || nent > BG_ENT) return false;
+    if (g.nvox && (g.nrow + nrow > BG_FILL || g.nvox + nvox > BG_VOX || g.nchan + nchan > BG_CHAN ||
+                   g.nent + nent > BG_ENT)) {
       out.groups.push_back(g);
       g = BgGroup{(uint32_t)out.vox.size(), 0, (uint32_t)out.chan.size(), 0, (uint32_t)out.row.size(), 0,
                   (uint32_t)out.ent.size(), 0};
     }
-    for (uint32_t v : p.vox) {
+    for (uint32_t k = 0; k < nvox; k++) {
+      const uint32_t v = pvox.begin(p)[k];
       local[v] = (uint16_t)g.nvox++;
       out.vox.push_back(all[v]);
     }
     const uint32_t c0 = g.nchan;
-    for (uint32_t c : p.chan) {
+    for (uint32_t k = 0; k < nchan; k++) {
+      const uint32_t c = pchan.begin(p)[k];
       out.chan.push_back(BgChan{local[chans[c].slot_to], chans[c].flux, chans[c].ch, chans[c].state});
       g.nchan++;
     }
-    for (uint32_t r : p.row) {
-      const BRow& w = rows[r];
+    for (uint32_t q = 0; q < nrow; q++) {
+      const BRow& w = rows[prow.begin(p)[q]];
       out.row.push_back(BgRow{local[w.slot], (uint16_t)w.skip, (uint16_t)g.nent, (uint16_t)(w.end - w.start)});
       g.nrow++;
       for (uint32_t e = w.start; e < w.end; e++) {
         const BEnt& x = ents[e];
         uint16_t chan = BG_NONE;
-        for (uint32_t k = 0; x.state != NO_ROW && k < p.chan.size(); k++)
-          if (chans[p.chan[k]].state == x.state) { chan = (uint16_t)(c0 + k); break; }
+        for (uint32_t k = 0; x.state != NO_ROW && k < nchan; k++)
+          if (chans[pchan.begin(p)[k]].state == x.state) { chan = (uint16_t)(c0 + k); break; }
         if (x.state != NO_ROW && chan == BG_NONE) return false;
         out.ent.push_back(BgEnt{local[x.slot_from], local[x.slot_to], chan, (uint16_t)x.flux_sign});
         g.nent++;

@@ -2123,8 +2123,12 @@ int setup_pass2(cs_context* c)
   const P2Geo rec{0, 0, 0, (uint32_t)g.plane, g.nx, g.ny, g.nz, 0};
   HIP_TRY(hipMalloc((void**)&c->d_p2_geo, sizeof rec));
   HIP_TRY(hipMemcpy(c->d_p2_geo, &rec, sizeof rec, hipMemcpyHostToDevice));
-  if (hipMalloc((void**)&c->d_p2_words, sizeof(uint32_t) * g.nv) != hipSuccess)
-    return set_err(CS_ENOMEM, "device allocation of %zu bytes failed", (size_t)(sizeof(uint32_t) * g.nv));
+  if (hipMalloc((void**)&c->d_p2_words, sizeof(uint32_t) * g.nv) != hipSuccess) {
+    /* no room beside the fields: the other passes need none */
+    (void)hipGetLastError();
+    c->d_p2_words = nullptr;
+    return CS_OK;
+  }
   cs_internal_id_words(c->d_ids, c->d_p2_geo, 1, g.nv, c->d_p2_words, c->stream);
   HIP_TRY(hipGetLastError());
   c->p2_ok = true;
