@@ -816,12 +816,19 @@ struct cs_batch {
 
 namespace {
 
+void drop_graphs(cs_batch* b)
+{
+  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second.exec);
+  for (auto g : b->graph_defs) (void)hipGraphDestroy(g);
+  b->graphs.clear();
+  b->graph_defs.clear();
+}
+
 void free_batch(cs_batch* b)
 {
   if (!b) return;
   (void)hipSetDevice(b->device);
-  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second.exec);
-  for (auto g : b->graph_defs) (void)hipGraphDestroy(g);
+  drop_graphs(b);
   void* ptrs[] = {b->d_u[0], b->d_u[1], b->d_ids, b->d_params, b->d_geo, b->d_tiles, b->d_queue, b->d_inst,
                   b->d_chan, b->d_rows, b->d_ents, b->d_states, b->d_recruited, b->d_active, b->d_last_open,
                   b->d_cgeo, b->d_nb_start, b->d_nb, b->d_cpred, b->d_fpred, b->d_chca, b->d_feat, b->d_flags,
@@ -906,6 +913,18 @@ int upload_tiles(cs_batch* b)
   return CS_OK;
 }
 
+/* No room beside the fields for what two-step passes need: one-step passes
+ * need none of it. */
+void drop_pass2(cs_batch* b)
+{
+  if (b->d_p2_geo) (void)hipFree(b->d_p2_geo);
+  if (b->d_p2_words) (void)hipFree(b->d_p2_words);
+  b->d_p2_geo = nullptr;
+  b->d_p2_words = nullptr;
+  b->p2_ok = b->p2_on = false;
+  (void)hipGetLastError();
+}
+
 /* Whether two-step passes (k_pass2) fit the ensemble: the five-slot layout
  * with its substeps, fluxes on Ca only, and on every grid at least two
  * columns either way and a split whose blocks hold a tile.  Half blocks:
@@ -930,14 +949,12 @@ int setup_pass2(cs_batch* b)
     cols += g.plane + 1;
   }
   if (cols >= (1ull << 32)) return CS_OK;
-  HIP_TRY(hipMalloc(&b->d_p2_geo, sizeof(P2Geo) * recs.size()));
-  HIP_TRY(hipMemcpy(b->d_p2_geo, recs.data(), sizeof(P2Geo) * recs.size(), hipMemcpyHostToDevice));
-  if (hipMalloc(&b->d_p2_words, sizeof(uint32_t) * std::max<uint64_t>(b->total_ids, 1)) != hipSuccess) {
-    /* no room beside the fields: one-step passes need none */
-    (void)hipGetLastError();
-    b->d_p2_words = nullptr;
+  if (hipMalloc(&b->d_p2_geo, sizeof(P2Geo) * recs.size()) != hipSuccess ||
+      hipMalloc(&b->d_p2_words, sizeof(uint32_t) * std::max<uint64_t>(b->total_ids, 1)) != hipSuccess) {
+    drop_pass2(b);
     return CS_OK;
   }
+  HIP_TRY(hipMemcpy(b->d_p2_geo, recs.data(), sizeof(P2Geo) * recs.size(), hipMemcpyHostToDevice));
   b->p2_ok = b->p2_on = true;
   return CS_OK;
 }
@@ -985,12 +1002,17 @@ int upload_pass2_tiles(cs_batch* b)
 
 /* The voxels whose level-1 Ca the passes keep: those of the boundary pairs
  * and, with near, those a closure reads.  Marks them in the ids, indexes
- * them by column and plane, and gives every record its slots. */
-int index_kept_voxels(cs_batch* b, bool near)
+ * them by column and plane, and gives every record its slots.  The new index
+ * takes the old one's place once all of it is on the device; without memory
+ * for it (fits false) everything stays as it was. */
+int index_kept_voxels(cs_batch* b, bool near, bool& fits)
 {
   std::vector<uint32_t> col_start, vz, slots;
   std::vector<uint8_t> ids(b->total_ids, 0);
-  if (near) slots.assign((size_t)CLOSURE_NEAR * b->h_chan.size(), 0);
+  std::vector<BatchChan> chan = b->h_chan;
+  std::vector<BRow> rows = b->h_rows;
+  std::vector<BEnt> ents = b->h_ents;
+  if (near) slots.assign((size_t)CLOSURE_NEAR * chan.size(), 0);
   for (uint32_t i = 0; i < b->count; i++) {
     const BatchGeo& g = b->geo[i];
     const BatchInst& in = b->h_inst[i];
@@ -1016,64 +1038,91 @@ int index_kept_voxels(cs_batch* b, bool near)
     const uint32_t base = (uint32_t)vz.size();
     const size_t c0 = col_start.size();
     col_start.resize(c0 + g.plane + 1, 0);
-    for (uint8_t& id : b->h_ids[i]) id &= (uint8_t)~ID_PAIR;
+    for (uint64_t v = 0; v < g.nv; v++) ids[g.id_off + v] = b->h_ids[i][v] & (uint8_t)~ID_PAIR;
     for (uint64_t k : keys) {
       const uint64_t col = k >> 32, z = k & 0xFFFFFFFFu;
       vz.push_back((uint32_t)z);
       col_start[c0 + col + 1]++;
-      b->h_ids[i][z * g.plane + col] |= ID_PAIR;
+      ids[g.id_off + z * g.plane + col] |= ID_PAIR;
     }
     col_start[c0] = base;
     for (uint64_t k = 1; k <= g.plane; k++) col_start[c0 + k] += col_start[c0 + k - 1];
-    memcpy(ids.data() + g.id_off, b->h_ids[i].data(), g.nv);
     auto slot = [&](uint64_t v) {
       return base + (uint32_t)(std::lower_bound(keys.begin(), keys.end(), key(v)) - keys.begin());
     };
     for (uint32_t c = in.chan_off; c < in.chan_off + in.nchan; c++) {
       const BatchChanGeo& cg = b->h_cgeo[c];
-      b->h_chan[c].slot_to = slot((uint64_t)cg.z * g.plane + (uint64_t)cg.y * g.nx + cg.x);
+      chan[c].slot_to = slot((uint64_t)cg.z * g.plane + (uint64_t)cg.y * g.nx + cg.x);
       if (near)
         for (uint32_t k = 0; k < CLOSURE_NEAR; k++) slots[(size_t)CLOSURE_NEAR * c + k] = slot(around(c, k));
     }
     for (uint32_t r = in.row_off; r < in.row_off + in.nrows; r++) {
-      b->h_rows[r].slot = slot(b->row_voxel[r]);
-      for (uint32_t e = b->h_rows[r].start; e < b->h_rows[r].end; e++) {
-        b->h_ents[e].slot_from = slot(b->ent_voxel[2 * e]);
-        b->h_ents[e].slot_to = slot(b->ent_voxel[2 * e + 1]);
+      rows[r].slot = slot(b->row_voxel[r]);
+      for (uint32_t e = rows[r].start; e < rows[r].end; e++) {
+        ents[e].slot_from = slot(b->ent_voxel[2 * e]);
+        ents[e].slot_to = slot(b->ent_voxel[2 * e + 1]);
       }
     }
   }
-  for (void** p : {(void**)&b->d_p2_col, (void**)&b->d_p2_z, (void**)&b->d_p2_fsum, &b->d_p2_l1, (void**)&b->d_near}) {
-    if (*p) HIP_TRY(hipFree(*p));
-    *p = nullptr;
-  }
   const size_t n = std::max<size_t>(vz.size(), 1);
-  HIP_TRY(hipMalloc(&b->d_p2_col, sizeof(uint32_t) * col_start.size()));
-  HIP_TRY(hipMalloc(&b->d_p2_z, sizeof(uint32_t) * n));
-  HIP_TRY(hipMalloc(&b->d_p2_fsum, sizeof(double) * (n + 1)));
-  HIP_TRY(hipMalloc(&b->d_p2_l1, b->esize * n));
-  if (near) HIP_TRY(hipMalloc(&b->d_near, sizeof(uint32_t) * std::max<size_t>(slots.size(), 1)));
   const std::vector<double> zero(n + 1, 0.0);   /* voxels without a row keep a zero sum */
-  auto up = [b](void* dst, const void* src, size_t bytes) -> int {
-    if (bytes) HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream));
-    return CS_OK;
+  struct Part { void** to; const void* src; size_t copied, bytes; };
+  const Part parts[] = {
+      {(void**)&b->d_p2_col, col_start.data(), sizeof(uint32_t) * col_start.size(), 0},
+      {(void**)&b->d_p2_z, vz.data(), sizeof(uint32_t) * vz.size(), sizeof(uint32_t) * n},
+      {(void**)&b->d_p2_fsum, zero.data(), sizeof(double) * (n + 1), 0},
+      {&b->d_p2_l1, nullptr, 0, b->esize * n},
+      {(void**)&b->d_near, slots.data(), sizeof(uint32_t) * slots.size(), near ? sizeof(uint32_t) : 0}};
+  constexpr size_t NPART = sizeof parts / sizeof parts[0];
+  void* fresh[NPART] = {nullptr};
+  auto drop = [&]() {
+    for (void* p : fresh)
+      if (p) (void)hipFree(p);
+    (void)hipGetLastError();
   };
-  int rc;
-  if ((rc = up(b->d_p2_col, col_start.data(), sizeof(uint32_t) * col_start.size())) != CS_OK ||
-      (rc = up(b->d_p2_z, vz.data(), sizeof(uint32_t) * vz.size())) != CS_OK ||
-      (rc = up(b->d_p2_fsum, zero.data(), sizeof(double) * (n + 1))) != CS_OK ||
-      (rc = up(b->d_near, slots.data(), sizeof(uint32_t) * slots.size())) != CS_OK ||
-      (rc = up(b->d_ids, ids.data(), ids.size())) != CS_OK ||
-      (rc = up(b->d_chan, b->h_chan.data(), sizeof(BatchChan) * b->h_chan.size())) != CS_OK ||
-      (rc = up(b->d_rows, b->h_rows.data(), sizeof(BRow) * b->h_rows.size())) != CS_OK ||
-      (rc = up(b->d_ents, b->h_ents.data(), sizeof(BEnt) * b->h_ents.size())) != CS_OK)
-    return rc;
+  fits = true;
+  for (size_t k = 0; k < NPART && fits; k++) {
+    const size_t bytes = std::max(parts[k].copied, parts[k].bytes);
+    if (bytes && hipMalloc(&fresh[k], bytes) != hipSuccess) {
+      fresh[k] = nullptr;
+      fits = false;
+    }
+  }
+  if (!fits) {
+    drop();
+    return CS_OK;
+  }
+  bool ok = true;
+  auto up = [&](void* dst, const void* src, size_t bytes) {
+    ok = ok && (!bytes || hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream) == hipSuccess);
+  };
+  for (size_t k = 0; k < NPART; k++) up(fresh[k], parts[k].src, parts[k].copied);
+  ok = ok && hipStreamSynchronize(b->stream) == hipSuccess;
+  if (!ok) {
+    drop();
+    return set_err(CS_EDEVICE, "upload of the kept voxels failed");
+  }
+  drop_graphs(b);   /* they read the old index */
+  for (size_t k = 0; k < NPART; k++) {
+    if (*parts[k].to) (void)hipFree(*parts[k].to);
+    *parts[k].to = fresh[k];
+  }
+  b->h_chan.swap(chan);
+  b->h_rows.swap(rows);
+  b->h_ents.swap(ents);
+  for (uint32_t i = 0; i < b->count; i++)
+    memcpy(b->h_ids[i].data(), ids.data() + b->geo[i].id_off, b->geo[i].nv);
+  b->near_ok = near;
+  up(b->d_ids, ids.data(), ids.size());
+  up(b->d_chan, b->h_chan.data(), sizeof(BatchChan) * b->h_chan.size());
+  up(b->d_rows, b->h_rows.data(), sizeof(BRow) * b->h_rows.size());
+  up(b->d_ents, b->h_ents.data(), sizeof(BEnt) * b->h_ents.size());
+  if (!ok) return set_err(CS_EDEVICE, "upload of the flux records failed");
   uint64_t most = 0;
   for (const BatchGeo& g : b->geo) most = std::max(most, g.nv);
   cs_internal_id_words(b->d_ids, b->d_p2_geo, b->count, most, b->d_p2_words, b->stream);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(b->stream));   /* the host vectors end here */
-  b->near_ok = near;
   return CS_OK;
 }
 
@@ -1435,14 +1484,6 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
   return CS_OK;
 }
 
-void drop_graphs(cs_batch* b)
-{
-  for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second.exec);
-  for (auto g : b->graph_defs) (void)hipGraphDestroy(g);
-  b->graphs.clear();
-  b->graph_defs.clear();
-}
-
 }  // namespace
 /* ------------------------------------------------------------- C ABI */
 
@@ -1728,7 +1769,10 @@ int cs_batch_create(const cs_problem* problems, uint32_t count, cs_batch** out)
     b->h_cgeo.swap(cgeo);
     b->h_rows.swap(rows);
     b->h_ents.swap(ents);
-    if ((rc = index_kept_voxels(b, false)) != CS_OK || (rc = upload_pass2_tiles(b)) != CS_OK) return bail(rc);
+    bool fits = false;
+    if ((rc = index_kept_voxels(b, false, fits)) != CS_OK) return bail(rc);
+    if (!fits) drop_pass2(b);
+    if ((rc = upload_pass2_tiles(b)) != CS_OK) return bail(rc);
   }
   rc = cs_batch_reset(b);
   if (rc != CS_OK) return bail(rc);
@@ -2133,7 +2177,10 @@ int cs_batch_set_gating(cs_batch* b, uint32_t mode, const cs_mlp* net)
     if (b->p2_ok && !b->near_ok) {
       HIP_TRY(hipSetDevice(b->device));
       HIP_TRY(hipStreamSynchronize(b->stream));
-      const int rc = index_kept_voxels(b, true);
+      /* without room for the wider index near_ok stays false, and the
+       * closure gates around one-step passes */
+      bool fits = false;
+      const int rc = index_kept_voxels(b, true, fits);
       if (rc != CS_OK) return rc;
     }
     b->d_net = (const MlpDev*)cs_internal_mlp_device(net);

@@ -1,0 +1,105 @@
+"""The library's host code on a stand-in for the HIP runtime
+(device_stub.cpp): no GPU, kernels do nothing, allocations fail on demand,
+and every launch is checked for pointers to memory that is not there.
+
+Each case runs in a process of its own, where the stand-in is loaded before
+the library.
+"""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PKG = os.path.join(os.path.dirname(HERE), "hpc-ca-phospattern_amd")
+
+
+class Stub:
+    """The stand-in's own entry points."""
+
+    def __init__(self, path):
+        self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        self.lib.stub_fail_alloc_in.argtypes = [C.c_long]
+        for name in ("stub_allocs", "stub_live_bytes", "stub_bad", "stub_launches"):
+            getattr(self.lib, name).restype = C.c_long
+        self.lib.stub_launches.argtypes = [C.c_char_p]
+        self.lib.stub_bad_at.argtypes = [C.c_long]
+        self.lib.stub_bad_at.restype = C.c_char_p
+
+    def launches(self, part):
+        return self.lib.stub_launches(part.encode())
+
+    def sound(self):
+        """No launch, copy or free touched memory that is not there, and no
+        error waits for a later call to trip over."""
+        bad = [self.lib.stub_bad_at(k).decode() for k in range(self.lib.stub_bad())]
+        assert not bad, bad[:5]
+        assert self.lib.stub_pending_error() == 0
+
+    def failing(self, k, call):
+        """`call` with its k-th allocation failing; whether it made that many."""
+        before = self.lib.stub_allocs()
+        self.lib.stub_fail_alloc_in(k)
+        try:
+            call()
+        finally:
+            self.lib.stub_fail_alloc_in(-1)
+        return self.lib.stub_allocs() - before > k
+
+
+def _ensemble(count=3, n=(20, 18, 14), **kw):
+    import csparks as cs
+    import dyad
+    ds = [dyad.small_dyad(n=n, seed=3 + k) for k in range(count)]
+    return cs.Ensemble([(d.geometry, d.model, cs.Options(seed=1 + k, open={"ryr": [0]}, **kw))
+                        for k, d in enumerate(ds)], instances=list(range(count)))
+
+
+def _net():
+    import closure
+    return closure.load(os.path.join(PKG, "closure_params.npz"))[0]
+
+
+def ensemble_closure_without_memory(stub):
+    """Closure gating needs a wider index of kept voxels than the ensemble
+    was made with.  Without memory for it the call still succeeds, and steps
+    (graphs among them) run on what there is; with it, they run in pairs."""
+    net, k, more = _net(), 0, True
+    while more:
+        ens = _ensemble()
+        ens.set_graph(True)
+        ens.step(ens.period)
+        more = stub.failing(k, lambda: ens.set_gating(ens.GATE_CLOSURE, net))
+        stub.sound()
+        pairs = stub.launches("k_pass2")
+        ens.step(ens.period + 3)
+        stub.sound()
+        assert (stub.launches("k_pass2") > pairs) == (not more), f"allocation {k}"
+        ens.set_gating(ens.GATE_OWN)
+        pairs = stub.launches("k_pass2")
+        ens.step(ens.period + 3)
+        stub.sound()
+        assert stub.launches("k_pass2") > pairs
+        ens.close()
+        k += 1
+    assert k > 1
+
+
+def _run(tmp_path, name):
+    stub = str(tmp_path / "device_stub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
+                    os.path.join(PKG, "csrc"), os.path.join(HERE, "device_stub.cpp"), "-o", stub], check=True)
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, name], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_ensemble_closure_without_memory(tmp_path):
+    _run(tmp_path, "ensemble_closure_without_memory")
+
+
+if __name__ == "__main__":
+    sys.path[:0] = [PKG]
+    stand_in = Stub(sys.argv[1])
+    globals()[sys.argv[2]](stand_in)
+    stand_in.sound()
