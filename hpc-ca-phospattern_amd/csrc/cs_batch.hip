@@ -782,6 +782,7 @@ struct cs_batch {
    * ones, the kept voxels (pair voxels, and with near_ok those around the
    * channels) by column, and what the passes keep there */
   bool p2_ok = false, p2_on = false, near_ok = false;
+  bool p2_tiled = false;                   /* d_p2_tiles is the active ones'  */
   std::vector<P2Split> p2_split;
   P2Geo* d_p2_geo = nullptr;
   uint32_t* d_p2_words = nullptr;
@@ -960,10 +961,14 @@ int setup_pass2(cs_batch* b)
 }
 
 /* The tiles of the active realisations: planes per block as p2_zparts finds
- * for a grid as deep as the deepest and all their tiles. */
+ * for a grid as deep as the deepest and all their tiles.  Fewer realisations
+ * may take more tiles (thinner blocks); without memory for them steps run
+ * one by one until the next choice of active ones finds room. */
 int upload_pass2_tiles(cs_batch* b)
 {
   if (!b->p2_ok) return CS_OK;
+  b->p2_tiled = false;
+  b->n_p2_tiles = 0;
   uint64_t cols = 0;
   uint32_t deep = 1;
   for (uint32_t i = 0; i < b->count; i++)
@@ -982,10 +987,13 @@ int upload_pass2_tiles(cs_batch* b)
     if (!p2_fits(t, (uint32_t)b->geo[t.inst].nx, (uint32_t)b->geo[t.inst].ny, b->esize, P2_HALF))
       return set_err(CS_EDEVICE, "a tile of %u x %u columns does not fit its block", t.w, t.h);
   if (tiles.size() > b->cap_p2_tiles) {
-    if (b->d_p2_tiles) HIP_TRY(hipFree(b->d_p2_tiles));
-    b->d_p2_tiles = nullptr;
-    b->cap_p2_tiles = 0;
-    HIP_TRY(hipMalloc(&b->d_p2_tiles, sizeof(P2Tile) * tiles.size()));
+    P2Tile* fresh = nullptr;
+    if (hipMalloc(&fresh, sizeof(P2Tile) * tiles.size()) != hipSuccess) {
+      (void)hipGetLastError();
+      return CS_OK;
+    }
+    if (b->d_p2_tiles) (void)hipFree(b->d_p2_tiles);
+    b->d_p2_tiles = fresh;
     b->cap_p2_tiles = (uint32_t)tiles.size();
   }
   if (!tiles.empty()) {
@@ -993,6 +1001,7 @@ int upload_pass2_tiles(cs_batch* b)
                            b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
   }
+  b->p2_tiled = true;
   b->n_p2_tiles = (uint32_t)tiles.size();
   b->p2_xcd = 0;
   for (int G = 16; G >= 2; G /= 2)
@@ -1260,9 +1269,12 @@ int launch_bpass2(cs_batch* b, const void* uin, void* uout, uint64_t ti)
   return CS_OK;
 }
 
-/* Whether steps run in pairs: two-step passes are on and, when a closure
- * gates, the passes keep what it reads. */
-bool b_pairs(const cs_batch* b) { return b->p2_on && (b->gating != CS_GATE_CLOSURE || b->near_ok); }
+/* Whether steps run in pairs: two-step passes are on, with the tiles of the
+ * active realisations, and keep what a gating closure reads. */
+bool b_pairs(const cs_batch* b)
+{
+  return b->p2_on && b->p2_tiled && (b->gating != CS_GATE_CLOSURE || b->near_ok);
+}
 
 /* Steps [first, first + n) in pairs (n even): per pair the pass and the
  * bridge (the second step's gating and fluxes, then the next pair's first

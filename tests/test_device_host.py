@@ -85,6 +85,31 @@ def ensemble_closure_without_memory(stub):
     assert k > 1
 
 
+def ensemble_retiring_without_memory(stub):
+    """Fewer active members may take more tiles than the list made for all
+    of them holds: 260 members of one column tile each run 12 planes to a
+    block, 250 of them 6 planes in twice as many blocks (at most 512 are
+    resident).  Without memory for the longer list, steps run one by one,
+    and in pairs again once a choice of members finds room."""
+    def keep(ens, n):
+        ens.set_active([k < n for k in range(ens.count)])
+
+    ens = _ensemble(count=260, n=(9, 9, 12))
+    ens.set_graph(True)
+    ens.step(ens.period)
+    assert stub.failing(0, lambda: keep(ens, 250)), "the case needs a longer list"
+    stub.sound()
+    pairs = stub.launches("k_pass2")
+    ens.step(ens.period + 5)
+    stub.sound()
+    assert stub.launches("k_pass2") == pairs
+    keep(ens, 249)
+    ens.step(ens.period + 5)
+    stub.sound()
+    assert stub.launches("k_pass2") > pairs
+    ens.close()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -96,6 +121,10 @@ def _run(tmp_path, name):
 
 def test_ensemble_closure_without_memory(tmp_path):
     _run(tmp_path, "ensemble_closure_without_memory")
+
+
+def test_ensemble_retiring_without_memory(tmp_path):
+    _run(tmp_path, "ensemble_retiring_without_memory")
 
 
 if __name__ == "__main__":
