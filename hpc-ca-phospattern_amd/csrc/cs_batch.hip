@@ -891,12 +891,19 @@ int upload_tiles(cs_batch* b)
 {
   std::vector<BatchTile> tiles;
   make_tiles(b, BX * b->launch.rows, b->launch.zchunk, tiles);
-  if (b->d_tiles) HIP_TRY(hipFree(b->d_tiles));
-  b->d_tiles = nullptr;
-  HIP_TRY(hipMalloc(&b->d_tiles, sizeof(BatchTile) * std::max<size_t>(tiles.size(), 1)));
-  HIP_TRY(hipMemcpyAsync(b->d_tiles, tiles.data(), sizeof(BatchTile) * tiles.size(), hipMemcpyHostToDevice,
-                         b->stream));
-  HIP_TRY(hipStreamSynchronize(b->stream));
+  BatchTile* fresh = nullptr;   /* the old list stays until the new one is there */
+  if (hipMalloc(&fresh, sizeof(BatchTile) * std::max<size_t>(tiles.size(), 1)) != hipSuccess) {
+    (void)hipGetLastError();
+    return set_err(CS_ENOMEM, "device allocation of %zu tiles failed", tiles.size());
+  }
+  if (hipMemcpyAsync(fresh, tiles.data(), sizeof(BatchTile) * tiles.size(), hipMemcpyHostToDevice, b->stream) !=
+          hipSuccess ||
+      hipStreamSynchronize(b->stream) != hipSuccess) {
+    (void)hipFree(fresh);
+    return set_err(CS_EDEVICE, "upload of tiles failed");
+  }
+  if (b->d_tiles) (void)hipFree(b->d_tiles);
+  b->d_tiles = fresh;
   b->ntiles = (uint32_t)tiles.size();
   /* persistent grid: as many blocks as stay resident, in whole rounds of
    * the eight XCDs, never more than there are tiles */
@@ -2109,11 +2116,15 @@ int cs_batch_set_launch(cs_batch* b, const cs_batch_launch* in)
   if (in->persistent > 1) return set_err(CS_EINVAL, "persistent must be 0 or 1");
   HIP_TRY(hipSetDevice(b->device));
   HIP_TRY(hipStreamSynchronize(b->stream));
+  const cs_batch_launch old = b->launch;
   b->launch = *in;
   b->launch.nontemporal = in->nontemporal ? 1 : 0;
   drop_graphs(b);
   int rc = b->esize == 8 ? upload_tiles<double>(b) : upload_tiles<float>(b);
-  if (rc != CS_OK) return rc;
+  if (rc != CS_OK) {
+    b->launch = old;
+    return rc;
+  }
   /* keep retired realisations out */
   const std::vector<uint8_t> act = b->h_active;
   return cs_batch_set_active(b, act.data());

@@ -110,6 +110,25 @@ def ensemble_retiring_without_memory(stub):
     ens.close()
 
 
+def ensemble_launch_without_memory(stub):
+    """A launch shape whose tiles find no memory is refused; the one before
+    stays, with its tiles (single steps run on them), also with members
+    retired."""
+    import pytest
+    ens = _ensemble(n=(64, 63, 24))
+    ens.set_active([True, False, True])
+    shape = ens.launch()
+    with pytest.raises(RuntimeError):
+        stub.failing(0, lambda: ens.set_launch(rows=1, zchunk=2))
+    assert ens.launch() == shape
+    stub.sound()
+    ens.step(1)
+    stub.sound()
+    ens.set_launch(rows=1, zchunk=2)
+    ens.step(1)
+    ens.close()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -125,6 +144,10 @@ def test_ensemble_closure_without_memory(tmp_path):
 
 def test_ensemble_retiring_without_memory(tmp_path):
     _run(tmp_path, "ensemble_retiring_without_memory")
+
+
+def test_ensemble_launch_without_memory(tmp_path):
+    _run(tmp_path, "ensemble_launch_without_memory")
 
 
 if __name__ == "__main__":
