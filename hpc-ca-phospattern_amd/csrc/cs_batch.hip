@@ -1287,12 +1287,14 @@ bool b_pairs(const cs_batch* b)
  * bridge (the second step's gating and fluxes, then the next pair's first
  * gating and flux sums).  With a closure the tail and the head are
  * launches of their own, each after the predictions from the state it
- * gates on (with the flux network every state is predicted from, since
- * its fluxes read the ratios).  gate_idx counts gating steps; ev and d_ti
- * as in b_run. */
+ * gates on (with the flux network every state is predicted from once, since
+ * its fluxes read the ratios; the call's last state too, for
+ * cs_batch_flux_predictions, unless a single step follows (more), which
+ * predicts from it itself).  gate_idx counts gating steps; ev and d_ti as
+ * in b_run. */
 template <typename T>
-int b_run_pairs(cs_batch* b, uint64_t first, uint64_t n, const double* d_uni, hipEvent_t* ev, const uint64_t* d_ti,
-                uint64_t& gate_idx)
+int b_run_pairs(cs_batch* b, uint64_t first, uint64_t n, bool more, const double* d_uni, hipEvent_t* ev,
+                const uint64_t* d_ti, uint64_t& gate_idx)
 {
   const bool closure = b->gating == CS_GATE_CLOSURE, fclosure = closure && b->d_fnet;
   auto part = [&](uint64_t ti) {
@@ -1319,7 +1321,7 @@ int b_run_pairs(cs_batch* b, uint64_t first, uint64_t n, const double* d_uni, hi
       if (tail.gate || fclosure) launch_predict<T>(b, b->d_p2_l1, b->d_near);
       launch(tail, none, u);
     }
-    if (head.gate || fclosure) launch_predict<T>(b, u);
+    if (head.on ? head.gate || fclosure : fclosure && !more) launch_predict<T>(b, u);
     if (head.on) launch(none, head, u);
   };
   bridge(Bridge2Step{}, part(first), b->d_u[b->cur]);
@@ -1354,7 +1356,7 @@ int b_run(cs_batch* b, uint64_t first, uint64_t n, const double* d_uni, hipEvent
   const uint64_t paired = b_pairs(b) ? n / 2 * 2 : 0;
   if (npasses) *npasses = paired / 2 + (n - paired);
   if (paired) {
-    const int rc = b_run_pairs<T>(b, first, paired, d_uni, ev, d_ti, gate_idx);
+    const int rc = b_run_pairs<T>(b, first, paired, n > paired, d_uni, ev, d_ti, gate_idx);
     if (rc != CS_OK) return rc;
     first += paired;
     n -= paired;

@@ -129,6 +129,22 @@ def ensemble_launch_without_memory(stub):
     ens.close()
 
 
+def flux_network_predicts_each_state_once(stub):
+    """With the flux network a call of n steps predicts from the state it
+    starts on and from the one after every step (n + 1 times; the range
+    monitor counts each), in pairs and with a last single step alike."""
+    import closure
+    fnet = closure.load_flux(os.path.join(PKG, "closure_params.npz"))[0]
+    net, ens = _net(), _ensemble()
+    ens.set_gating(ens.GATE_CLOSURE, net)
+    ens.set_flux_closure(fnet)
+    for n in (1, 2, 3, 20, 21):
+        before = stub.launches("k_closure_predict")
+        ens.step(n)
+        assert stub.launches("k_closure_predict") - before == n + 1, n
+    ens.close()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -148,6 +164,10 @@ def test_ensemble_retiring_without_memory(tmp_path):
 
 def test_ensemble_launch_without_memory(tmp_path):
     _run(tmp_path, "ensemble_launch_without_memory")
+
+
+def test_flux_network_predicts_each_state_once(tmp_path):
+    _run(tmp_path, "flux_network_predicts_each_state_once")
 
 
 if __name__ == "__main__":
