@@ -777,7 +777,8 @@ struct cs_batch {
   uint32_t rfast = 0, rbound = 0;
   uint32_t fsm = 0;
   /* two-step passes: whether the model and every grid admit them (p2_ok),
-   * whether they run (autotune may find one-step passes faster), a record
+   * whether they run (a launch shape may ask for one-step passes, autotune
+   * may find those faster), a record
    * and a split per realisation, the tiles of the active
    * ones, the kept voxels (pair voxels, and with near_ok those around the
    * channels) by column, and what the passes keep there */
@@ -1505,6 +1506,23 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
   return CS_OK;
 }
 
+/* The shape of one-step passes. */
+int set_shape(cs_batch* b, const cs_batch_launch& shape)
+{
+  const cs_batch_launch old = b->launch;
+  b->launch = shape;
+  b->launch.nontemporal = shape.nontemporal ? 1 : 0;
+  drop_graphs(b);
+  const int rc = b->esize == 8 ? upload_tiles<double>(b) : upload_tiles<float>(b);
+  if (rc != CS_OK) {
+    b->launch = old;
+    return rc;
+  }
+  /* keep retired realisations out */
+  const std::vector<uint8_t> act = b->h_active;
+  return cs_batch_set_active(b, act.data());
+}
+
 }  // namespace
 /* ------------------------------------------------------------- C ABI */
 
@@ -2106,6 +2124,7 @@ int cs_batch_get_launch(const cs_batch* b, cs_batch_launch* out)
 {
   if (!b || !out) return set_err(CS_EINVAL, "NULL argument");
   *out = b->launch;
+  if (b->p2_on) out->persistent = 2;
   return CS_OK;
 }
 
@@ -2115,21 +2134,16 @@ int cs_batch_set_launch(cs_batch* b, const cs_batch_launch* in)
   if (in->rows < 1 || in->rows > 8) return set_err(CS_EINVAL, "rows must be 1..8");
   if (in->zchunk < 1) return set_err(CS_EINVAL, "zchunk must be >= 1");
   if (in->prefetch < 1 || in->prefetch > 2) return set_err(CS_EINVAL, "prefetch must be 1 or 2");
-  if (in->persistent > 1) return set_err(CS_EINVAL, "persistent must be 0 or 1");
+  if (in->persistent > (b->p2_ok ? 2u : 1u))
+    return set_err(CS_EINVAL, b->p2_ok ? "persistent must be 0, 1 or 2"
+                                       : "persistent must be 0 or 1 (two-step passes unavailable)");
   HIP_TRY(hipSetDevice(b->device));
   HIP_TRY(hipStreamSynchronize(b->stream));
-  const cs_batch_launch old = b->launch;
-  b->launch = *in;
-  b->launch.nontemporal = in->nontemporal ? 1 : 0;
-  drop_graphs(b);
-  int rc = b->esize == 8 ? upload_tiles<double>(b) : upload_tiles<float>(b);
-  if (rc != CS_OK) {
-    b->launch = old;
-    return rc;
-  }
-  /* keep retired realisations out */
-  const std::vector<uint8_t> act = b->h_active;
-  return cs_batch_set_active(b, act.data());
+  cs_batch_launch shape = *in;
+  if (in->persistent == 2) shape.persistent = b->launch.persistent;
+  const int rc = set_shape(b, shape);
+  if (rc == CS_OK) b->p2_on = in->persistent == 2;
+  return rc;
 }
 
 int cs_batch_step_period(const cs_batch* b, uint64_t* period)
@@ -2375,7 +2389,7 @@ int cs_batch_autotune(cs_batch* b, uint64_t first, uint32_t reps, cs_batch_launc
   cs_batch_launch wcfg = keep;
   int rc = CS_OK;
   for (const cs_batch_launch& L : cand) {
-    if ((rc = cs_batch_set_launch(b, &L)) != CS_OK) break;
+    if ((rc = set_shape(b, L)) != CS_OK) break;
     double tot = 0.0;
     uint32_t wsum = 0;
     for (const auto& kv : pattern) {
@@ -2403,10 +2417,10 @@ int cs_batch_autotune(cs_batch* b, uint64_t first, uint32_t reps, cs_batch_launc
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc != CS_OK) {
-    cs_batch_set_launch(b, &keep);
+    (void)set_shape(b, keep);
     return rc;
   }
-  rc = cs_batch_set_launch(b, &wcfg);
+  rc = set_shape(b, wcfg);
   if (rc != CS_OK) return rc;
   /* two-step passes over the pairs of two periods, each counting as two
    * steps: they run unless the one-step shape found above beats them */
@@ -2444,7 +2458,7 @@ int cs_batch_autotune(cs_batch* b, uint64_t first, uint32_t reps, cs_batch_launc
     b->p2_on = per_step <= win;
     if (b->p2_on) win = per_step;
   }
-  if (best) *best = wcfg;
+  if (best) cs_batch_get_launch(b, best);
   if (best_ms) *best_ms = win;
   return CS_OK;
 }

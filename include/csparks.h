@@ -371,18 +371,19 @@ int cs_batch_monitor(cs_batch* b, uint32_t* flags);
  * persistent = 1 runs one persistent block per resident slot, taking tiles
  * from eight per-XCD work queues; 0 launches one block per tile, the tiles
  * numbered in groups per XCD, and leaves the scheduling to the hardware
- * (same results, bit for bit).  Ensembles of the five-slot species layout
- * run their steps in pairs, as two-step passes of their own shape (see
- * cs_launch_config); there one-step passes take only a last odd step.  No
- * reference counterpart. */
+ * (same results, bit for bit).  persistent = 2, for ensembles of the
+ * five-slot species layout (see cs_launch_config) and their default, runs
+ * steps in pairs, as two-step passes of their own shape (same results to
+ * rounding); a last odd step takes the one-step pass.  No reference
+ * counterpart. */
 typedef struct cs_batch_launch {
   uint32_t rows, zchunk, prefetch, nontemporal, persistent;
 } cs_batch_launch;
 int cs_batch_get_launch(const cs_batch* b, cs_batch_launch* cfg);
 int cs_batch_set_launch(cs_batch* b, const cs_batch_launch* cfg);
 /* Time every candidate shape on one period of the step pattern from
- * first_time_ind (state unchanged) and keep the fastest; two-step passes
- * stay off if the best one-step shape beats them.  best_ms is the mean
+ * first_time_ind (state unchanged) and keep the fastest: persistent = 2
+ * with the best one-step shape, or that shape alone if it is faster.  best_ms is the mean
  * kernel time per step of the form that runs. */
 int cs_batch_autotune(cs_batch* b, uint64_t first_time_ind, uint32_t reps, cs_batch_launch* best,
                       double* best_ms);

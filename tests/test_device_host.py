@@ -6,9 +6,13 @@ Each case runs in a process of its own, where the stand-in is loaded before
 the library.
 """
 import ctypes as C
+import dataclasses
 import os
 import subprocess
 import sys
+
+import numpy as np
+import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.join(os.path.dirname(HERE), "hpc-ca-phospattern_amd")
@@ -114,7 +118,6 @@ def ensemble_launch_without_memory(stub):
     """A launch shape whose tiles find no memory is refused; the one before
     stays, with its tiles (single steps run on them), also with members
     retired."""
-    import pytest
     ens = _ensemble(n=(64, 63, 24))
     ens.set_active([True, False, True])
     shape = ens.launch()
@@ -145,6 +148,50 @@ def flux_network_predicts_each_state_once(stub):
     ens.close()
 
 
+def ensemble_launch_names_the_form(stub):
+    """persistent says which passes run: 2 (the default of five-slot
+    models) pairs of steps, 0 and 1 one-step passes of the given shape.
+    What is read can be written back; the shape's other keys leave the form;
+    autotune's answer, given to set_launch, keeps what it chose."""
+    import csparks as cs
+    import dyad
+    forms = ("k_batch_tiles", "k_batch_stencil", "k_pass2")
+
+    def passes(ens, n=4):
+        before = [stub.launches(f) for f in forms]
+        ens.step(n)
+        return [stub.launches(f) - k for f, k in zip(forms, before)]
+
+    ens = _ensemble()
+    assert ens.launch()["persistent"] == 2 and passes(ens) == [0, 0, 2]
+    ens.set_launch(**ens.launch())
+    ens.set_launch(rows=8, zchunk=8)
+    assert ens.launch()["persistent"] == 2 and passes(ens) == [0, 0, 2]
+    for form in (0, 1):
+        ens.set_launch(persistent=form)
+        assert ens.launch()["persistent"] == form and passes(ens) == [4 * (form == k) for k in range(3)]
+    ens.set_launch(persistent=2)
+    assert passes(ens, 5) == [0, 1, 2]   # the odd step as it ran before
+    with pytest.raises(RuntimeError):
+        ens.set_launch(persistent=3)
+    best, _ = ens.autotune(1)
+    want = passes(ens)
+    ens.set_launch(**best)
+    assert passes(ens) == want and ens.launch() == best
+    ens.close()
+
+    d = dyad.small_dyad()   # a slab of one column in x cannot pair
+    geom = cs.Geometry(voxels=np.ascontiguousarray(d.geometry.voxels[:1]), h=d.geometry.h,
+                       domain_names=list(d.geometry.domain_names),
+                       domain_connections=d.geometry.domain_connections, boundaries=[])
+    one = cs.Ensemble([(geom, dataclasses.replace(d.model, ryr=None, p_ryr=None), cs.Options(seed=1))])
+    assert one.launch()["persistent"] == 0
+    with pytest.raises(RuntimeError):
+        one.set_launch(persistent=2)
+    assert sum(passes(one)) == 4
+    one.close()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -168,6 +215,10 @@ def test_ensemble_launch_without_memory(tmp_path):
 
 def test_flux_network_predicts_each_state_once(tmp_path):
     _run(tmp_path, "flux_network_predicts_each_state_once")
+
+
+def test_ensemble_launch_names_the_form(tmp_path):
+    _run(tmp_path, "ensemble_launch_names_the_form")
 
 
 if __name__ == "__main__":
