@@ -854,7 +854,13 @@ class Simulation:
         return cfg.as_dict()
 
     def set_launch_config(self, **kw):
-        cfg = CLaunchConfig(**{**self.launch_config(), **kw})
+        """Change keys of the launch shape.  `fuse` given alone decides the
+        form of the passes: fuse_fixed = 2 (pairs whatever fuse says)
+        becomes 1."""
+        cfg = {**self.launch_config(), **kw}
+        if "fuse" in kw and "fuse_fixed" not in kw:
+            cfg["fuse_fixed"] = min(cfg["fuse_fixed"], 1)
+        cfg = CLaunchConfig(**cfg)
         _check(device_lib().cs_set_launch_config(self.ctx, C.byref(cfg)), "cs_set_launch_config")
 
     def autotune(self, reps: int = 1):

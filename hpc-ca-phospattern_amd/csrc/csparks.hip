@@ -87,7 +87,8 @@ struct LaunchCfg {
   int fuse;      /* 1: pairs of eligible steps run as one k_step2 pass     */
   int fz;        /* planes per block of k_step2                             */
   int fx;        /* xcd_tile map of k_step2's blocks                        */
-  int ff;        /* 1: k_pass2 (compiled masks) where the model fits it */
+  int ff;        /* 1: k_pass2 (compiled masks) where the model fits it;
+                    2: and pairs run so whatever fuse is                    */
 };
 
 template <typename T, int NS, int PF, bool NT>
@@ -1464,7 +1465,6 @@ struct cs_context {
   /* k_pass2: whether the model admits it, the domain's record, its split
    * into column tiles, and a tile list per number of planes per block */
   bool p2_ok = false, p2_whole = false;
-  bool auto_form = true;             /* no launch shape was set or tuned yet  */
   P2Split p2_split{0, 0};
   P2Geo* d_p2_geo = nullptr;
   uint32_t* d_p2_words = nullptr;
@@ -1788,7 +1788,7 @@ F2Step step_info(const cs_context* c, uint64_t ti, uint64_t uni_base)
  * both steps, so its neighbours are at hand at both levels. */
 bool can_fuse(const cs_context* c, const LaunchCfg& L, uint64_t ti)
 {
-  if (!c->f2_ok || !(L.fuse || (c->auto_form && c->p2_ok))) return false;
+  if (!c->f2_ok || !(L.fuse || (L.ff == 2 && c->p2_ok))) return false;
   return (c->fsm & ~diffusing(c, ti)) == 0 && (c->fsm & ~diffusing(c, ti + 1)) == 0;
 }
 
@@ -2385,8 +2385,8 @@ int cs_create(const cs_problem* p, cs_context** out)
   rc = setup_pass2(c);
   if (rc != CS_OK) return bail(rc);
   c->launch = default_launch(g, c->esize, cus);
-  /* Until a shape is set or tuned (auto_form), every pair of steps that
-   * k_pass2 takes runs so: it beat one-step passes on every grid measured,
+  /* Every pair of steps that k_pass2 takes runs so (launch.ff = 2 where
+   * launch.fuse is 0): it beat one-step passes on every grid measured,
    * per step with gating and fluxes 12 against 22 us on 64x64x25 (FP64), 19
    * against 35 on 84^3 (FP64), 16 against 27 on 131x97x53 (FP32), 335
    * against 560 on 400x400x200 (FP64), 174 against 260 on that in FP32.
@@ -2401,6 +2401,7 @@ int cs_create(const cs_problem* p, cs_context** out)
   const long fused_blocks = fused_tiles * ((g.nz + c->launch.fz - 1) / std::max(c->launch.fz, 1));
   c->launch.fuse = (c->f2_ok && c->esize == 4 && 2 * fused_blocks >= cus) ? 1 : 0;
   if (c->p2_ok) {
+    if (!c->launch.fuse) c->launch.ff = 2;
     /* k_pass2's own planes per block and tile order */
     const long cols = (long)c->p2_split.kx * c->p2_split.ky;
     const uint32_t parts = p2_zparts((uint64_t)cols, (uint32_t)g.nz, c->p2_whole ? cus : 2 * cus,
@@ -2716,7 +2717,8 @@ int cs_set_launch_config(cs_context* c, const cs_launch_config* in)
   if (in->fuse > 1) return set_err(CS_EINVAL, "fuse must be 0 or 1");
   if (in->fuse && !c->f2_ok) return set_err(CS_EINVAL, "fused passes unavailable: %s", c->f2_why.c_str());
   if (in->fuse_xcd > 64) return set_err(CS_EINVAL, "fuse_xcd is 0, 1 or a group size up to 64");
-  if (in->fuse_fixed > 1) return set_err(CS_EINVAL, "fuse_fixed must be 0 or 1");
+  if (in->fuse_fixed > 2) return set_err(CS_EINVAL, "fuse_fixed must be 0, 1 or 2");
+  if (in->fuse_fixed == 2 && !c->p2_ok) return set_err(CS_EINVAL, "compiled two-step passes unavailable");
   const int fzmax = max_fused_zchunk(c->geo, c->esize);
   if (in->fuse_zchunk < 1) return set_err(CS_EINVAL, "fuse_zchunk must be >= 1");
   if (fzmax >= 1 && (int)std::min<uint32_t>(in->fuse_zchunk, (uint32_t)c->geo.nz) > fzmax)
@@ -2726,7 +2728,6 @@ int cs_set_launch_config(cs_context* c, const cs_launch_config* in)
   L.fx = (int)in->fuse_xcd;
   L.ff = (int)in->fuse_fixed;
   c->launch = L;
-  c->auto_form = false;
   return CS_OK;
 }
 
@@ -2818,7 +2819,7 @@ int cs_autotune(cs_context* c, uint64_t first_time_ind, uint32_t reps, cs_launch
   winner.fuse = 0;
   winner.fz = c->launch.fz;
   winner.fx = c->launch.fx;
-  winner.ff = c->launch.ff;
+  winner.ff = std::min(c->launch.ff, 1);   /* fuse says which form won */
   /* fused two-step passes: the pairs (ti, ti+1) of two periods that may
    * fuse, grouped by their patterns, without gating (so the channel
    * states and recruitment flags stay as they are); a pass counts as two
@@ -2896,7 +2897,6 @@ done:
   if (rc != CS_OK) return rc;
   HIP_TRY(hipGetLastError());
   c->launch = winner;
-  c->auto_form = false;
   if (best) cs_get_launch_config(c, best);
   if (best_ms) *best_ms = wms;
   return CS_OK;

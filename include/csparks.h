@@ -228,13 +228,14 @@ int cs_fused_available(const cs_context* ctx, char* why, size_t why_len);
  * its tile order (as xcd_remap).  The other steps, and every step with
  * fuse = 0, run one at a time.  cs_create sets fuse = 1 for FP32 fields
  * when the problem admits fused passes and their launch has at least
- * half as many blocks as the device has CUs, else 0; until
- * cs_set_launch_config or cs_autotune chooses a shape, models of the
- * reference's five-slot species layout (Ca, dye, CMDN-CSQN, ATP, TRPN; Ca
- * and ATP diffusing on every step, TRPN on none) run two-step passes
- * whatever fuse says, since there they are the faster form at every size
- * and in both precisions.  fuse_fixed = 1 (the default) runs that layout's
- * passes with kernels compiled for each pair of step masks (k_pass2); 0
+ * half as many blocks as the device has CUs, else 0.  fuse_fixed = 1 runs
+ * the two-step passes of the reference's five-slot species layout (Ca, dye,
+ * CMDN-CSQN, ATP, TRPN; Ca and ATP diffusing on every step, TRPN on none)
+ * with kernels compiled for each pair of step masks (k_pass2); 2 does so
+ * and runs pairs whatever fuse says.  cs_create sets 2 for that layout where
+ * it sets fuse = 0, since there pairs are the faster form at every size and
+ * in both precisions (so a config that is read can be written back; one-step
+ * passes take fuse = 0 and fuse_fixed below 2), else 1.  0
  * runs every pass with the masks read at run time (k_step2; same results
  * to rounding).  No reference counterpart: the reference's
  * OpenMP/AVX-512 loop has no launch shape (kernel_generic.cpp:561-600). */

@@ -192,6 +192,61 @@ def ensemble_launch_names_the_form(stub):
     one.close()
 
 
+def launch_config_names_the_form(stub):
+    """Five-slot models run pairs by default in both precisions and at every
+    size; the launch config says so (fuse = 1, or fuse_fixed = 2), can be
+    written back, and keeps the form when another key changes.  fuse = 0
+    asks for one-step passes, and autotune's answer for what it chose."""
+    import csparks as cs
+    import dyad
+
+    def pairs(sim, n=4):
+        before = [stub.launches(k) for k in ("k_pass2", "k_stencil")]
+        sim.step(n)
+        two, one = (stub.launches(k) - b for k, b in zip(("k_pass2", "k_stencil"), before))
+        assert 2 * two + one == n
+        return two
+
+    def says(cfg):
+        return cfg["fuse"] == 1 or cfg["fuse_fixed"] == 2
+
+    for n, precision in (((20, 18, 14), "f64"), ((20, 18, 14), "f32"), ((300, 300, 40), "f32")):
+        d = dyad.small_dyad(n=n)
+        sim = cs.Simulation(d.geometry, d.model, cs.Options(seed=1, open={"ryr": [0]}, precision=precision))
+        assert pairs(sim) == 2 and says(sim.launch_config())
+        sim.set_launch_config(**sim.launch_config())
+        assert pairs(sim) == 2
+        sim.set_launch_config(fuse_xcd=4)
+        sim.set_launch_config(rows=8, zchunk=4)
+        assert pairs(sim) == 2 and says(sim.launch_config())
+        sim.set_launch_config(fuse=0)
+        assert pairs(sim) == 0 and not says(sim.launch_config())
+        sim.set_launch_config(rows=4)
+        assert pairs(sim) == 0
+        sim.set_launch_config(fuse=1)
+        assert pairs(sim) == 2
+        sim.set_launch_config(fuse=0, fuse_fixed=2)
+        assert pairs(sim) == 2
+        best, _ = sim.autotune(1)
+        want = pairs(sim)
+        assert (want == 2) == says(best)
+        sim.set_launch_config(**best)
+        assert pairs(sim) == want
+        with pytest.raises(RuntimeError):
+            sim.set_launch_config(fuse_fixed=3)
+        sim.close()
+
+    d = dyad.small_dyad()   # a slab of one column in x has no compiled pass
+    geom = cs.Geometry(voxels=np.ascontiguousarray(d.geometry.voxels[:1]), h=d.geometry.h,
+                       domain_names=list(d.geometry.domain_names),
+                       domain_connections=d.geometry.domain_connections, boundaries=[])
+    one = cs.Simulation(geom, dataclasses.replace(d.model, ryr=None, p_ryr=None), cs.Options(seed=1))
+    assert not says(one.launch_config()) and pairs(one) == 0
+    with pytest.raises(RuntimeError):
+        one.set_launch_config(fuse_fixed=2)
+    one.close()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -219,6 +274,10 @@ def test_flux_network_predicts_each_state_once(tmp_path):
 
 def test_ensemble_launch_names_the_form(tmp_path):
     _run(tmp_path, "ensemble_launch_names_the_form")
+
+
+def test_launch_config_names_the_form(tmp_path):
+    _run(tmp_path, "launch_config_names_the_form")
 
 
 if __name__ == "__main__":
