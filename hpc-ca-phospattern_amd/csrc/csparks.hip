@@ -1792,37 +1792,39 @@ bool can_fuse(const cs_context* c, const LaunchCfg& L, uint64_t ti)
   return (c->fsm & ~diffusing(c, ti)) == 0 && (c->fsm & ~diffusing(c, ti + 1)) == 0;
 }
 
-/* The tile list of blocks of at most fz planes (built once per fz; the
- * launch shapes that cs_autotune tries are few). */
-int pass2_tiles(cs_context* c, int fz, cs_context::TileList& out)
+/* Makes the tile list of blocks of at most fz planes (once per fz; the
+ * launch shapes that cs_autotune tries are few).  The calls that choose a
+ * shape make it, so steps allocate nothing.  CS_ENOMEM, with no error left
+ * pending, when there is no room. */
+int make_pass2_tiles(cs_context* c, int fz)
 {
-  auto it = c->p2_lists.find(fz);
-  if (it == c->p2_lists.end()) {
-    std::vector<P2Tile> tiles;
-    p2_tiles(0, (uint32_t)c->geo.nx, (uint32_t)c->geo.ny, (uint32_t)c->geo.nz, c->p2_split,
-             (uint32_t)((c->geo.nz + fz - 1) / fz), tiles);
-    for (const P2Tile& q : tiles)
-      if (!p2_fits(q, (uint32_t)c->geo.nx, (uint32_t)c->geo.ny, c->esize, c->p2_whole))
-        return set_err(CS_EDEVICE, "a tile of %u x %u columns does not fit its block", q.w, q.h);
-    cs_context::TileList t;
-    t.n = (uint32_t)tiles.size();
-    HIP_TRY(hipMalloc((void**)&t.d, sizeof(P2Tile) * tiles.size()));
-    const hipError_t e = hipMemcpy(t.d, tiles.data(), sizeof(P2Tile) * tiles.size(), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      hipFree(t.d);
-      return set_err(CS_EDEVICE, "upload of tiles failed: %s", hipGetErrorString(e));
-    }
-    it = c->p2_lists.emplace(fz, t).first;
+  if (c->p2_lists.count(fz)) return CS_OK;
+  std::vector<P2Tile> tiles;
+  p2_tiles(0, (uint32_t)c->geo.nx, (uint32_t)c->geo.ny, (uint32_t)c->geo.nz, c->p2_split,
+           (uint32_t)((c->geo.nz + fz - 1) / fz), tiles);
+  for (const P2Tile& q : tiles)
+    if (!p2_fits(q, (uint32_t)c->geo.nx, (uint32_t)c->geo.ny, c->esize, c->p2_whole))
+      return set_err(CS_EDEVICE, "a tile of %u x %u columns does not fit its block", q.w, q.h);
+  cs_context::TileList t;
+  t.n = (uint32_t)tiles.size();
+  if (hipMalloc((void**)&t.d, sizeof(P2Tile) * tiles.size()) != hipSuccess) {
+    (void)hipGetLastError();
+    return set_err(CS_ENOMEM, "device allocation of %u tiles failed", t.n);
   }
-  out = it->second;
+  const hipError_t e = hipMemcpy(t.d, tiles.data(), sizeof(P2Tile) * tiles.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    hipFree(t.d);
+    return set_err(CS_EDEVICE, "upload of tiles failed: %s", hipGetErrorString(e));
+  }
+  c->p2_lists.emplace(fz, t);
   return CS_OK;
 }
 
 int launch_pass2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a, const F2Step& b)
 {
-  cs_context::TileList tl;
-  const int rc = pass2_tiles(c, std::max(1, std::min(L.fz, c->geo.nz)), tl);
-  if (rc != CS_OK) return rc;
+  const auto it = c->p2_lists.find(L.fz);
+  if (it == c->p2_lists.end()) return set_err(CS_EDEVICE, "no tiles for blocks of %d planes", L.fz);
+  const cs_context::TileList& tl = it->second;
   P2Args p{};
   p.u = uin;
   p.un = uout;
@@ -2106,6 +2108,18 @@ int copy_species(cs_context* c, uint32_t s, double* host)
   return CS_OK;
 }
 
+/* No room beside the fields for k_pass2's records: the other passes need
+ * none of them. */
+void drop_pass2(cs_context* c)
+{
+  if (c->d_p2_geo) (void)hipFree(c->d_p2_geo);
+  if (c->d_p2_words) (void)hipFree(c->d_p2_words);
+  c->d_p2_geo = nullptr;
+  c->d_p2_words = nullptr;
+  c->p2_ok = false;
+  (void)hipGetLastError();
+}
+
 /* Whether k_pass2 fits the problem, and its records: the five-slot layout
  * with its substeps (then every step has a compiled mask, and reacts, if at
  * all, in species-major form), fused passes at all, at least two columns
@@ -2121,14 +2135,12 @@ int setup_pass2(cs_context* c)
   c->p2_split = p2_split((uint32_t)g.nx, (uint32_t)g.ny, c->esize, c->p2_whole);
   if (!c->p2_split.kx) return CS_OK;
   const P2Geo rec{0, 0, 0, (uint32_t)g.plane, g.nx, g.ny, g.nz, 0};
-  HIP_TRY(hipMalloc((void**)&c->d_p2_geo, sizeof rec));
-  HIP_TRY(hipMemcpy(c->d_p2_geo, &rec, sizeof rec, hipMemcpyHostToDevice));
-  if (hipMalloc((void**)&c->d_p2_words, sizeof(uint32_t) * g.nv) != hipSuccess) {
-    /* no room beside the fields: the other passes need none */
-    (void)hipGetLastError();
-    c->d_p2_words = nullptr;
+  if (hipMalloc((void**)&c->d_p2_geo, sizeof rec) != hipSuccess ||
+      hipMalloc((void**)&c->d_p2_words, sizeof(uint32_t) * g.nv) != hipSuccess) {
+    drop_pass2(c);
     return CS_OK;
   }
+  HIP_TRY(hipMemcpy(c->d_p2_geo, &rec, sizeof rec, hipMemcpyHostToDevice));
   cs_internal_id_words(c->d_ids, c->d_p2_geo, 1, g.nv, c->d_p2_words, c->stream);
   HIP_TRY(hipGetLastError());
   c->p2_ok = true;
@@ -2401,15 +2413,22 @@ int cs_create(const cs_problem* p, cs_context** out)
   const long fused_blocks = fused_tiles * ((g.nz + c->launch.fz - 1) / std::max(c->launch.fz, 1));
   c->launch.fuse = (c->f2_ok && c->esize == 4 && 2 * fused_blocks >= cus) ? 1 : 0;
   if (c->p2_ok) {
-    if (!c->launch.fuse) c->launch.ff = 2;
     /* k_pass2's own planes per block and tile order */
     const long cols = (long)c->p2_split.kx * c->p2_split.ky;
     const uint32_t parts = p2_zparts((uint64_t)cols, (uint32_t)g.nz, c->p2_whole ? cus : 2 * cus,
                                      (uint32_t)max_fused_zchunk(g, c->esize));
-    c->launch.fz = (g.nz + (int)parts - 1) / (int)parts;
-    c->launch.fx = 0;
-    for (int G = 16; G >= 2; G /= 2)
-      if (cols * parts >= 8L * 3 * G) { c->launch.fx = G; break; }
+    const int fz = (g.nz + (int)parts - 1) / (int)parts;
+    rc = make_pass2_tiles(c, fz);
+    if (rc != CS_OK && rc != CS_ENOMEM) return bail(rc);
+    if (rc == CS_ENOMEM) {
+      drop_pass2(c);
+    } else {
+      if (!c->launch.fuse) c->launch.ff = 2;
+      c->launch.fz = fz;
+      c->launch.fx = 0;
+      for (int G = 16; G >= 2; G /= 2)
+        if (cols * parts >= 8L * 3 * G) { c->launch.fx = G; break; }
+    }
   }
   rc = c->esize == 8 ? fill_init<double>(c) : fill_init<float>(c);
   if (rc != CS_OK) return bail(rc);
@@ -2727,6 +2746,10 @@ int cs_set_launch_config(cs_context* c, const cs_launch_config* in)
   L.fz = (int)std::min<uint32_t>(in->fuse_zchunk, (uint32_t)c->geo.nz);
   L.fx = (int)in->fuse_xcd;
   L.ff = (int)in->fuse_fixed;
+  if (c->p2_ok && L.ff) {
+    const int rc = make_pass2_tiles(c, L.fz);
+    if (rc != CS_OK) return rc;
+  }
   c->launch = L;
   return CS_OK;
 }
@@ -2860,6 +2883,7 @@ int cs_autotune(cs_context* c, uint64_t first_time_ind, uint32_t reps, cs_launch
         L.fuse = 1;
         L.fz = zc;
         L.fx = fx;
+        if (c->p2_ok && L.ff && (rc = make_pass2_tiles(c, L.fz)) != CS_OK) goto done;
         double mean = 0;
         for (const Pair& q : prs) {
           /* the pass and its bridge (tail and the next head, no gating) */

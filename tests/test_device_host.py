@@ -247,6 +247,54 @@ def launch_config_names_the_form(stub):
     one.close()
 
 
+def steps_allocate_nothing(stub):
+    """The calls that choose a launch shape make its tile list: steps need
+    no memory.  A shape whose list finds none is refused and the one before
+    stays; a context that finds no room for what two-step passes need runs
+    without them."""
+    import csparks as cs
+    import dyad
+    d = dyad.small_dyad(n=(64, 63, 24))
+    opts = cs.Options(seed=1, open={"ryr": [0]})
+
+    def steps(sim):
+        before = stub.lib.stub_allocs()
+        two = stub.launches("k_pass2")
+        sim.step(4)
+        stub.sound()
+        assert stub.lib.stub_allocs() == before
+        return stub.launches("k_pass2") - two
+
+    sim = cs.Simulation(d.geometry, d.model, opts)
+    assert steps(sim) == 2
+    shape = sim.launch_config()
+    with pytest.raises(RuntimeError):
+        stub.failing(0, lambda: sim.set_launch_config(fuse_zchunk=7))
+    stub.sound()
+    assert sim.launch_config() == shape and steps(sim) == 2
+    sim.set_launch_config(fuse_zchunk=7)
+    assert steps(sim) == 2
+    sim.set_launch_config(fuse_zchunk=100)   # the grid's depth at most
+    assert steps(sim) == 2
+    sim.autotune(1)
+    steps(sim)
+    sim.close()
+
+    # every allocation of cs_create in turn: refused, or without two-step passes
+    made, k, more = [], 0, True
+    while more:
+        held = []
+        try:
+            more = stub.failing(k, lambda: held.append(cs.Simulation(d.geometry, d.model, opts)))
+            made.append(steps(held[0]))
+            stub.sound()
+            held[0].close()
+        except RuntimeError:
+            stub.lib.hipGetLastError()   # a refused context leaves its error to the caller
+        k += 1
+    assert made == [0, 0, 0, 2], made    # the domain's record, the words, the tiles; then none fails
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -278,6 +326,10 @@ def test_ensemble_launch_names_the_form(tmp_path):
 
 def test_launch_config_names_the_form(tmp_path):
     _run(tmp_path, "launch_config_names_the_form")
+
+
+def test_steps_allocate_nothing(tmp_path):
+    _run(tmp_path, "steps_allocate_nothing")
 
 
 if __name__ == "__main__":
