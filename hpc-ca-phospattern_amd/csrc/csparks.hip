@@ -1430,7 +1430,6 @@ struct cs_context {
   double* d_stats = nullptr;
   double* d_lweights = nullptr;   /* linescan weights, nx + ny + nz        */
   double* d_lpart = nullptr;      /* linescan partial sums                  */
-  double* d_xyz = nullptr;        /* a slab of a species in the caller's layout */
   double* scratch = nullptr;      /* this device's `scratch` (no-alloc scan)  */
   /* host copies */
   cs_problem prob{};
@@ -1535,7 +1534,7 @@ void free_ctx(cs_context* c)
   void* ptrs[] = {c->d_u[0], c->d_u[1], c->d_ids, c->d_params, c->d_pairs, c->d_states, c->d_recruited,
                   c->d_row_voxel, c->d_row_species, c->d_row_start, c->d_ent_pair,
                   c->d_ent_flux, c->d_ent_sign, c->d_uniforms, c->d_partial, c->d_stats,
-                  c->d_lweights, c->d_lpart, c->d_xyz, c->d_f2_col, c->d_f2_z,
+                  c->d_lweights, c->d_lpart, c->d_f2_col, c->d_f2_z,
                   c->d_f2_l1, c->d_f2_fsum, c->d_bchan, c->d_brow, c->d_bent, c->d_p2_geo, c->d_p2_words,
                   c->d_bg_group, c->d_bg_vox, c->d_bg_chan, c->d_bg_row, c->d_bg_ent};
   for (auto& kv : c->p2_lists)
@@ -2082,27 +2081,35 @@ void launch_linescan(cs_context* c, uint32_t species, uint32_t axis, uint32_t do
                      g, gyc, axis, dproj);
 }
 
+/* Bytes of a field stack: the fields, what a row's last chunk may read
+ * beyond them, and in any case room for one x plane in double
+ * (copy_species). */
+size_t stack_bytes(const Geo& g, size_t esize)
+{
+  return std::max<size_t>(esize * g.ns * g.nv + P2_PAD, sizeof(double) * g.ny * g.nz);
+}
+
 /* Copy species s up to the stack or down from it, by slabs of x planes of
- * at most 64 MB through the context's staging buffer. */
+ * at most 64 MB.  They are staged in the field stack that the next pass
+ * overwrites and nothing reads before, so fields can be read and set
+ * however full the device is. */
 template <typename T, bool UP>
 int copy_species(cs_context* c, uint32_t s, double* host)
 {
   const Geo& g = c->geo;
   const uint64_t row = (uint64_t)g.ny * g.nz;   /* values of one x */
-  const int slab = (int)std::min<uint64_t>((uint64_t)g.nx, std::max<uint64_t>(1, (8ull << 20) / row));
-  if (!c->d_xyz && hipMalloc(&c->d_xyz, sizeof(double) * row * slab) != hipSuccess) {
-    c->d_xyz = nullptr;
-    return set_err(CS_ENOMEM, "device allocation of a species slab failed");
-  }
+  const uint64_t room = std::min<uint64_t>(8ull << 20, stack_bytes(g, c->esize) / sizeof(double));
+  const int slab = (int)std::min<uint64_t>((uint64_t)g.nx, std::max<uint64_t>(1, room / row));
+  double* xyz = (double*)c->d_u[c->cur ^ 1];
   for (int x0 = 0; x0 < g.nx; x0 += slab) {
     const int nxs = std::min(slab, g.nx - x0);
     double* part = host + row * x0;
     const uint64_t blocks = (uint64_t)((nxs + XPOSE - 1) / XPOSE) * ((g.nz + XPOSE - 1) / XPOSE) * g.ny;
-    if (UP) HIP_TRY(hipMemcpyAsync(c->d_xyz, part, sizeof(double) * row * nxs, hipMemcpyHostToDevice, c->stream));
+    if (UP) HIP_TRY(hipMemcpyAsync(xyz, part, sizeof(double) * row * nxs, hipMemcpyHostToDevice, c->stream));
     hipLaunchKernelGGL((k_species_xyz<T, UP>), dim3((unsigned)blocks), dim3(XPOSE, 8), 0, c->stream,
-                       (T*)c->d_u[c->cur], c->d_xyz, c->d_ids, (const DevParams<T>*)c->d_params, g, s, x0, nxs);
+                       (T*)c->d_u[c->cur], xyz, c->d_ids, (const DevParams<T>*)c->d_params, g, s, x0, nxs);
     HIP_TRY(hipGetLastError());
-    if (!UP) HIP_TRY(hipMemcpyAsync(part, c->d_xyz, sizeof(double) * row * nxs, hipMemcpyDeviceToHost, c->stream));
+    if (!UP) HIP_TRY(hipMemcpyAsync(part, xyz, sizeof(double) * row * nxs, hipMemcpyDeviceToHost, c->stream));
   }
   HIP_TRY(hipStreamSynchronize(c->stream));   /* the caller's array may end here */
   return CS_OK;
@@ -2379,8 +2386,8 @@ int cs_create(const cs_problem* p, cs_context** out)
       }
   if (hipMalloc(&c->d_ids, g.nv) != hipSuccess) return bail(set_err(CS_ENOMEM, "device allocation of ids failed"));
   for (int b = 0; b < 2; b++)
-    if (hipMalloc(&c->d_u[b], c->esize * c->ns * g.nv + P2_PAD) != hipSuccess)
-      return bail(set_err(CS_ENOMEM, "device allocation of %zu bytes failed", c->esize * c->ns * g.nv));
+    if (hipMalloc(&c->d_u[b], stack_bytes(g, c->esize)) != hipSuccess)
+      return bail(set_err(CS_ENOMEM, "device allocation of %zu bytes failed", stack_bytes(g, c->esize)));
   c->h_ids.swap(ids);
   for (uint8_t id : c->h_ids)
     if ((id & 7) < MAXD) c->dcount[id & 7]++;

@@ -295,6 +295,36 @@ def steps_allocate_nothing(stub):
     assert made == [0, 0, 0, 2], made    # the domain's record, the words, the tiles; then none fails
 
 
+def fields_move_without_memory(stub):
+    """Setting and reading fields allocates nothing, and their staging stays
+    inside the context's own memory, down to a plane of one species whose
+    doubles are larger than the field."""
+    import csparks as cs
+    import dyad
+    d = dyad.small_dyad(n=(33, 31, 14))
+    g, m = d.geometry, d.model
+    ca = dataclasses.replace(m, species_names=m.species_names[:1], init=np.asarray(m.init)[:, :1],
+                             diffusive=[[s for s in k if s == 0] for k in m.diffusive],
+                             sigma=[[v for v, s in zip(sg, k) if s == 0] for sg, k in zip(m.sigma, m.diffusive)],
+                             buffers=[[] for _ in m.buffers], ryr=None, p_ryr=None)
+
+    def cut(x, y, z):
+        return cs.Geometry(voxels=np.ascontiguousarray(g.voxels[:x, :y, :z]), h=g.h,
+                           domain_names=list(g.domain_names), domain_connections=g.domain_connections,
+                           boundaries=[])
+
+    for geom, model in ((g, m), (cut(1, 31, 14), ca), (cut(2, 31, 14), ca), (cut(1, 1, 14), ca), (cut(33, 1, 1), ca)):
+        for precision in ("f32", "f64"):
+            sim = cs.Simulation(geom, model, cs.Options(seed=1, precision=precision))
+            before = stub.lib.stub_allocs()
+            stub.lib.stub_fail_alloc_in(0)
+            sim.set_species(0, sim.species(0))
+            stub.lib.stub_fail_alloc_in(-1)
+            assert stub.lib.stub_allocs() == before
+            stub.sound()
+            sim.close()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -330,6 +360,10 @@ def test_launch_config_names_the_form(tmp_path):
 
 def test_steps_allocate_nothing(tmp_path):
     _run(tmp_path, "steps_allocate_nothing")
+
+
+def test_fields_move_without_memory(tmp_path):
+    _run(tmp_path, "fields_move_without_memory")
 
 
 if __name__ == "__main__":
