@@ -644,7 +644,14 @@ struct F2Voxels {
  * voxel is kept in its slot: step 2's gating and fluxes need only those
  * values, and its fluxes add to the result after the pass (k_bridge),
  * since no other voxel's step-2 update reads them. */
-template <typename T, int NS, int WY, bool NT>
+/* Step masks of a pass fixed at compile time: FM1/FM2 are the diffusing
+ * species of its two steps and FR the reaction mode of both, or F2_DYN for
+ * values taken from s1/s2 at run time.  With fixed masks the species loops
+ * keep only the species that diffuse, where run-time bits leave every
+ * species' code in the loop behind a test. */
+constexpr uint32_t F2_DYN = 0xFFFFFFFFu;
+
+template <typename T, int NS, int WY, bool NT, uint32_t FM1 = F2_DYN, uint32_t FM2 = F2_DYN, uint32_t FR = F2_DYN>
 __global__ void __launch_bounds__(BX * WY)
 k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__ ids,
         const DevParams<T>* __restrict__ P, Geo g, F2Voxels fv, const double* __restrict__ fsum,
@@ -698,7 +705,8 @@ k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__
   auto iofs = [&](int zz) { return (uint32_t)(min(max(zz, zb), ze - 1) - zb) * (uint32_t)plane; };
 
   const uint32_t react_nb = (uint32_t)P->nb;
-  uint32_t dm1 = s1.dmask, dm2 = s2.dmask, re1 = s1.react, re2 = s2.react, rbound = P->rbound;
+  uint32_t dm1 = FM1 != F2_DYN ? FM1 : s1.dmask, dm2 = FM2 != F2_DYN ? FM2 : s2.dmask;
+  uint32_t re1 = FR != F2_DYN ? FR : s1.react, re2 = FR != F2_DYN ? FR : s2.react, rbound = P->rbound;
   __shared__ uint32_t msk[5];
   if (lane == 0 && wy == 0) {
     msk[0] = dm1;
@@ -863,10 +871,12 @@ k_step2(const T* __restrict__ u, T* __restrict__ un, const uint8_t* __restrict__
      * orders the first read after the write): each species test is then a
      * bit test of one scalar register, not a flag hoisted out of the loop,
      * of which there are too many to keep in scalar registers */
-    dm1 = __builtin_amdgcn_readfirstlane(msk[0]);
-    dm2 = __builtin_amdgcn_readfirstlane(msk[1]);
-    re1 = __builtin_amdgcn_readfirstlane(msk[2]);
-    re2 = __builtin_amdgcn_readfirstlane(msk[3]);
+    if constexpr (FM1 == F2_DYN) dm1 = __builtin_amdgcn_readfirstlane(msk[0]);
+    if constexpr (FM2 == F2_DYN) dm2 = __builtin_amdgcn_readfirstlane(msk[1]);
+    if constexpr (FR == F2_DYN) {
+      re1 = __builtin_amdgcn_readfirstlane(msk[2]);
+      re2 = __builtin_amdgcn_readfirstlane(msk[3]);
+    }
     rbound = __builtin_amdgcn_readfirstlane(msk[4]);
     const bool below = z < nz;
     if (below) {
@@ -1846,9 +1856,9 @@ int launch_pass2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout,
   return CS_OK;
 }
 
-template <typename T, int NS>
-void launch_step2_ns(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
-                     const F2Step& b)
+template <typename T, int NS, uint32_t FM1 = F2_DYN, uint32_t FM2 = F2_DYN, uint32_t FR = F2_DYN>
+void launch_step2_k(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
+                    const F2Step& b)
 {
   constexpr int WY = sizeof(T) == 4 ? 16 : 8;
   const Geo& g = c->geo;
@@ -1859,13 +1869,43 @@ void launch_step2_ns(cs_context* c, const LaunchCfg& L, const void* uin, void* u
   const F2Voxels fv{c->d_f2_col, c->d_f2_z};
   /* plain stores: on the 400x400x200 dyad non-temporal ones cost 2% (472 against
    * 463 us per pass at z chunk 40 and groups of 32) */
-  hipLaunchKernelGGL((k_step2<T, NS, WY, false>), dim3(xcd_launch(nblocks, L.fx)), dim3(BX, WY), 0, c->stream,
-                     (const T*)uin, (T*)uout, c->d_ids, (const DevParams<T>*)c->d_params, g, fv,
+  hipLaunchKernelGGL((k_step2<T, NS, WY, false, FM1, FM2, FR>), dim3(xcd_launch(nblocks, L.fx)), dim3(BX, WY), 0,
+                     c->stream, (const T*)uin, (T*)uout, c->d_ids, (const DevParams<T>*)c->d_params, g, fv,
                      (const double*)c->d_f2_fsum, (T*)c->d_f2_l1, a, b, zc, tx, ty, nblocks, L.fx);
 }
 
-/* Two steps in one pass: k_pass2 where it applies, else k_step2 with the
- * masks read at run time. */
+/* Five species in FP32 that k_pass2 does not take (a species that no buffer
+ * binds, TRPN diffusing on a substep, no room for the words): the pairs of
+ * step masks that are every pair of consecutive steps when Ca and ATP
+ * diffuse on every step (0x9) and the dye and CMDN on multiples of dt of at
+ * least 2 (0x2, 0x4), compiled with fixed masks, the reaction species-major
+ * on both steps.  With a species unbound a pass takes 443 us on 400x400x200
+ * and 88 us on 201x187x91, with the masks read at run time 483 and 109 us.
+ * Other pairs, species counts and FP64 read the masks at run time. */
+template <typename T, int NS>
+void launch_step2_ns(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
+                     const F2Step& b)
+{
+  if constexpr (sizeof(T) == 4 && NS == 5) {
+    if (L.ff && a.react == 2 && b.react == 2) {
+      switch ((a.dmask << 8) | b.dmask) {
+        case 0x0909: return launch_step2_k<T, NS, 0x9, 0x9, 2>(c, L, uin, uout, a, b);
+        case 0x0B09: return launch_step2_k<T, NS, 0xB, 0x9, 2>(c, L, uin, uout, a, b);
+        case 0x090B: return launch_step2_k<T, NS, 0x9, 0xB, 2>(c, L, uin, uout, a, b);
+        case 0x0D09: return launch_step2_k<T, NS, 0xD, 0x9, 2>(c, L, uin, uout, a, b);
+        case 0x090D: return launch_step2_k<T, NS, 0x9, 0xD, 2>(c, L, uin, uout, a, b);
+        case 0x0F09: return launch_step2_k<T, NS, 0xF, 0x9, 2>(c, L, uin, uout, a, b);
+        case 0x090F: return launch_step2_k<T, NS, 0x9, 0xF, 2>(c, L, uin, uout, a, b);
+        case 0x0B0D: return launch_step2_k<T, NS, 0xB, 0xD, 2>(c, L, uin, uout, a, b);
+        case 0x0D0B: return launch_step2_k<T, NS, 0xD, 0xB, 2>(c, L, uin, uout, a, b);
+        default: break;
+      }
+    }
+  }
+  launch_step2_k<T, NS>(c, L, uin, uout, a, b);
+}
+
+/* Two steps in one pass: k_pass2 where it applies, else k_step2. */
 template <typename T>
 int launch_step2(cs_context* c, const LaunchCfg& L, const void* uin, void* uout, const F2Step& a,
                  const F2Step& b)

@@ -231,8 +231,10 @@ int cs_fused_available(const cs_context* ctx, char* why, size_t why_len);
  * half as many blocks as the device has CUs, else 0.  fuse_fixed = 1 runs
  * the two-step passes of the reference's five-slot species layout (Ca, dye,
  * CMDN-CSQN, ATP, TRPN; Ca and ATP diffusing on every step, TRPN on none)
- * with kernels compiled for each pair of step masks (k_pass2); 2 does so
- * and runs pairs whatever fuse says.  cs_create sets 2 for that layout where
+ * with kernels compiled for each pair of step masks (k_pass2), and in FP32
+ * those of other models of five species with ones compiled for the most
+ * frequent pairs of masks (k_step2); 2 does so and, for that layout, runs
+ * pairs whatever fuse says.  cs_create sets 2 for that layout where
  * it sets fuse = 0, since there pairs are the faster form at every size and
  * in both precisions (so a config that is read can be written back; one-step
  * passes take fuse = 0 and fuse_fixed below 2), else 1.  0

@@ -325,6 +325,29 @@ def fields_move_without_memory(stub):
             sim.close()
 
 
+def five_species_outside_the_layout_run_compiled_masks(stub):
+    """FP32 models of five species that the compiled pass of the five-slot
+    layout does not take (a species without a buffer, TRPN diffusing on a
+    substep) run two-step passes with their step masks compiled in, unless
+    fuse_fixed = 0 asks for run-time masks."""
+    import csparks as cs
+    import dyad
+    d = dyad.small_dyad(n=(40, 23, 9))
+    m = d.model
+    unbound = dataclasses.replace(m, buffers=[[b for b in bs if b.bound != 4] for bs in m.buffers])
+    slow = dataclasses.replace(m, diffusive=[list(k) + [4] for k in m.diffusive],
+                               sigma=[list(s) + [220000.0 / 100.25] for s in m.sigma])
+    for model in (unbound, slow):
+        sim = cs.Simulation(d.geometry, model, cs.Options(seed=1, open={"ryr": [0]}, precision="f32"))
+        for fixed, masks in ((1, "9u, 9u, 2u>"), (0, "4294967295u, 4294967295u, 4294967295u>")):
+            sim.set_launch_config(fuse=1, fuse_fixed=fixed)
+            before = stub.launches("k_step2<float, 5, 16, false, " + masks)
+            sim.step(40)
+            assert stub.launches("k_step2<float, 5, 16, false, " + masks) > before, (fixed, masks)
+        sim.close()
+    assert stub.launches("k_pass2") == 0
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -364,6 +387,10 @@ def test_steps_allocate_nothing(tmp_path):
 
 def test_fields_move_without_memory(tmp_path):
     _run(tmp_path, "fields_move_without_memory")
+
+
+def test_five_species_outside_the_layout_run_compiled_masks(tmp_path):
+    _run(tmp_path, "five_species_outside_the_layout_run_compiled_masks")
 
 
 if __name__ == "__main__":
