@@ -76,12 +76,21 @@ inline bool p2_whole(uint64_t stack_bytes) { return 2 * stack_bytes > (256ull <<
 /* The field stacks end in this many bytes that a row's last chunk may read. */
 constexpr size_t P2_PAD = 64;
 
-/* Launch the pass compiled for the step masks m1, m2; false when there is
- * none. */
+/* Most planes of a block of a two-step pass: it spans four z-groups (every
+ * species of a plane, `group` bytes) more than its planes, and `pad` bytes,
+ * under 32-bit descriptor offsets.  0 when not even one plane fits. */
+inline int p2_zlimit(uint64_t group, uint64_t nz, uint64_t pad)
+{
+  const uint64_t fit = ((1ull << 32) - 1 - pad) / group;
+  return fit > 4 ? (int)std::min<uint64_t>(nz, fit - 4) : 0;
+}
+
 /* The words of `count` domains from their ids (blocks of 256 voxels of the
  * largest one, for each). */
 void cs_internal_id_words(const uint8_t* ids, const P2Geo* geos, uint32_t count, uint64_t most_voxels,
                           uint32_t* words, hipStream_t stream);
+/* Launch the pass compiled for the step masks m1, m2; false when there is
+ * none. */
 bool cs_internal_pass2(size_t esize, bool whole, uint32_t m1, uint32_t m2, const P2Args& a, hipStream_t stream);
 bool cs_internal_pass2_f32(bool whole, uint32_t m1, uint32_t m2, const P2Args& a, hipStream_t stream);
 bool cs_internal_pass2_f64(bool whole, uint32_t m1, uint32_t m2, const P2Args& a, hipStream_t stream);

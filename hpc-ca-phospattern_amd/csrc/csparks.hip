@@ -1500,14 +1500,10 @@ int max_zchunk(const Geo& g, size_t esize)
   return (int)std::min<uint64_t>((uint64_t)g.nz, ((1ull << 32) - 1) / group - 3);
 }
 
-/* Largest z chunk of a two-step pass, whose blocks span (chunk + 4)
- * z-groups (and k_pass2's a last chunk's padding) under 32-bit descriptor
- * offsets (0 when not even one plane fits). */
-int max_fused_zchunk(const Geo& g, size_t esize)
+/* Largest z chunk of k_step2 and, with its rows' last chunks, of k_pass2. */
+int max_fused_zchunk(const Geo& g, size_t esize, bool pass2 = false)
 {
-  const uint64_t group = g.plane * esize * g.ns;
-  const uint64_t fit = ((1ull << 32) - 1 - P2_PAD) / group;
-  return fit > 4 ? (int)std::min<uint64_t>((uint64_t)g.nz, fit - 4) : 0;
+  return p2_zlimit(g.plane * esize * g.ns, (uint64_t)g.nz, pass2 ? P2_PAD : 0);
 }
 
 /* Default launch shape, the fastest measured on MI355X for the 32M-voxel
@@ -2176,7 +2172,7 @@ int setup_pass2(cs_context* c)
   const Geo& g = c->geo;
   c->p2_ok = false;
   if (!c->f2_ok || c->ns != 5 || (c->prob.num_buffers && (!c->rfast || c->rbound != 0x1Eu)) || !p2_substeps(c->substeps) ||
-      g.nx < 2 || g.ny < 2)
+      g.nx < 2 || g.ny < 2 || max_fused_zchunk(g, c->esize, true) < 1)
     return CS_OK;
   c->p2_whole = p2_whole(g.nv * c->ns * c->esize);
   c->p2_split = p2_split((uint32_t)g.nx, (uint32_t)g.ny, c->esize, c->p2_whole);
@@ -2463,7 +2459,7 @@ int cs_create(const cs_problem* p, cs_context** out)
     /* k_pass2's own planes per block and tile order */
     const long cols = (long)c->p2_split.kx * c->p2_split.ky;
     const uint32_t parts = p2_zparts((uint64_t)cols, (uint32_t)g.nz, c->p2_whole ? cus : 2 * cus,
-                                     (uint32_t)max_fused_zchunk(g, c->esize));
+                                     (uint32_t)max_fused_zchunk(g, c->esize, true));
     const int fz = (g.nz + (int)parts - 1) / (int)parts;
     rc = make_pass2_tiles(c, fz);
     if (rc != CS_OK && rc != CS_ENOMEM) return bail(rc);
@@ -2785,7 +2781,7 @@ int cs_set_launch_config(cs_context* c, const cs_launch_config* in)
   if (in->fuse_xcd > 64) return set_err(CS_EINVAL, "fuse_xcd is 0, 1 or a group size up to 64");
   if (in->fuse_fixed > 2) return set_err(CS_EINVAL, "fuse_fixed must be 0, 1 or 2");
   if (in->fuse_fixed == 2 && !c->p2_ok) return set_err(CS_EINVAL, "compiled two-step passes unavailable");
-  const int fzmax = max_fused_zchunk(c->geo, c->esize);
+  const int fzmax = max_fused_zchunk(c->geo, c->esize, c->p2_ok && in->fuse_fixed);
   if (in->fuse_zchunk < 1) return set_err(CS_EINVAL, "fuse_zchunk must be >= 1");
   if (fzmax >= 1 && (int)std::min<uint32_t>(in->fuse_zchunk, (uint32_t)c->geo.nz) > fzmax)
     return set_err(CS_EINVAL, "fuse_zchunk %u exceeds %d for this grid", in->fuse_zchunk, fzmax);
@@ -2912,7 +2908,7 @@ int cs_autotune(cs_context* c, uint64_t first_time_ind, uint32_t reps, cs_launch
             q.b.react == b.react && q.b.fluxmask == b.fluxmask) { q.count++; found = true; break; }
       if (!found) prs.push_back({a, b, 1});
     }
-    const int fzmax = max_fused_zchunk(c->geo, c->esize);
+    const int fzmax = max_fused_zchunk(c->geo, c->esize, c->p2_ok && winner.ff);
     std::vector<int> fzs;
     for (int zc : {16, 25, 32, 50, 64, 100})
       if (zc < nz && zc <= fzmax) fzs.push_back(zc);

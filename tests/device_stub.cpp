@@ -137,6 +137,7 @@ long stub_launches(const char* part)
 long stub_bad(void) { return (long)g_bad.size(); }
 const char* stub_bad_at(long k) { return g_bad[(size_t)k].c_str(); }
 int stub_pending_error(void) { return (int)g_last; }
+int stub_zlimit(uint64_t group, uint64_t nz, uint64_t pad) { return p2_zlimit(group, nz, pad); }
 
 /* ------------------------------------------------------- the runtime */
 

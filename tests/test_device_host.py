@@ -348,6 +348,22 @@ def five_species_outside_the_layout_run_compiled_masks(stub):
     assert stub.launches("k_pass2") == 0
 
 
+def planes_under_32_bit_offsets(stub):
+    """A block's z-groups end below 2^32 bytes, those of the five-slot pass
+    with what a row's last chunk reads beyond them; the general pass reads
+    nothing there, and its largest block is not smaller for it."""
+    f = stub.lib.stub_zlimit
+    f.argtypes = [C.c_uint64] * 3
+    group = 20 * 17895697                  # 12 groups are 16 bytes short of 2^32
+    assert (f(group, 100, 0), f(group, 100, 64)) == (8, 7)
+    assert (f(group, 5, 0), f(group, 5, 64)) == (5, 5)
+    assert (f(858993459, 9, 0), f(858993460, 9, 0), f(858993459, 9, 64)) == (1, 0, 0)
+    for g in (4, 20, 40, 12345680, 858993440):
+        for pad in (0, 64):
+            k = f(g, 1 << 30, pad)
+            assert (k + 4) * g + pad < 1 << 32 <= (k + 5) * g + pad or k == 1 << 30
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -391,6 +407,10 @@ def test_fields_move_without_memory(tmp_path):
 
 def test_five_species_outside_the_layout_run_compiled_masks(tmp_path):
     _run(tmp_path, "five_species_outside_the_layout_run_compiled_masks")
+
+
+def test_planes_under_32_bit_offsets(tmp_path):
+    _run(tmp_path, "planes_under_32_bit_offsets")
 
 
 if __name__ == "__main__":
