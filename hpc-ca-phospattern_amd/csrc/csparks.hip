@@ -65,6 +65,9 @@ int cs_internal_set_err(int code, const char* fmt, ...)
   vsnprintf(buf, sizeof buf, fmt, ap);
   va_end(ap);
   g_err = buf;
+  /* the failed runtime call's error is reported here and must not fail a
+   * later launch's check */
+  if (code == CS_ENOMEM || code == CS_EDEVICE) (void)hipGetLastError();
   return code;
 }
 

@@ -290,7 +290,7 @@ def steps_allocate_nothing(stub):
             stub.sound()
             held[0].close()
         except RuntimeError:
-            stub.lib.hipGetLastError()   # a refused context leaves its error to the caller
+            pass
         k += 1
     assert made == [0, 0, 0, 2], made    # the domain's record, the words, the tiles; then none fails
 
@@ -364,6 +364,26 @@ def planes_under_32_bit_offsets(stub):
             assert (k + 4) * g + pad < 1 << 32 <= (k + 5) * g + pad or k == 1 << 30
 
 
+def a_failed_call_leaves_no_error(stub):
+    """A call that fails for want of memory reports it, once: steps of this
+    and other contexts go on."""
+    import csparks as cs
+    import dyad
+    d = dyad.small_dyad()
+    opts = cs.Options(seed=1, open={"ryr": [0]})
+    sim, ens, net = cs.Simulation(d.geometry, d.model, opts), _ensemble(), _net()
+    line = (0, (0, 0, -3), d.model.conv)
+    calls = [lambda: cs.Simulation(d.geometry, d.model, opts), lambda: sim.linescan(1, *line), _ensemble,
+             lambda: ens.linescans(1, *line), ens.closure_features, ens.channel_ca, _net,
+             lambda: net.forward(np.zeros((64, 30))), lambda: net.set_data(np.zeros((64, 30)), np.zeros(64))]
+    for call in calls:
+        with pytest.raises(RuntimeError):
+            stub.failing(0, call)
+        stub.sound()
+        sim.step(2)
+        ens.step(2)
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -411,6 +431,10 @@ def test_five_species_outside_the_layout_run_compiled_masks(tmp_path):
 
 def test_planes_under_32_bit_offsets(tmp_path):
     _run(tmp_path, "planes_under_32_bit_offsets")
+
+
+def test_a_failed_call_leaves_no_error(tmp_path):
+    _run(tmp_path, "a_failed_call_leaves_no_error")
 
 
 if __name__ == "__main__":
