@@ -1448,6 +1448,7 @@ int b_step(cs_batch* b, uint64_t first, uint64_t n, const double* host_uni, uint
     if (need > b->uniform_cap) {
       if (b->d_uniforms) HIP_TRY(hipFree(b->d_uniforms));
       b->d_uniforms = nullptr;
+      b->uniform_cap = 0;
       HIP_TRY(hipMalloc(&b->d_uniforms, sizeof(double) * need));
       b->uniform_cap = need;
     }

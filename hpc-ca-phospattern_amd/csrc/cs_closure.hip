@@ -442,7 +442,8 @@ int pack(cs_mlp* m)
 
 int ensure_scratch(cs_mlp* m, uint64_t n)
 {
-  if (n <= m->scratch_n && m->d_xs) return CS_OK;
+  if (n <= m->scratch_n) return CS_OK;
+  m->scratch_n = 0;   /* until all four are there */
   void** ptrs[] = {(void**)&m->d_xs, (void**)&m->d_xbs, (void**)&m->d_ts, (void**)&m->d_ys};
   for (void** p : ptrs)
     if (*p) { HIP_TRY(hipFree(*p)); *p = nullptr; }

@@ -2006,6 +2006,7 @@ int run_steps(cs_context* c, uint64_t first, uint64_t n, const double* host_uni,
     if (need > c->uniform_cap) {
       if (c->d_uniforms) HIP_TRY(hipFree(c->d_uniforms));
       c->d_uniforms = nullptr;
+      c->uniform_cap = 0;
       HIP_TRY(hipMalloc(&c->d_uniforms, sizeof(double) * need));
       c->uniform_cap = need;
     }

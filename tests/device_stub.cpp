@@ -8,8 +8,9 @@
  * allocation from now fail, and checks what a launch would have read: every
  * pointer among a kernel's arguments must be null or lie in an allocation
  * that is still there (in a captured graph, at the time of its launch), and
- * every pointer of a two-step pass must not be null.  Freed memory stays
- * reserved, so a stale pointer is never taken for a new one.
+ * the pointers of two-step passes and of the network's forward kernels must
+ * not be null.  Freed memory stays reserved, so a stale pointer is never
+ * taken for a new one.
  */
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
@@ -190,6 +191,8 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     l.need_all = true;
     l.ptrs = {a.u, a.un, a.words, a.params, a.geos, a.tiles, a.col_start, a.vz, a.fsum, a.l1};
   }
+  l.need_all = l.need_all || l.name.find("k_mlp_to_bf16") != std::string::npos ||
+               l.name.find("k_mlp_forward") != std::string::npos;
   if (g_capture) g_capture->push_back(l);
   else check(l);
   return hipSuccess;
@@ -226,12 +229,11 @@ hipError_t hipHostFree(void* p)
 }
 static hipError_t copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind)
 {
-  const void* ends[2] = {kind != hipMemcpyDeviceToHost ? dst : nullptr, kind != hipMemcpyHostToDevice ? src : nullptr};
-  for (const void* p : ends)
-    if (bytes && p && (where(p) != 1 || where((const char*)p + bytes - 1) != 1)) {
-      g_bad.push_back("a copy outside device memory");
-      return fail(hipErrorInvalidValue);
-    }
+  auto outside = [bytes](const void* p) { return bytes && (where(p) != 1 || where((const char*)p + bytes - 1) != 1); };
+  if ((kind != hipMemcpyDeviceToHost && outside(dst)) || (kind != hipMemcpyHostToDevice && outside(src))) {
+    g_bad.push_back("a copy outside device memory");
+    return fail(hipErrorInvalidValue);
+  }
   memmove(dst, src, bytes);
   return hipSuccess;
 }

@@ -384,6 +384,30 @@ def a_failed_call_leaves_no_error(stub):
         ens.step(2)
 
 
+def buffers_that_failed_to_grow(stub):
+    """A call that finds no memory for more samples or draws fails; a
+    smaller one after it allocates what it needs and runs."""
+    import csparks as cs
+    import dyad
+    net = _net()
+    for k in range(4):
+        net.forward(np.zeros((100, 30)))
+        with pytest.raises(RuntimeError):
+            stub.failing(k, lambda: net.forward(np.zeros((500 + k, 30))))
+        net.forward(np.zeros((80, 30)))
+        net.grad(np.zeros((90, 30)), np.zeros(90))
+        stub.sound()
+    d = dyad.small_dyad()
+    sim = cs.Simulation(d.geometry, d.model, cs.Options(seed=1, open={"ryr": [0]}, rng="mt"))
+    for run in (sim, _ensemble(rng="mt")):
+        run.step(4)
+        with pytest.raises(RuntimeError):
+            stub.failing(0, lambda: run.step(400))
+        stub.sound()
+        run.step(2)
+        stub.sound()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -435,6 +459,10 @@ def test_planes_under_32_bit_offsets(tmp_path):
 
 def test_a_failed_call_leaves_no_error(tmp_path):
     _run(tmp_path, "a_failed_call_leaves_no_error")
+
+
+def test_buffers_that_failed_to_grow(tmp_path):
+    _run(tmp_path, "buffers_that_failed_to_grow")
 
 
 if __name__ == "__main__":
