@@ -2794,6 +2794,7 @@ int cs_set_launch_config(cs_context* c, const cs_launch_config* in)
   L.fx = (int)in->fuse_xcd;
   L.ff = (int)in->fuse_fixed;
   if (c->p2_ok && L.ff) {
+    HIP_TRY(hipSetDevice(c->device));
     const int rc = make_pass2_tiles(c, L.fz);
     if (rc != CS_OK) return rc;
   }

@@ -7,8 +7,8 @@
  * It counts launches by kernel name and allocations, lets the n-th
  * allocation from now fail, and checks what a launch would have read: every
  * pointer among a kernel's arguments must be null or lie in an allocation
- * that is still there (in a captured graph, at the time of its launch), and
- * the pointers of two-step passes and of the network's forward kernels must
+ * that is still there (in a captured graph, at the time of its launch) and
+ * on the device that is current, and the pointers of two-step passes and of the network's forward kernels must
  * not be null.  Freed memory stays reserved, so a stale pointer is never
  * taken for a new one.
  */
@@ -34,7 +34,9 @@ namespace {
 struct Block {
   size_t bytes;
   bool live;
+  int device;
 };
+int g_device = 0;
 std::map<uintptr_t, Block> g_blocks;   /* by first byte */
 std::map<const void*, std::string> g_names;
 std::map<std::string, long> g_launches;
@@ -51,14 +53,15 @@ std::vector<Launch>* g_capture = nullptr;
 
 hipError_t fail(hipError_t e) { return g_last = e; }
 
-/* 1: in a live allocation, 0: in none, -1: in a freed one */
+/* 1: in a live allocation of the current device, 2: of another, 0: in none,
+ * -1: in a freed one */
 int where(const void* p)
 {
   auto it = g_blocks.upper_bound((uintptr_t)p);
   if (it == g_blocks.begin()) return 0;
   --it;
   if ((uintptr_t)p >= it->first + it->second.bytes) return 0;
-  return it->second.live ? 1 : -1;
+  return !it->second.live ? -1 : it->second.device == g_device ? 1 : 2;
 }
 
 void check(const Launch& l)
@@ -68,7 +71,9 @@ void check(const Launch& l)
     const void* p = l.ptrs[k];
     if (p ? where(p) == 1 : !l.need_all) continue;
     char msg[64];
-    snprintf(msg, sizeof msg, ": pointer %zu is %s", k, p ? (where(p) ? "freed" : "no device memory") : "null");
+    const int at = p ? where(p) : 0;
+    snprintf(msg, sizeof msg, ": pointer %zu is %s", k,
+             !p ? "null" : at == 2 ? "on another device" : at ? "freed" : "no device memory");
     g_bad.push_back(l.name + msg);
   }
 }
@@ -159,7 +164,7 @@ static std::map<const void*, void*> g_vars;
 void __hipRegisterVar(void**, void* var, char*, char*, int, size_t size, int, int)
 {
   void* p = calloc(1, size);
-  g_blocks[(uintptr_t)p] = Block{size, true};
+  g_blocks[(uintptr_t)p] = Block{size, true, 0};
   g_vars[var] = p;
 }
 static struct { dim3 grid, block; size_t shmem; hipStream_t stream; } g_config;
@@ -203,7 +208,7 @@ hipError_t hipMalloc(void** p, size_t bytes)
   g_allocs++;
   if (g_fail_in >= 0 && g_fail_in-- == 0) return fail(hipErrorOutOfMemory);
   *p = calloc(1, bytes ? bytes : 1);
-  g_blocks[(uintptr_t)*p] = Block{bytes, true};
+  g_blocks[(uintptr_t)*p] = Block{bytes, true, g_device};
   return hipSuccess;
 }
 hipError_t hipFree(void* p)
@@ -268,10 +273,14 @@ hipError_t hipGetSymbolAddress(void** p, const void* var)
 
 hipError_t hipGetDevice(int* d)
 {
-  *d = 0;
+  *d = g_device;
   return hipSuccess;
 }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipSetDevice(int d)
+{
+  g_device = d;
+  return hipSuccess;
+}
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int)
 {
   memset(p, 0, sizeof *p);

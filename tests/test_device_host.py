@@ -408,6 +408,29 @@ def buffers_that_failed_to_grow(stub):
         stub.sound()
 
 
+def calls_use_their_own_device(stub):
+    """Launch shapes, fields, outputs and steps of a context, an ensemble and
+    a network stay on the device they were made on, whichever is current."""
+    import csparks as cs
+    import dyad
+    d = dyad.small_dyad()
+    sim = cs.Simulation(d.geometry, d.model, cs.Options(seed=1, open={"ryr": [0]}))
+    ens, net = _ensemble(), _net()
+    line = (0, (0, 0, -3), d.model.conv)
+    for call in (lambda: sim.set_launch_config(fuse=1, fuse_zchunk=7), lambda: sim.step(4), lambda: sim.autotune(1),
+                 lambda: sim.set_species(0, sim.species(0)), lambda: sim.linescan(1, *line), sim.stats,
+                 lambda: ens.set_launch(zchunk=4), lambda: ens.set_active([True, False, True]),
+                 lambda: ens.set_gating(ens.GATE_CLOSURE, net), lambda: ens.step(5), lambda: ens.autotune(1),
+                 lambda: ens.linescans(1, *line), lambda: net.forward(np.zeros((64, 30)))):
+        stub.lib.hipSetDevice(1)
+        call()
+        stub.sound()
+    stub.lib.hipSetDevice(1)
+    sim.step(4)
+    ens.step(5)
+    stub.sound()
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -463,6 +486,10 @@ def test_a_failed_call_leaves_no_error(tmp_path):
 
 def test_buffers_that_failed_to_grow(tmp_path):
     _run(tmp_path, "buffers_that_failed_to_grow")
+
+
+def test_calls_use_their_own_device(tmp_path):
+    _run(tmp_path, "calls_use_their_own_device")
 
 
 if __name__ == "__main__":
