@@ -936,10 +936,14 @@ void drop_pass2(cs_batch* b)
 
 /* Whether two-step passes (k_pass2) fit the ensemble: the five-slot layout
  * with its substeps, fluxes on Ca only, and on every grid at least two
- * columns either way and a split whose blocks hold a tile.  Half blocks:
- * planes of 43 to 171 columns a side leave little to gain from wider tiles
- * (512 dyads at 6 nm 342 us per step and 338 with whole blocks, 8 dyads at
- * 3 nm 155 and 158, 1024 dyads at 12 nm 368 and 382). */
+ * columns either way and a split whose blocks hold a tile.  Half blocks: on
+ * the ensembles of the spark statistics (planes of 43 to 342 columns a side)
+ * they are the better ones or even (512 dyads at 6 nm 342 us per step and
+ * 338 with whole blocks, 8 dyads at 3 nm 155 and 158, 1024 dyads at 12 nm
+ * 368 and 382).  On larger ones they beat one-step passes but not whole
+ * blocks: 16 dyads of 401x401x25 in FP32 402 us per step (whole 355,
+ * one-step 634), 2 of 400x400x200 442 (325 and 536), in FP64 818 (644 and
+ * 1095). */
 int setup_pass2(cs_batch* b)
 {
   b->p2_ok = b->p2_on = false;

@@ -32,7 +32,9 @@
  *   k_pass2   the same for the reference's five-slot layout, compiled for
  *             each pair of step masks (k_pass2.h);
  *   k_bridge  one block gates the channels and applies the boundary
- *             fluxes around the passes, with k_gate's and k_flux's code.
+ *             fluxes around the passes, with k_gate's and k_flux's code;
+ *             k_bridge_groups (cs_bridge.hip) does so in a block per group
+ *             of connected pairs, where every component of them fits one.
  */
 #include <hip/hip_runtime.h>
 

@@ -17,17 +17,18 @@
  * is its own (no flux through the face), so no lane selects anything.  z
  * neighbours sit in register rings that rotate by renaming.
  *
- * What bounds it: on a domain beyond the last-level cache, HBM (400x400x200
- * FP32 moves 1.56 GB a pass at 4.6 TB/s, the rate of a plain copy).  Within
- * the cache, the phases of a plane one after the other: a block's waves
- * move in step through loads, LDS, arithmetic (38% of cycles) and stores,
- * and row segments that start off a line or are shared by two tiles load
- * the L1; hence chunks instead of a load per value and neighbour, tiles
- * wide in x, and two blocks to a compute unit for smaller domains
- * (p2_whole).  On small domains, the latency of a block's few planes.  A
- * pass over two steps, before (k_step2 in FP32, two k_stencil in FP64) and
- * now: 400x400x200 FP32 455 and 329 us, FP64 1076 and 669 us; 201x187x91
- * FP32 78 and 39 us; 84^3 FP64 43 and 23 us; 64x64x25 FP64 21 and 14 us.
+ * What bounds it: the phases of a plane one after the other, since a
+ * block's waves move in step through loads, LDS, arithmetic (38% of cycles)
+ * and stores, and row segments that start off a line or are shared by two
+ * tiles load the L1; hence chunks instead of a load per value and neighbour,
+ * tiles wide in x, and two blocks to a compute unit for smaller domains
+ * (p2_whole).  On a domain beyond the last-level cache memory is next:
+ * 400x400x200 FP32 moves 1.56 GB a pass at 4.6 TB/s, where k_stencil, whose
+ * waves run apart, moves its bytes at 5.6 TB/s on the same grid.  On small
+ * domains, the latency of a block's few planes.  A pass over two steps,
+ * before (k_step2 in FP32, two k_stencil in FP64) and now: 400x400x200 FP32
+ * 455 and 329 us, FP64 1076 and 669 us; 201x187x91 FP32 78 and 39 us; 84^3
+ * FP64 43 and 23 us; 64x64x25 FP64 21 and 14 us.
  *
  * A lane reads one word per voxel, its id and its six neighbours' domains
  * (k_id_words), three planes ahead.  Bytes of ids, with six more loads where
