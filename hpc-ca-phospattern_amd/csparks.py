@@ -1076,6 +1076,8 @@ class Ensemble:
         return cfg.as_dict()
 
     def set_launch(self, **kw):
+        """Change keys of the launch shape; `persistent` names the form of
+        the passes (2: steps in pairs, 0 and 1: one-step passes)."""
         cfg = CBatchLaunch(**{**self.launch(), **kw})
         _check(device_lib().cs_batch_set_launch(self.handle, C.byref(cfg)), "cs_batch_set_launch")
 

@@ -292,7 +292,8 @@ int cs_batch_destroy(cs_batch* b);
  * active (Species_init_values per realisation, species.c:887-935). */
 int cs_batch_reset(cs_batch* b);
 /* Realisations, voxels over all of them, and device bytes of the fields
- * (two stacks) plus domain ids. */
+ * (two stacks) plus domain ids, without what two-step passes keep (4 bytes
+ * a voxel). */
 int cs_batch_info(const cs_batch* b, uint32_t* count, uint64_t* voxels, uint64_t* field_bytes);
 int cs_batch_upload_species(cs_batch* b, uint32_t realisation, uint32_t species, const double* src);
 int cs_batch_download_species(cs_batch* b, uint32_t realisation, uint32_t species, double* dst);
