@@ -631,10 +631,16 @@ int cs_mlp_set_data(cs_mlp* m, const float* x, const float* t, uint64_t n, uint6
   if (!m->idx_done) HIP_TRY(hipEventCreateWithFlags(&m->idx_done, hipEventDisableTiming));
   HIP_TRY(hipHostMalloc((void**)&m->h_idx, sizeof(uint32_t) * std::min(n, IDX_CHUNK), hipHostMallocDefault));
   float* d_xf = nullptr;
-  HIP_TRY(hipMalloc(&d_xf, sizeof(float) * n * MLP_IN));
-  HIP_TRY(hipMalloc(&m->d_x, sizeof(uint16_t) * n * MLP_PAD));
-  HIP_TRY(hipMalloc(&m->d_t, sizeof(float) * n));
-  HIP_TRY(hipMalloc(&m->d_idx, sizeof(uint32_t) * n));
+  if (hipMalloc(&d_xf, sizeof(float) * n * MLP_IN) != hipSuccess ||
+      hipMalloc(&m->d_x, sizeof(uint16_t) * n * MLP_PAD) != hipSuccess ||
+      hipMalloc(&m->d_t, sizeof(float) * n) != hipSuccess ||
+      hipMalloc(&m->d_idx, sizeof(uint32_t) * n) != hipSuccess) {
+    const int rc = set_err(CS_ENOMEM, "device allocation of %llu training samples failed", (unsigned long long)n);
+    if (d_xf) (void)hipFree(d_xf);
+    for (void** p : ptrs)
+      if (*p) { (void)hipFree(*p); *p = nullptr; }
+    return rc;
+  }
   HIP_TRY(hipMemcpyAsync(d_xf, x, sizeof(float) * n * MLP_IN, hipMemcpyHostToDevice, m->stream));
   HIP_TRY(hipMemcpyAsync(m->d_t, t, sizeof(float) * n, hipMemcpyHostToDevice, m->stream));
   int rc = to_bf16_rows(m, d_xf, n, m->d_x);

@@ -431,6 +431,26 @@ def calls_use_their_own_device(stub):
     stub.sound()
 
 
+def a_refused_training_set_is_given_back(stub):
+    """cs_mlp_set_data without memory for all of the set keeps none of it;
+    training asks for data, and a set that fits trains."""
+    net = _net()
+    x, t = np.zeros((400, 30)), np.zeros(400)
+    empty = stub.lib.stub_live_bytes()
+    k, more = 0, True
+    while more:
+        try:
+            more = stub.failing(k, lambda: net.set_data(x, t))
+        except RuntimeError:
+            assert stub.lib.stub_live_bytes() == empty, k
+            with pytest.raises(RuntimeError):
+                net.train(1, 64, 1e-3)
+        stub.sound()
+        k += 1
+    assert k == 5   # four allocations, then none fails
+    net.train(3, 64, 1e-3)
+
+
 def _run(tmp_path, name):
     stub = str(tmp_path / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
@@ -490,6 +510,10 @@ def test_buffers_that_failed_to_grow(tmp_path):
 
 def test_calls_use_their_own_device(tmp_path):
     _run(tmp_path, "calls_use_their_own_device")
+
+
+def test_a_refused_training_set_is_given_back(tmp_path):
+    _run(tmp_path, "a_refused_training_set_is_given_back")
 
 
 if __name__ == "__main__":
