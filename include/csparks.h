@@ -234,13 +234,13 @@ int cs_fused_available(const cs_context* ctx, char* why, size_t why_len);
  * with kernels compiled for each pair of step masks (k_pass2), and in FP32
  * those of other models of five species with ones compiled for the most
  * frequent pairs of masks (k_step2); 2 does so and, for that layout, runs
- * pairs whatever fuse says.  cs_create sets 2 for that layout where
- * it sets fuse = 0, since there pairs are the faster form at every size and
- * in both precisions (so a config that is read can be written back; one-step
- * passes take fuse = 0 and fuse_fixed below 2), else 1.  0
- * runs every pass with the masks read at run time (k_step2; same results
- * to rounding).  No reference counterpart: the reference's
- * OpenMP/AVX-512 loop has no launch shape (kernel_generic.cpp:561-600). */
+ * pairs whatever fuse says.  cs_create sets 2 for that layout where it sets
+ * fuse = 0, since there pairs are the faster form at every size and in both
+ * precisions (so a config that is read can be written back; one-step passes
+ * take fuse = 0 and fuse_fixed below 2), else 1.  0 runs every pass with the
+ * masks read at run time (k_step2; same results to rounding).  No reference
+ * counterpart: the reference's OpenMP/AVX-512 loop has no launch shape
+ * (kernel_generic.cpp:561-600). */
 typedef struct cs_launch_config {
   uint32_t rows, zchunk, xcd_remap, prefetch, nontemporal, lds_tile, linear, yblock;
   uint32_t fuse, fuse_zchunk, fuse_xcd, fuse_fixed;
@@ -387,8 +387,8 @@ int cs_batch_get_launch(const cs_batch* b, cs_batch_launch* cfg);
 int cs_batch_set_launch(cs_batch* b, const cs_batch_launch* cfg);
 /* Time every candidate shape on one period of the step pattern from
  * first_time_ind (state unchanged) and keep the fastest: persistent = 2
- * with the best one-step shape, or that shape alone if it is faster.  best_ms is the mean
- * kernel time per step of the form that runs. */
+ * with the best one-step shape, or that shape alone if it is faster.
+ * best_ms is the mean kernel time per step of the form that runs. */
 int cs_batch_autotune(cs_batch* b, uint64_t first_time_ind, uint32_t reps, cs_batch_launch* best,
                       double* best_ms);
 /* on != 0: cs_batch_step replays whole periods of the step pattern (the
