@@ -451,69 +451,35 @@ def a_refused_training_set_is_given_back(stub):
     net.train(3, 64, 1e-3)
 
 
-def _run(tmp_path, name):
-    stub = str(tmp_path / "device_stub.so")
+CASES = (ensemble_closure_without_memory,
+         ensemble_retiring_without_memory,
+         ensemble_launch_without_memory,
+         flux_network_predicts_each_state_once,
+         ensemble_launch_names_the_form,
+         launch_config_names_the_form,
+         steps_allocate_nothing,
+         fields_move_without_memory,
+         five_species_outside_the_layout_run_compiled_masks,
+         planes_under_32_bit_offsets,
+         a_failed_call_leaves_no_error,
+         buffers_that_failed_to_grow,
+         calls_use_their_own_device,
+         a_refused_training_set_is_given_back)
+
+
+@pytest.fixture(scope="module")
+def stand_in_library(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("stub") / "device_stub.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", "/opt/rocm/include", "-I",
-                    os.path.join(PKG, "csrc"), os.path.join(HERE, "device_stub.cpp"), "-o", stub], check=True)
-    r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, name], capture_output=True, text=True,
-                       timeout=300)
+                    os.path.join(PKG, "csrc"), os.path.join(HERE, "device_stub.cpp"), "-o", path], check=True)
+    return path
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: c.__name__)
+def test_host_code(case, stand_in_library):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), stand_in_library, case.__name__],
+                       capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
-
-
-def test_ensemble_closure_without_memory(tmp_path):
-    _run(tmp_path, "ensemble_closure_without_memory")
-
-
-def test_ensemble_retiring_without_memory(tmp_path):
-    _run(tmp_path, "ensemble_retiring_without_memory")
-
-
-def test_ensemble_launch_without_memory(tmp_path):
-    _run(tmp_path, "ensemble_launch_without_memory")
-
-
-def test_flux_network_predicts_each_state_once(tmp_path):
-    _run(tmp_path, "flux_network_predicts_each_state_once")
-
-
-def test_ensemble_launch_names_the_form(tmp_path):
-    _run(tmp_path, "ensemble_launch_names_the_form")
-
-
-def test_launch_config_names_the_form(tmp_path):
-    _run(tmp_path, "launch_config_names_the_form")
-
-
-def test_steps_allocate_nothing(tmp_path):
-    _run(tmp_path, "steps_allocate_nothing")
-
-
-def test_fields_move_without_memory(tmp_path):
-    _run(tmp_path, "fields_move_without_memory")
-
-
-def test_five_species_outside_the_layout_run_compiled_masks(tmp_path):
-    _run(tmp_path, "five_species_outside_the_layout_run_compiled_masks")
-
-
-def test_planes_under_32_bit_offsets(tmp_path):
-    _run(tmp_path, "planes_under_32_bit_offsets")
-
-
-def test_a_failed_call_leaves_no_error(tmp_path):
-    _run(tmp_path, "a_failed_call_leaves_no_error")
-
-
-def test_buffers_that_failed_to_grow(tmp_path):
-    _run(tmp_path, "buffers_that_failed_to_grow")
-
-
-def test_calls_use_their_own_device(tmp_path):
-    _run(tmp_path, "calls_use_their_own_device")
-
-
-def test_a_refused_training_set_is_given_back(tmp_path):
-    _run(tmp_path, "a_refused_training_set_is_given_back")
 
 
 if __name__ == "__main__":
